@@ -63,8 +63,6 @@ struct p9idg_plan {
     // device buffers
     double* d_uvw = nullptr;
     double* d_wavenumbers = nullptr;
-    p9idg_subgrid* d_meta = nullptr;
-    int32_t* d_order = nullptr;
     float2* d_vis = nullptr;
     float2* d_model_vis = nullptr;
     float2* d_grid = nullptr;
@@ -79,12 +77,18 @@ struct p9idg_plan {
     void* d_staging = nullptr;
     size_t staging_bytes = 0;
 
-    // work queues (one item list per direction) and the queue counter
-    std::vector<p9idg_subgrid> meta_host;
-    std::vector<int32_t> order_host;
-    WorkItem* d_items_grid = nullptr;
-    WorkItem* d_items_degrid = nullptr;
-    int32_t nitems_grid = 0, nitems_degrid = 0;
+    // The rows that the kernels work on: the observation's own (direct), or its
+    // time-resampled ones (rs_view).  A view has the subgrids' metadata and
+    // schedule and its work queues, one item list per direction.
+    struct View {
+        std::vector<p9idg_subgrid> meta;
+        std::vector<int32_t> order;
+        p9idg_subgrid* d_meta = nullptr;
+        int32_t* d_order = nullptr;
+        WorkItem* d_items_grid = nullptr;
+        WorkItem* d_items_degrid = nullptr;
+        int32_t nitems_grid = 0, nitems_degrid = 0;
+    } direct, rs_view;
     int32_t* d_counter = nullptr;
     // launch shape (tunable): queue mode, visibilities per work item, workgroups
     // residual visibilities (vis - model_vis, 0 where flagged) and the
@@ -131,6 +135,22 @@ struct p9idg_plan {
         int32_t n_bins = 0, n_chunks = 0;
     } gather[3];
 
+    // Time-resampled observation (kernels_resample.hip): rs_view's subgrids
+    // index its rows (baseline 0, rows from time_sample_start), d_rs_uvw holds
+    // its tracks and d_rs_vis its visibilities: the gridder's input, gathered
+    // from the visibilities before each launch, or the degridder's output,
+    // spread to the timesteps after it.  have_rs: built for this observation;
+    // resampled: used by the plan's kernel (want_resample).
+    bool have_rs = false;
+    bool resampled = false;
+    Resample rs;
+    double* d_rs_uvw = nullptr;
+    float2* d_rs_vis = nullptr;
+    // the two allocations that all of its arrays (and rs_view's) lie in
+    uint8_t* d_rs_chunks = nullptr;
+    uint8_t* d_rs_rows = nullptr;
+    size_t alloc_rs_chunks = 0, alloc_rs_rows = 0;
+
     hipfftHandle fft_one = 0;
     bool have_fft_one = false;
 
@@ -154,6 +174,16 @@ struct p9idg_plan {
 
 namespace {
 
+// Resampling is built for observations of at least kResampleMinVis
+// visibilities where it leaves at most kResamplePays of the rows; the MFMA
+// kernels use it from kResampleMinVisMfma visibilities.  Grid / degrid at 256^2
+// (us, direct -> resampled): FP32 S = 32, 27 k visibilities 148 / 137 ->
+// 31 / 50, S = 8 82 / 20 -> 24 / 19; split-BF16 S = 32, 58 k 30 / 23 -> 28 / 23,
+// 209 k 64 / 33 -> 56 / 33, 442 k 76 / 52 -> 40 / 32.
+constexpr int64_t kResampleMinVis = 1 << 14;
+constexpr int64_t kResampleMinVisMfma = 1 << 18;
+constexpr double kResamplePays = 0.6;
+
 size_t padded(size_t bytes) { return (bytes + 255) & ~(size_t)255; }
 
 template <typename T>
@@ -175,6 +205,18 @@ template <typename T>
 void dev_free(T*& p) {
     if (p) (void)hipFree(p);
     p = nullptr;
+}
+
+// At least `count` elements (contents are not kept).  Called with the plan's
+// stream idle and its recorded graph dropped.
+template <typename T>
+int dev_reserve(T*& p, size_t& have, size_t count) {
+    if (have >= count && p) return P9IDG_OK;
+    dev_free(p);
+    have = 0;
+    if (int st = dev_alloc(&p, std::max<size_t>(count, 1))) return st;
+    have = count;
+    return P9IDG_OK;
 }
 
 struct DeviceGuard {
@@ -254,6 +296,125 @@ int build_footprints(p9idg_plan* p, const p9idg_subgrid* meta, int64_t nsub) {
         if (int st = dev_alloc(&p->d_fp[mode], used.size())) return st;
         P9_HIP(hipMemcpy(p->d_fp[mode], used.data(), used.size() * sizeof(Box), hipMemcpyHostToDevice));
     }
+    return P9IDG_OK;
+}
+
+// A view's schedule (most rows first) and its arrays on the device.
+int upload_view(p9idg_plan* p, p9idg_plan::View& v) {
+    v.order.resize(v.meta.size());
+    std::iota(v.order.begin(), v.order.end(), 0);
+    std::stable_sort(v.order.begin(), v.order.end(), [&](int32_t a, int32_t b) {
+        return v.meta[a].time_sample_count > v.meta[b].time_sample_count;
+    });
+    if (v.meta.empty()) return P9IDG_OK;
+    P9_HIP(hipMemcpyAsync(v.d_meta, v.meta.data(), v.meta.size() * sizeof(p9idg_subgrid), hipMemcpyHostToDevice, p->stream));
+    P9_HIP(hipMemcpyAsync(v.d_order, v.order.data(), v.order.size() * sizeof(int32_t), hipMemcpyHostToDevice, p->stream));
+    return P9IDG_OK;
+}
+
+// Whether the plan's kernel works on the resampled rows.
+bool want_resample(const p9idg_plan* p) {
+    return p->have_rs && (p->kernel == P9IDG_KERNEL_FP32 || p->kernel == P9IDG_KERNEL_FP32_SEP
+                              ? true
+                              : p->gridded_vis >= kResampleMinVisMfma);
+}
+
+// Splits the subgrids' timesteps into chunks, measures which of them can be
+// resampled and, where that pays, builds the resampled observation.  Called
+// with the plan's stream idle and the tracks' upload queued.
+int build_resample(p9idg_plan* p, int T, int C, const double* freq) {
+    p->have_rs = p->resampled = false;
+    std::vector<p9idg_subgrid> meta = p->direct.meta;
+    const int S = p->c.subgrid_size;
+    const float image_size = p->c.scale_arcsec * (float)p->c.grid_size;
+    std::vector<ResampleChunk> chunks;
+    int64_t rows = 0;
+    for (const p9idg_subgrid& m : meta) {
+        const int nt = m.time_sample_count, n = (nt + kResampleMaxLen - 1) / kResampleMaxLen;
+        // multiples of 16 up to the last chunk, so few weight tables serve all
+        const int step = n > 0 ? ((nt + n - 1) / n + 15) / 16 * 16 : 1;
+        for (int t = 0; t < nt; t += step)
+            chunks.push_back({(int64_t)m.baseline_idx * T + m.time_sample_start + t, 0, 0, std::min(step, nt - t), 0, 0});
+        rows += nt;
+    }
+    if (rows * C < kResampleMinVis || rows > INT32_MAX) return P9IDG_OK;
+    // corner pixel and highest wavenumber (Gridder.cs:163-174; n in double: an upper estimate suffices)
+    double fmax = 0.0;
+    for (int i = 0; i < C; i++) fmax = std::max(fmax, std::fabs(freq[i]));
+    const double l = (0.5 * S - 0.5) * (double)image_size / S, t = 2.0 * l * l;
+    const double kl = fmax / 299792458.0 * l, kn = fmax / 299792458.0 * (t < 1.0 ? t / (t + std::sqrt(1.0 - t)) : 1.0);
+    const size_t nc = chunks.size();
+    const size_t nodes_at = padded(nc * sizeof(ResampleChunk));
+    if (int st = dev_reserve(p->d_rs_chunks, p->alloc_rs_chunks, nodes_at + nc * sizeof(int32_t))) return st;
+    p->rs.chunks = reinterpret_cast<ResampleChunk*>(p->d_rs_chunks);
+    int32_t* const d_nodes = reinterpret_cast<int32_t*>(p->d_rs_chunks + nodes_at);
+    P9_HIP(hipMemcpyAsync(p->rs.chunks, chunks.data(), nc * sizeof(ResampleChunk), hipMemcpyHostToDevice, p->stream));
+    P9_HIP(launch_resample_analyse(p->rs.chunks, (int)nc, p->d_uvw, kl, kn, d_nodes, p->stream));
+    std::vector<int32_t> nodes(nc);
+    P9_HIP(hipMemcpyAsync(nodes.data(), d_nodes, nc * sizeof(int32_t), hipMemcpyDeviceToHost, p->stream));
+    P9_HIP(hipStreamSynchronize(p->stream));
+    int64_t kept = 0;
+    for (size_t i = 0; i < nc; i++) kept += nodes[i] > 0 ? nodes[i] : chunks[i].len;
+    if ((double)kept > kResamplePays * (double)rows) return P9IDG_OK;
+    // rows in subgrid order, one weight table per (len, nodes) pair
+    constexpr int kNodeSteps = kResampleMaxNodes / 4 + 1;
+    std::vector<int64_t> table((size_t)(kResampleMaxLen + 1) * kNodeSteps, -1);
+    std::vector<ResamplePair> pairs;
+    int64_t weights = 0;
+    int32_t dst = 0;
+    size_t i = 0;
+    for (p9idg_subgrid& m : meta) {
+        const int32_t row0 = dst;
+        for (int t = 0; t < m.time_sample_count; i++) {
+            ResampleChunk& c = chunks[i];
+            c.nodes = nodes[i];
+            c.dst = dst;
+            dst += c.nodes > 0 ? c.nodes : c.len;
+            t += c.len;
+            if (c.nodes == 0) continue;
+            int64_t& at = table[(size_t)c.len * kNodeSteps + c.nodes / 4];
+            if (at < 0) {
+                at = weights;
+                pairs.push_back({weights, c.len, c.nodes});
+                weights += 2 * (int64_t)c.len * c.nodes;
+            }
+            c.weights = at;
+        }
+        m.baseline_idx = 0;
+        m.time_sample_start = row0;
+        m.time_sample_count = dst - row0;
+    }
+    // largest first, chunks of one table side by side
+    std::stable_sort(chunks.begin(), chunks.end(), [](const ResampleChunk& a, const ResampleChunk& b) {
+        return a.len * a.nodes != b.len * b.nodes ? a.len * a.nodes > b.len * b.nodes : a.weights < b.weights;
+    });
+    size_t end = 0;
+    auto place = [&](size_t bytes) {
+        const size_t at = end;
+        end += padded(bytes);
+        return at;
+    };
+    const size_t at_pairs = place(pairs.size() * sizeof(ResamplePair)), at_weights = place(weights * sizeof(float)),
+                 at_uvw = place((size_t)dst * 3 * sizeof(double)), at_vis = place((size_t)dst * C * sizeof(float2)),
+                 at_meta = place(meta.size() * sizeof(p9idg_subgrid)), at_order = place(meta.size() * sizeof(int32_t));
+    if (int st = dev_reserve(p->d_rs_rows, p->alloc_rs_rows, end)) return st;
+    ResamplePair* const d_pairs = reinterpret_cast<ResamplePair*>(p->d_rs_rows + at_pairs);
+    p->rs.weights = reinterpret_cast<float*>(p->d_rs_rows + at_weights);
+    p->d_rs_uvw = reinterpret_cast<double*>(p->d_rs_rows + at_uvw);
+    p->d_rs_vis = reinterpret_cast<float2*>(p->d_rs_rows + at_vis);
+    p->rs_view.d_meta = reinterpret_cast<p9idg_subgrid*>(p->d_rs_rows + at_meta);
+    p->rs_view.d_order = reinterpret_cast<int32_t*>(p->d_rs_rows + at_order);
+    P9_HIP(hipMemcpyAsync(p->rs.chunks, chunks.data(), nc * sizeof(ResampleChunk), hipMemcpyHostToDevice, p->stream));
+    if (!pairs.empty())
+        P9_HIP(hipMemcpyAsync(d_pairs, pairs.data(), pairs.size() * sizeof(ResamplePair), hipMemcpyHostToDevice,
+                              p->stream));
+    P9_HIP(launch_resample_tables(d_pairs, (int)pairs.size(), p->rs.weights, p->rs.chunks, (int)nc, p->d_uvw,
+                                  p->d_rs_uvw, p->stream));
+    p->rs_view.meta = std::move(meta);
+    if (int st = upload_view(p, p->rs_view)) return st;
+    P9_HIP(hipStreamSynchronize(p->stream));  // the host vectors end here
+    p->rs.nchunks = (int32_t)nc;
+    p->have_rs = true;
     return P9IDG_OK;
 }
 
@@ -414,26 +575,42 @@ void free_gather(p9idg_plan::Gather& g) {
     g.valid = false;
 }
 
+// The view that the plan's launches use.
+const p9idg_plan::View& active_view(const p9idg_plan* p) { return p->resampled ? p->rs_view : p->direct; }
+
+void free_items(p9idg_plan::View& v) {
+    dev_free(v.d_items_grid);
+    dev_free(v.d_items_degrid);
+    v.nitems_grid = v.nitems_degrid = 0;
+}
+
+int upload_list(const std::vector<WorkItem>& items, WorkItem*& d, int32_t& n, hipStream_t st) {
+    if (items.size() > (size_t)INT32_MAX) return fail(P9IDG_ERR_ARGUMENT, "too many work items");
+    if (int s = dev_alloc(&d, items.size())) return s;
+    P9_HIP(hipMemcpyAsync(d, items.data(), items.size() * sizeof(WorkItem), hipMemcpyHostToDevice, st));
+    P9_HIP(hipStreamSynchronize(st));
+    n = (int32_t)items.size();
+    return P9IDG_OK;
+}
+
+// The active view's work items for the plan's launch shape, and the direct
+// degridder's (p9idg_degrid and the other calls that return double).
 int upload_items(p9idg_plan* p) {
     DeviceGuard dg(p->device);
     P9_HIP(hipStreamSynchronize(p->stream));  // queued launches may still read the old arrays
     drop_graph(p);  // a captured step holds the old item arrays and tile lists
     for (auto& g : p->gather) free_gather(g);
-    dev_free(p->d_items_grid);
-    dev_free(p->d_items_degrid);
-    p->nitems_grid = p->nitems_degrid = 0;
+    free_items(p->direct);
+    free_items(p->rs_view);
     if (p->nsub == 0) return P9IDG_OK;
-    const auto gi = make_items(p->meta_host, p->order_host, p->C, p->grid_chunk);
-    const auto di = make_items(p->meta_host, p->order_host, p->C, p->degrid_chunk);
-    if (gi.size() > (size_t)INT32_MAX || di.size() > (size_t)INT32_MAX)
-        return fail(P9IDG_ERR_ARGUMENT, "too many work items");
-    if (int st = dev_alloc(&p->d_items_grid, gi.size())) return st;
-    if (int st = dev_alloc(&p->d_items_degrid, di.size())) return st;
-    P9_HIP(hipMemcpyAsync(p->d_items_grid, gi.data(), gi.size() * sizeof(WorkItem), hipMemcpyHostToDevice, p->stream));
-    P9_HIP(hipMemcpyAsync(p->d_items_degrid, di.data(), di.size() * sizeof(WorkItem), hipMemcpyHostToDevice, p->stream));
-    P9_HIP(hipStreamSynchronize(p->stream));
-    p->nitems_grid = (int32_t)gi.size();
-    p->nitems_degrid = (int32_t)di.size();
+    p9idg_plan::View& v = p->resampled ? p->rs_view : p->direct;
+    if (int st = upload_list(make_items(v.meta, v.order, p->C, p->grid_chunk), v.d_items_grid, v.nitems_grid, p->stream))
+        return st;
+    if (int st = upload_list(make_items(v.meta, v.order, p->C, p->degrid_chunk), v.d_items_degrid, v.nitems_degrid, p->stream))
+        return st;
+    p9idg_plan::View& d = p->direct;
+    if (p->resampled)
+        return upload_list(make_items(d.meta, d.order, p->C, p->degrid_chunk), d.d_items_degrid, d.nitems_degrid, p->stream);
     return P9IDG_OK;
 }
 
@@ -444,15 +621,17 @@ LaunchCfg launch_cfg(const p9idg_plan* p, bool grid) {
     return cfg;
 }
 
-KernelArgs make_args(const p9idg_plan* p, int mode) {
+// resampled: for the rows of rs_view instead of the observation's own.
+KernelArgs make_args(const p9idg_plan* p, int mode, bool resampled) {
     KernelArgs a{};
-    a.meta = p->d_meta;
-    a.order = p->d_order;
+    const p9idg_plan::View& v = resampled ? p->rs_view : p->direct;
+    a.meta = v.d_meta;
+    a.order = v.d_order;
     a.nr_subgrids = (int32_t)p->nsub;
-    a.uvw = p->d_uvw;
+    a.uvw = resampled ? p->d_rs_uvw : p->d_uvw;
     a.wavenumbers = p->d_wavenumbers;
-    a.vis = p->grid_src == P9IDG_SRC_RESIDUAL ? p->d_resid : p->d_vis;
-    a.vis_out = p->d_model_vis;
+    a.vis = resampled ? p->d_rs_vis : p->grid_src == P9IDG_SRC_RESIDUAL ? p->d_resid : p->d_vis;
+    a.vis_out = resampled ? p->d_rs_vis : p->d_model_vis;
     a.twiddle = p->d_twiddle;
     a.adder_phasor = p->d_phasor;
     a.rtab = p->d_rtab;
@@ -487,8 +666,9 @@ int prepare_gather(p9idg_plan* p, int mode) {
     p9idg_plan::Gather& gt = p->gather[mode];
     if (gt.valid) return P9IDG_OK;  // valid until the work items change (upload_items)
     const int S = p->c.subgrid_size, G = p->c.grid_size, L = p->c.wlayer_count;
+    const p9idg_plan::View& v = active_view(p);
     const std::vector<WorkItem> items =
-        make_items(p->meta_host, p->order_host, p->C, p->use_queue ? p->grid_chunk : 0);
+        make_items(v.meta, v.order, p->C, p->use_queue ? p->grid_chunk : 0);
     const size_t need = items.size() * (size_t)S * S;
     P9_HIP(hipStreamSynchronize(p->stream));  // queued launches may still use the old buffers
     if (p->alloc_scratch != need) {
@@ -505,7 +685,7 @@ int prepare_gather(p9idg_plan* p, int mode) {
     std::vector<SlotCorner> corner(items.size());
     std::vector<int32_t> layer(items.size(), -1);  // -1: the adder skips the slot
     for (const WorkItem& w : items) {
-        const p9idg_subgrid& m = p->meta_host[w.sidx];
+        const p9idg_subgrid& m = v.meta[w.sidx];
         int X = m.u_pixel, Y = m.v_pixel, W = 0;
         bool ok;
         if (mode == P9IDG_GRID_PLAIN) {
@@ -586,10 +766,10 @@ int do_exec_grid(p9idg_plan* p, int mode) {
         target = p->d_layers;
         n *= (size_t)p->c.wlayer_count;
     }
-    KernelArgs a = make_args(p, mode);
+    KernelArgs a = make_args(p, mode, p->resampled);
     a.grid = target;
-    a.items = p->d_items_grid;
-    a.nitems = p->nitems_grid;
+    a.items = active_view(p).d_items_grid;
+    a.nitems = active_view(p).nitems_grid;
     if (p->deterministic) {
         if (p->capturing && !p->gather[mode].valid)
             return fail(P9IDG_ERR_STATE, "deterministic adder not prepared for this mode before capture");
@@ -601,6 +781,9 @@ int do_exec_grid(p9idg_plan* p, int mode) {
     if (int st = span_next(p, P9IDG_STAGE_GRIDDER)) return st;
     if (int st_ = record(p, 1)) return st_;
     hipError_t e;
+    if (p->resampled)
+        P9_HIP(launch_resample_gather(p->rs, p->C, p->grid_src == P9IDG_SRC_RESIDUAL ? p->d_resid : p->d_vis, p->d_rs_vis,
+                                      p->stream));
     if (p->kernel == P9IDG_KERNEL_FP32 || p->kernel == P9IDG_KERNEL_FP32_SEP)
         e = launch_grid_fp32(a, p->c.subgrid_size, p->kernel == P9IDG_KERNEL_FP32_SEP, launch_cfg(p, true),
                              p->stream);
@@ -619,14 +802,18 @@ int do_exec_grid(p9idg_plan* p, int mode) {
     return P9IDG_OK;
 }
 
-int do_exec_degrid(p9idg_plan* p, int mode) {
+// direct: every timestep's visibilities by the degridder itself, also where
+// the plan resamples.
+int do_exec_degrid(p9idg_plan* p, int mode, bool direct = false) {
     if (int st = check_obs(p)) return st;
     if (mode != P9IDG_DEGRID_PLAIN && mode != P9IDG_DEGRID_WSTACK)
         return fail(P9IDG_ERR_ARGUMENT, "unknown degrid mode");
     DeviceGuard dg(p->device);
-    KernelArgs a = make_args(p, mode);
-    a.items = p->d_items_degrid;
-    a.nitems = p->nitems_degrid;
+    const bool resampled = p->resampled && !direct;
+    KernelArgs a = make_args(p, mode, resampled);
+    const p9idg_plan::View& v = resampled ? p->rs_view : p->direct;
+    a.items = v.d_items_degrid;
+    a.nitems = v.nitems_degrid;
     // Gridder.cs:96: uncovered timesteps stay 0; only the degridder writes
     // this buffer, and always the same (covered) entries
     if (p->capturing || !p->model_vis_clean) {
@@ -645,6 +832,7 @@ int do_exec_degrid(p9idg_plan* p, int mode) {
     else
         e = launch_degrid_mfma(a, p->c.subgrid_size, p->kernel, launch_cfg(p, false), p->stream);
     if (e != hipSuccess) return hip_fail(e, "degridder launch");
+    if (resampled) P9_HIP(launch_resample_spread(p->rs, p->C, p->d_rs_vis, p->d_model_vis, p->stream));
     if (int st = span_end(p)) return st;
     if (int st_ = record(p, 4)) return st_;
     p->timed_degrid = true;
@@ -919,8 +1107,10 @@ int p9idg_destroy(p9idg_plan* p) {
     if (p->have_fft_one) (void)hipfftDestroy(p->fft_one);
     dev_free(p->d_uvw);
     dev_free(p->d_wavenumbers);
-    dev_free(p->d_meta);
-    dev_free(p->d_order);
+    dev_free(p->direct.d_meta);
+    dev_free(p->direct.d_order);
+    free_items(p->direct);
+    free_items(p->rs_view);
     dev_free(p->d_vis);
     dev_free(p->d_model_vis);
     dev_free(p->d_grid);
@@ -935,10 +1125,10 @@ int p9idg_destroy(p9idg_plan* p) {
     dev_free(p->d_flags);
     dev_free(p->d_counter);
     dev_free(p->d_resid);
+    dev_free(p->d_rs_chunks);
+    dev_free(p->d_rs_rows);
     for (auto& f : p->d_fp) dev_free(f);
     drop_graph(p);
-    dev_free(p->d_items_grid);
-    dev_free(p->d_items_degrid);
     dev_free(p->d_scratch);
     for (auto& g : p->gather) free_gather(g);
     if (p->d_staging) (void)hipFree(p->d_staging);
@@ -957,6 +1147,10 @@ int p9idg_set_kernel(p9idg_plan* p, int32_t kernel) {
         return fail(P9IDG_ERR_ARGUMENT, "unknown kernel");
     if (p->kernel != kernel) drop_graph(p);  // a captured step holds the old kernel
     p->kernel = kernel;
+    if (p->have_obs && p->resampled != want_resample(p)) {
+        p->resampled = !p->resampled;
+        return upload_items(p);
+    }
     return P9IDG_OK;
 }
 
@@ -1047,8 +1241,8 @@ int p9idg_set_observation(p9idg_plan* p, const double* uvw, int32_t B, int32_t T
         p->alloc_wn = 0;
     }
     if (p->alloc_sub != n_sub) {
-        dev_free(p->d_meta);
-        dev_free(p->d_order);
+        dev_free(p->direct.d_meta);
+        dev_free(p->direct.d_order);
         p->alloc_sub = 0;
     }
     p->have_obs = false;
@@ -1057,7 +1251,7 @@ int p9idg_set_observation(p9idg_plan* p, const double* uvw, int32_t B, int32_t T
     p->alloc_uvw = n_uvw;
     if ((st = dev_alloc(&p->d_wavenumbers, (size_t)C))) return st;
     p->alloc_wn = (size_t)C;
-    if ((st = dev_alloc(&p->d_meta, n_sub)) || (st = dev_alloc(&p->d_order, n_sub))) return st;
+    if ((st = dev_alloc(&p->direct.d_meta, n_sub)) || (st = dev_alloc(&p->direct.d_order, n_sub))) return st;
     p->alloc_sub = n_sub;
     if ((st = dev_alloc(&p->d_vis, n_vis)) || (st = dev_alloc(&p->d_model_vis, n_vis))) return st;
     p->alloc_vis = n_vis;
@@ -1069,18 +1263,11 @@ int p9idg_set_observation(p9idg_plan* p, const double* uvw, int32_t B, int32_t T
         const double dk = (k[C - 1] - k[0]) / (C - 1), tol = 1e-12 * std::fabs(k[C - 1]);
         for (int i = 0; i < C; i++) uniform = uniform && std::fabs(k[i] - (k[0] + i * dk)) <= tol;
     }
-    // schedule: most visibilities first
-    std::vector<int32_t> order(nsub);
-    std::iota(order.begin(), order.end(), 0);
-    std::stable_sort(order.begin(), order.end(), [&](int32_t a, int32_t b) {
-        return meta[a].time_sample_count > meta[b].time_sample_count;
-    });
     P9_HIP(hipMemcpyAsync(p->d_uvw, uvw, (size_t)B * T * 3 * sizeof(double), hipMemcpyHostToDevice, p->stream));
     P9_HIP(hipMemcpyAsync(p->d_wavenumbers, k.data(), C * sizeof(double), hipMemcpyHostToDevice, p->stream));
-    if (nsub > 0) {
-        P9_HIP(hipMemcpyAsync(p->d_meta, meta, nsub * sizeof(p9idg_subgrid), hipMemcpyHostToDevice, p->stream));
-        P9_HIP(hipMemcpyAsync(p->d_order, order.data(), nsub * sizeof(int32_t), hipMemcpyHostToDevice, p->stream));
-    }
+    p->direct.meta.assign(meta, meta + nsub);
+    if (int st = upload_view(p, p->direct)) return st;
+    if (int st = build_resample(p, T, C, freq)) return st;
     P9_HIP(hipStreamSynchronize(p->stream));
     p->chan_uniform = uniform;
     p->B = B;
@@ -1089,8 +1276,7 @@ int p9idg_set_observation(p9idg_plan* p, const double* uvw, int32_t B, int32_t T
     p->nsub = nsub;
     p->plain_adder_ok = plain_ok;
     p->gridded_vis = gridded;
-    p->meta_host.assign(meta, meta + nsub);
-    p->order_host = order;
+    p->resampled = want_resample(p);
     mark_unknown(p);
     if (int st = build_footprints(p, meta, nsub)) return st;
     if (int st = upload_items(p)) return st;
@@ -1121,7 +1307,7 @@ static int degrid_host(p9idg_plan* p, const double* grid, double* vis_out, int m
     if (!vis_out) return fail(P9IDG_ERR_ARGUMENT, "vis_out is NULL");
     DeviceGuard dg(p->device);
     if (int st = upload_grid_c128(p, grid)) return st;
-    if (int st = do_exec_degrid(p, mode)) return st;
+    if (int st = do_exec_degrid(p, mode, true)) return st;
     return download_c128(p, p->d_model_vis, vis_out, vis_elems(p));
 }
 
@@ -1194,7 +1380,7 @@ int p9idg_image_to_vis(p9idg_plan* p, const float* img, double* vis_out) {
     P9_HIP(hipMemcpyAsync(p->d_image, img, grid_elems(p) * sizeof(float), hipMemcpyHostToDevice,
                           p->stream));
     if (int st = do_image_to_grid(p)) return st;
-    if (int st = do_exec_degrid(p, P9IDG_DEGRID_WSTACK)) return st;
+    if (int st = do_exec_degrid(p, P9IDG_DEGRID_WSTACK, true)) return st;
     return download_c128(p, p->d_model_vis, vis_out, vis_elems(p));
 }
 
@@ -1613,6 +1799,7 @@ struct p9idg_batch {
     struct Group {
         int S = 0, kernel = 0, workgroups = 0, workgroups_degrid = 0;
         std::vector<int> members;  // plan indices; item.inst indexes this list
+        std::vector<bool> resampled;  // per member, at prepare
         KernelArgs* d_args_grid = nullptr;
         KernelArgs* d_args_degrid = nullptr;
         WorkItem* d_items_grid = nullptr;
@@ -1697,13 +1884,22 @@ int batch_launch_groups(p9idg_batch* b, bool grid) {
         auto& g = b->groups[i];
         hipStream_t st = fan ? b->side[i] : b->stream;
         if (fan) P9_HIP(hipStreamWaitEvent(st, b->fork, 0));
-        hipError_t e;
+        hipError_t e = hipSuccess;
         if (grid) {
+            for (size_t m = 0; m < g.members.size(); m++) {
+                const p9idg_plan* p = b->plans[g.members[m]];
+                if (g.resampled[m]) P9_HIP(launch_resample_gather(p->rs, p->C, p->d_vis, p->d_rs_vis, st));
+            }
             BatchArgs ba{g.d_args_grid, g.d_items_grid, g.n_grid, g.d_counter};
             e = launch_grid_batch(ba, g.S, g.kernel, g.workgroups, st);
         } else {
             BatchArgs ba{g.d_args_degrid, g.d_items_degrid, g.n_degrid, g.d_counter};
             e = launch_degrid_batch(ba, g.S, g.kernel, g.workgroups_degrid, st);
+            for (size_t m = 0; m < g.members.size(); m++) {
+                const p9idg_plan* p = b->plans[g.members[m]];
+                if (g.resampled[m] && e == hipSuccess)
+                    e = launch_resample_spread(p->rs, p->C, p->d_rs_vis, p->d_model_vis, st);
+            }
         }
         if (e != hipSuccess) return hip_fail(e, grid ? "batched gridder launch" : "batched degridder launch");
         if (fan) P9_HIP(hipEventRecord(b->side_done[i], st));
@@ -1828,17 +2024,19 @@ int p9idg_batch_prepare(p9idg_batch* b, int32_t grid_mode, int32_t degrid_mode) 
         std::vector<WorkItem> ig, id;
         for (int m = 0; m < (int)g.members.size(); m++) {
             p9idg_plan* p = b->plans[g.members[m]];
-            KernelArgs a = make_args(p, grid_mode);
-            a.vis = p->d_vis;
+            g.resampled.push_back(p->resampled);
+            const p9idg_plan::View& v = active_view(p);
+            KernelArgs a = make_args(p, grid_mode, p->resampled);
+            if (!p->resampled) a.vis = p->d_vis;
             a.grid = grid_mode == P9IDG_GRID_WSTACK ? p->d_layers : p->d_grid;
             ag.push_back(a);
-            KernelArgs d = make_args(p, degrid_mode);
+            KernelArgs d = make_args(p, degrid_mode, p->resampled);
             ad.push_back(d);
-            for (WorkItem w : make_items(p->meta_host, p->order_host, p->C, p->grid_chunk)) {
+            for (WorkItem w : make_items(v.meta, v.order, p->C, p->grid_chunk)) {
                 w.inst = m;
                 ig.push_back(w);
             }
-            for (WorkItem w : make_items(p->meta_host, p->order_host, p->C, p->degrid_chunk)) {
+            for (WorkItem w : make_items(v.meta, v.order, p->C, p->degrid_chunk)) {
                 w.inst = m;
                 id.push_back(w);
             }

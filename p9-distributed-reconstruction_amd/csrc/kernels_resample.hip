@@ -1,0 +1,370 @@
+// Time resampling of the visibilities around the gridder and degridder.
+//
+// Within a subgrid a baseline's phasor at any pixel (Gridder.cs:62-70),
+//   f(t) = exp(2 pi i (off - k (u(t) l + v(t) m + w(t) n))),
+// is a smooth function of the timestep: Earth rotation moves the uv point by
+// a few hundredths of a grid pixel per step.  Over a chunk of `len` steps it
+// therefore equals its Chebyshev interpolant f(t) = sum_j W[t][j] f(t_j) on
+// `nodes` < len nodes t_j, with real weights W that depend on (len, nodes)
+// only, and the subgrid sums rearrange to
+//   gridder:   sum_t V[t] f(t)      = sum_j (sum_t W[t][j] V[t]) f(t_j)
+//   degridder: conj f(t) contracted = sum_j W[t][j] (conj f(t_j) contracted)
+// so the gridder reads `nodes` rows of channels per chunk instead of `len`,
+// and the degridder's rows are interpolated back to the timesteps.
+// Observations whose tracks move 0.01-0.1 pixel per step keep 1/6-1/10 of
+// their rows.
+//
+// Which chunks qualify is measured, not assumed: analyse_kernel evaluates the
+// interpolant at every timestep of the chunk, at the four corner pixels (where
+// the phase varies most) and the highest channel, against the phasor of the
+// track itself, and takes the smallest number of nodes whose error is below
+// kResampleTol everywhere.  A track with a jump, noise or a gap fails the test
+// and keeps its rows as they are.
+#include "device_common.h"
+
+namespace p9idg {
+namespace dev {
+
+constexpr int kMaxLen = kResampleMaxLen;
+constexpr int kMaxNodes = kResampleMaxNodes;
+// samples that the track itself is interpolated from (degree 11: exact to
+// ~1e-14 of the track for chunks of an hour)
+constexpr int kBase = 12;
+
+typedef float rs_f32x4 __attribute__((ext_vector_type(4)));
+
+// Angle of timestep t in a chunk of `len` (x = cos(angle) runs from 1 to -1)
+// and of Chebyshev node j of J.
+__device__ __forceinline__ double angle_of(double t, int len) {
+    const double x = 1.0 - 2.0 * t / (double)(len - 1);
+    return acos(fmin(1.0, fmax(-1.0, x)));
+}
+__device__ __forceinline__ double node_angle(int j, int J) { return (kTwoPi / 4.0) * (double)(2 * j + 1) / (double)J; }
+
+// Cardinal function of node j at angle th: with D = th - th_j,
+//   w = sin(th_j) sin(J D) / (2 J sin((th + th_j) / 2) sin(D / 2)),
+// the Lagrange polynomial of the node written without a difference of cosines.
+__device__ __forceinline__ double cardinal(double th, double thj, int J) {
+    const double d = th - thj;
+    const double ratio = fabs(d) < 1e-12 ? 2.0 * (double)J : sin((double)J * d) / sin(0.5 * d);
+    return sin(thj) * ratio / (2.0 * (double)J * sin(0.5 * (th + thj)));
+}
+
+// The chunk's base samples: distinct timesteps near Chebyshev nodes.
+__device__ __forceinline__ int base_sample(int b, int nb, int len) {
+    if (nb >= len) return b;
+    const double t = 0.5 * (double)(len - 1) * (1.0 - cos((kTwoPi / 2.0) * (double)b / (double)(nb - 1)));
+    int s = (int)rint(t);
+    return min(max(s, b), len - nb + b);  // distinct: at least b from either end
+}
+
+// The track at time t from the nb base samples (Lagrange form, FP64).
+__device__ __forceinline__ void track_at(double t, const double (*base)[3], const int* bt, int nb, double out[3]) {
+    out[0] = out[1] = out[2] = 0.0;
+    for (int b = 0; b < nb; b++) {
+        double w = 1.0;
+        for (int q = 0; q < nb; q++)
+            if (q != b) w *= (t - (double)bt[q]) / (double)(bt[b] - bt[q]);
+        out[0] += w * base[b][0];
+        out[1] += w * base[b][1];
+        out[2] += w * base[b][2];
+    }
+}
+
+__device__ __forceinline__ double block_max_d(double v, double* red) {
+    for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o));
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+    __syncthreads();
+    return fmax(fmax(red[0], red[1]), fmax(red[2], red[3]));
+}
+
+// One workgroup per chunk (thread t: timestep t): the smallest multiple of
+// four nodes whose interpolant reproduces the corner phasors of every
+// timestep to kResampleTol, or 0.  kl, kn: highest wavenumber / 2 pi times the
+// corner pixel's l and n.
+__global__ __launch_bounds__(kMaxLen) void analyse_kernel(const ResampleChunk* chunks, const double* uvw, double kl,
+                                                          double kn, int32_t* nodes_out) {
+    static_assert(kMaxLen == 256, "four waves reduce");
+    __shared__ double s_base[kBase][3];
+    __shared__ int s_bt[kBase];
+    __shared__ double2 s_node[kMaxNodes][4];
+    __shared__ double s_red[4];
+    const ResampleChunk c = chunks[blockIdx.x];
+    const int tid = threadIdx.x, len = c.len;
+    const int nb = min(kBase, len);
+    const double* track = uvw + (size_t)c.src * 3;
+    if (tid < nb) {
+        const int t = base_sample(tid, nb, len);
+        s_bt[tid] = t;
+        for (int k = 0; k < 3; k++) s_base[tid][k] = track[(size_t)t * 3 + k];
+    }
+    __syncthreads();
+    // this timestep's corner phases relative to the chunk's first sample, in turns
+    const int tc = min(tid, len - 1);
+    const double u0 = s_base[0][0], v0 = s_base[0][1], w0 = s_base[0][2];
+    const double du = (track[(size_t)tc * 3] - u0) * kl, dv = (track[(size_t)tc * 3 + 1] - v0) * kl;
+    const double dw = (track[(size_t)tc * 3 + 2] - w0) * kn;
+    double2 own[4];
+    double span = 0.0;
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const double ph = ((q & 1) ? -du : du) + ((q & 2) ? -dv : dv) + dw;
+        sincospi(2.0 * ph, &own[q].y, &own[q].x);
+        span = fmax(span, fabs(ph));
+    }
+    // not finite: fails every test below
+    const bool bad = !(fabs(du) < 1e12 && fabs(dv) < 1e12 && fabs(dw) < 1e12);
+    // start where the Chebyshev coefficients 2 (z / 2)^J / J! of exp(i z s) fall
+    // below the tolerance for z of half the span from the first sample
+    span = block_max_d(bad ? 1e9 : span, s_red);
+    const double z = (kTwoPi / 2.0) * span;
+    int start = 1;
+    double term = 2.0 * (0.5 * z);
+    while (start < kMaxNodes && (term > kResampleTol || (double)start < 0.5 * z)) {
+        start++;
+        term *= 0.5 * z / (double)start;
+    }
+    const int limit = min(kMaxNodes, (int)(kResampleKeep * (double)len)) & ~3;
+    int found = 0;
+    const double th = angle_of((double)tc, len);
+    for (int J = (start + 3) & ~3; J <= limit; J += 4) {  // uniform
+        __syncthreads();  // the previous candidate's nodes are read
+        if (tid < J) {
+            double p[3];
+            track_at(0.5 * (double)(len - 1) * (1.0 - cos(node_angle(tid, J))), s_base, s_bt, nb, p);
+            const double nu = (p[0] - u0) * kl, nv = (p[1] - v0) * kl, nw = (p[2] - w0) * kn;
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const double ph = ((q & 1) ? -nu : nu) + ((q & 2) ? -nv : nv) + nw;
+                sincospi(2.0 * ph, &s_node[tid][q].y, &s_node[tid][q].x);
+            }
+        }
+        __syncthreads();
+        double2 e[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) e[q] = own[q];
+        for (int j = 0; j < J; j++) {
+            const double w = cardinal(th, node_angle(j, J), J);
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                e[q].x -= w * s_node[j][q].x;
+                e[q].y -= w * s_node[j][q].y;
+            }
+        }
+        double err = 0.0;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const double m = fmax(fabs(e[q].x), fabs(e[q].y));
+            err = m <= kResampleTol ? fmax(err, m) : 1e9;  // NaN counts as a failure
+            if (err > kResampleTol) break;
+        }
+        if (block_max_d(err, s_red) <= kResampleTol) {
+            found = J;
+            break;
+        }
+    }
+    if (tid == 0) nodes_out[blockIdx.x] = found;
+}
+
+// Weights of one (len, nodes) pair per workgroup, FP64 rounded to float, in
+// both orders: to[j][t] for the degridder's interpolation behind from[t][j]
+// for the gridder's sums.
+__global__ void weights_kernel(const ResamplePair* pairs, float* weights) {
+    const ResamplePair p = pairs[blockIdx.x];
+    float* from = weights + p.offset;
+    float* to = from + (size_t)p.len * p.nodes;
+    for (int i = threadIdx.x; i < p.len * p.nodes; i += blockDim.x) {
+        const int t = i / p.nodes, j = i - t * p.nodes;
+        const float w = (float)cardinal(angle_of((double)t, p.len), node_angle(j, p.nodes), p.nodes);
+        from[i] = w;
+        to[(size_t)j * p.len + t] = w;
+    }
+}
+
+// Track rows of the resampled observation: the track at the nodes, or the
+// chunk's own rows where it is not resampled.
+__global__ __launch_bounds__(kMaxLen) void node_track_kernel(const ResampleChunk* chunks, const double* uvw, double* out) {
+    __shared__ double s_base[kBase][3];
+    __shared__ int s_bt[kBase];
+    const ResampleChunk c = chunks[blockIdx.x];
+    const int tid = threadIdx.x, nb = min(kBase, c.len);
+    const double* track = uvw + (size_t)c.src * 3;
+    if (c.nodes == 0) {
+        for (int i = tid; i < 3 * c.len; i += blockDim.x) out[(size_t)c.dst * 3 + i] = track[i];
+        return;
+    }
+    if (tid < nb) {
+        const int t = base_sample(tid, nb, c.len);
+        s_bt[tid] = t;
+        for (int k = 0; k < 3; k++) s_base[tid][k] = track[(size_t)t * 3 + k];
+    }
+    __syncthreads();
+    if (tid < c.nodes) {
+        double p[3];
+        track_at(0.5 * (double)(c.len - 1) * (1.0 - cos(node_angle(tid, c.nodes))), s_base, s_bt, nb, p);
+        for (int k = 0; k < 3; k++) out[((size_t)c.dst + tid) * 3 + k] = p[k];
+    }
+}
+
+// Rows of one chunk copied as they are (16 floats per column tile).
+__device__ __forceinline__ void copy_rows(const float* in, float* out, int rows, int width, int n, int g, bool col) {
+    if (!col) return;
+    for (int r = g; r < rows; r += 4) out[(size_t)r * width + n] = in[(size_t)r * width + n];
+}
+
+// One chunk's 16 columns for up to 16 Q nodes, in one sweep over the timesteps.
+template <int Q>
+__device__ __forceinline__ void gather_chunk(const float* src, const float* w, float* dst, int len, int J, int width, int n,
+                                             int nc, int m, int g, bool col) {
+    rs_f32x4 acc[Q];
+    int jq[Q];
+#pragma unroll
+    for (int q = 0; q < Q; q++) {
+        acc[q] = (rs_f32x4){};
+        jq[q] = min(16 * q + m, J - 1);
+    }
+    for (int t0 = 0; t0 < len; t0 += 16) {
+        float v[4], wt[4][Q];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const int t = t0 + 4 * k + g, tt = min(t, len - 1);
+            v[k] = src[(size_t)tt * width + nc];
+#pragma unroll
+            for (int q = 0; q < Q; q++) wt[k][q] = w[(size_t)tt * J + jq[q]];
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const float b = t0 + 4 * k + g < len ? v[k] : 0.f;
+#pragma unroll
+            for (int q = 0; q < Q; q++) acc[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(wt[k][q], b, acc[q], 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < Q; q++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int j = 16 * q + 4 * g + r;
+            if (j < J && col) dst[(size_t)j * width + n] = acc[q][r];
+        }
+}
+
+// out[j][n] = sum_t W[t][j] in[t][n] for every chunk, n over the real columns
+// of a row of channels, on v_mfma_f32_16x16x4_f32: FP32 products and sums on
+// the matrix cores, so the visibilities and weights keep 24 bits.  A wave owns
+// a chunk and 16 columns (8 channels): A = W (16 nodes x 4 timesteps), B = 4
+// rows of visibilities straight from HBM (256 contiguous bytes per load at 8
+// channels).
+__global__ __launch_bounds__(256) void gather_rows_kernel(const ResampleChunk* chunks, int nchunks, int ntiles,
+                                                          const float* weights, int width, const float* in, float* out) {
+    const int unit = (int)(blockIdx.x * 4 + (threadIdx.x >> 6));
+    const int ci = unit / ntiles;
+    if (ci >= nchunks) return;  // whole waves
+    const ResampleChunk c = chunks[ci];
+    const int lane = threadIdx.x & 63, m = lane & 15, g = lane >> 4;
+    const int n = (unit - ci * ntiles) * 16 + m;
+    const bool col = n < width;
+    const float* src = in + (size_t)c.src * width;
+    float* dst = out + (size_t)c.dst * width;
+    if (c.nodes == 0) return copy_rows(src, dst, c.len, width, n, g, col);
+    const float* w = weights + c.weights;
+    const int J = c.nodes, len = c.len, nc = col ? n : 0;
+    switch ((J + 15) >> 4) {  // uniform
+        case 1: return gather_chunk<1>(src, w, dst, len, J, width, n, nc, m, g, col);
+        case 2: return gather_chunk<2>(src, w, dst, len, J, width, n, nc, m, g, col);
+        case 3: return gather_chunk<3>(src, w, dst, len, J, width, n, nc, m, g, col);
+        default: return gather_chunk<4>(src, w, dst, len, J, width, n, nc, m, g, col);
+    }
+}
+
+// One chunk's 16 columns from up to 16 Q node rows, held in registers.
+template <int Q>
+__device__ __forceinline__ void spread_chunk(const float* src, const float* w, float* dst, int len, int J, int width, int n,
+                                             int nc, int m, int g, bool col) {
+    float b[4 * Q];
+#pragma unroll
+    for (int k = 0; k < 4 * Q; k++) b[k] = src[(size_t)min(4 * k + g, J - 1) * width + nc];
+    for (int t0 = 0; t0 < len; t0 += 16) {
+        const int ta = min(t0 + m, len - 1);
+        float a[4 * Q];
+#pragma unroll
+        for (int k = 0; k < 4 * Q; k++) {
+            const float wt = w[(size_t)min(4 * k + g, J - 1) * len + ta];
+            a[k] = 4 * k + g < J ? wt : 0.f;
+        }
+        rs_f32x4 acc[2] = {(rs_f32x4){}, (rs_f32x4){}};
+#pragma unroll
+        for (int k = 0; k < 4 * Q; k++) acc[k & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[k], b[k], acc[k & 1], 0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int t = t0 + 4 * g + r;
+            if (t < len && col) dst[(size_t)t * width + n] = acc[0][r] + acc[1][r];
+        }
+    }
+}
+
+// out[t][n] = sum_j W[t][j] in[j][n]: the degridded nodes interpolated to the
+// timesteps, 16 timesteps x 16 columns per MFMA tile, the chunk's node rows
+// held in registers as the B operands.
+__global__ __launch_bounds__(256) void spread_rows_kernel(const ResampleChunk* chunks, int nchunks, int ntiles,
+                                                          const float* weights, int width, const float* in, float* out) {
+    const int unit = (int)(blockIdx.x * 4 + (threadIdx.x >> 6));
+    const int ci = unit / ntiles;
+    if (ci >= nchunks) return;
+    const ResampleChunk c = chunks[ci];
+    const int lane = threadIdx.x & 63, m = lane & 15, g = lane >> 4;
+    const int n = (unit - ci * ntiles) * 16 + m;
+    const bool col = n < width;
+    const float* src = in + (size_t)c.dst * width;
+    float* dst = out + (size_t)c.src * width;
+    if (c.nodes == 0) return copy_rows(src, dst, c.len, width, n, g, col);
+    const int J = c.nodes, len = c.len, nc = col ? n : 0;
+    const float* w = weights + c.weights + (size_t)len * J;  // [j][t]
+    switch ((J + 15) >> 4) {  // uniform
+        case 1: return spread_chunk<1>(src, w, dst, len, J, width, n, nc, m, g, col);
+        case 2: return spread_chunk<2>(src, w, dst, len, J, width, n, nc, m, g, col);
+        case 3: return spread_chunk<3>(src, w, dst, len, J, width, n, nc, m, g, col);
+        default: return spread_chunk<4>(src, w, dst, len, J, width, n, nc, m, g, col);
+    }
+}
+
+}  // namespace dev
+
+hipError_t launch_resample_analyse(const ResampleChunk* chunks, int nchunks, const double* uvw, double kl, double kn,
+                                   int32_t* nodes, hipStream_t st) {
+    if (nchunks <= 0) return hipSuccess;
+    hipLaunchKernelGGL(dev::analyse_kernel, dim3(nchunks), dim3(kResampleMaxLen), 0, st, chunks, uvw, kl, kn, nodes);
+    return hipGetLastError();
+}
+hipError_t launch_resample_tables(const ResamplePair* pairs, int npairs, float* weights, const ResampleChunk* chunks,
+                                  int nchunks, const double* uvw, double* out, hipStream_t st) {
+    if (npairs > 0) {
+        hipLaunchKernelGGL(dev::weights_kernel, dim3(npairs), dim3(256), 0, st, pairs, weights);
+        if (hipError_t e = hipGetLastError()) return e;
+    }
+    if (nchunks > 0)
+        hipLaunchKernelGGL(dev::node_track_kernel, dim3(nchunks), dim3(kResampleMaxLen), 0, st, chunks, uvw, out);
+    return hipGetLastError();
+}
+namespace {
+unsigned row_blocks(const Resample& r, int C) {
+    const int64_t units = (int64_t)r.nchunks * ((2 * C + 15) / 16);
+    return (unsigned)((units + 3) / 4);
+}
+}  // namespace
+hipError_t launch_resample_gather(const Resample& r, int C, const float2* vis, float2* out, hipStream_t st) {
+    if (r.nchunks <= 0) return hipSuccess;
+    hipLaunchKernelGGL(dev::gather_rows_kernel, dim3(row_blocks(r, C)), dim3(256), 0, st, r.chunks, r.nchunks,
+                       (2 * C + 15) / 16, r.weights, 2 * C, reinterpret_cast<const float*>(vis),
+                       reinterpret_cast<float*>(out));
+    return hipGetLastError();
+}
+hipError_t launch_resample_spread(const Resample& r, int C, const float2* rows, float2* vis, hipStream_t st) {
+    if (r.nchunks <= 0) return hipSuccess;
+    hipLaunchKernelGGL(dev::spread_rows_kernel, dim3(row_blocks(r, C)), dim3(256), 0, st, r.chunks, r.nchunks,
+                       (2 * C + 15) / 16, r.weights, 2 * C, reinterpret_cast<const float*>(rows),
+                       reinterpret_cast<float*>(vis));
+    return hipGetLastError();
+}
+
+}  // namespace p9idg

@@ -81,6 +81,32 @@ struct SlotCorner {
     int32_t y0, x0;
 };
 
+// Time resampling (kernels_resample.hip): `len` consecutive rows (timesteps x
+// C channels) of the observation from row `src` become `nodes` rows from row
+// `dst` of the resampled observation; nodes 0: the rows are copied.  weights:
+// float offset of the (len, nodes) pair's tables.
+constexpr int kResampleMaxLen = 256;
+constexpr int kResampleMaxNodes = 64;
+// Largest interpolation error of a unit phasor: below the rounding of the
+// FP32 weights and sums (6e-8).
+constexpr double kResampleTol = 1e-8;
+// A chunk is resampled if that leaves at most this share of its rows.
+constexpr double kResampleKeep = 0.7;
+struct ResampleChunk {
+    int64_t src, weights;
+    int32_t dst, len, nodes, pad;
+};
+struct ResamplePair {
+    int64_t offset;  // from[len][nodes], then to[nodes][len]
+    int32_t len, nodes;
+};
+// The device tables of a plan's resampled observation.
+struct Resample {
+    ResampleChunk* chunks = nullptr;
+    float* weights = nullptr;
+    int32_t nchunks = 0;
+};
+
 // Kernel launch parameters shared by host and device code.
 struct KernelArgs {
     const p9idg_subgrid* meta;
@@ -167,6 +193,17 @@ hipError_t launch_zero_boxes(float2* base, const Box* boxes, int nboxes, int G, 
 hipError_t launch_gather_slots(const GatherBin* bins, int nbins, const GatherChunk* chunks, int nchunks,
                                const int32_t* slots, const SlotCorner* corners, const float2* scratch, int S, int G,
                                float2* partial, float2* base, hipStream_t st);
+// nodes[i]: nodes that chunk i needs (0: not resampled).  kl, kn: highest
+// wavenumber / 2 pi times the corner pixel's l and n.
+hipError_t launch_resample_analyse(const ResampleChunk* chunks, int nchunks, const double* uvw, double kl, double kn,
+                                   int32_t* nodes, hipStream_t st);
+// The pairs' weight tables and the resampled observation's track rows.
+hipError_t launch_resample_tables(const ResamplePair* pairs, int npairs, float* weights, const ResampleChunk* chunks,
+                                  int nchunks, const double* uvw, double* out, hipStream_t st);
+// Visibilities [rows][C] -> resampled rows (gridder input), and the degridded
+// rows -> visibilities of every covered timestep.
+hipError_t launch_resample_gather(const Resample& r, int C, const float2* vis, float2* out, hipStream_t st);
+hipError_t launch_resample_spread(const Resample& r, int C, const float2* rows, float2* vis, hipStream_t st);
 hipError_t launch_sum_layers(const float2* layers, int L, size_t GG, float2* out, hipStream_t st);
 hipError_t launch_sum_layer_boxes(const float2* layers, const Box* boxes, int nboxes, int G, Box u,
                                   float2* out, hipStream_t st);
