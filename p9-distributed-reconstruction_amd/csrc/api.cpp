@@ -112,6 +112,7 @@ struct p9idg_plan {
     Box fp_union[3] = {};                         // bounding box of each mode's boxes
     float2* d_lsum = nullptr;                     // layer sum for the w-stacked ToImage
     int32_t use_queue = 1;
+    bool launch_chosen = false;  // by p9idg_set_launch or p9idg_autotune
     int32_t grid_chunk = 2048;
     int32_t degrid_chunk = 2048;
     int32_t workgroups = 0;         // gridder's persistent workgroups (0: CUs x occupancy)
@@ -614,9 +615,17 @@ int upload_items(p9idg_plan* p) {
     return P9IDG_OK;
 }
 
+// Whether launches run persistent workgroups over the work queue.  A resampled
+// observation's subgrids are short (a few hundred rows at most), so unless the
+// caller has chosen a launch shape each is one workgroup that the hardware
+// dispatches: the queue's claims would be a tenth of its time.  Split BF16, grid /
+// degrid us with the queue -> without: 3072^2 207 / 195 -> 187 / 178, 512^2 106 /
+// 72 -> 69 / 65, 2048^2 68 / 49 -> 57 / 41.
+bool queue_on(const p9idg_plan* p) { return p->use_queue != 0 && (p->launch_chosen || !p->resampled); }
+
 LaunchCfg launch_cfg(const p9idg_plan* p, bool grid) {
     LaunchCfg cfg;
-    cfg.queue = p->use_queue != 0;
+    cfg.queue = queue_on(p);
     cfg.workgroups = grid ? p->workgroups : p->workgroups_degrid;
     return cfg;
 }
@@ -668,7 +677,7 @@ int prepare_gather(p9idg_plan* p, int mode) {
     const int S = p->c.subgrid_size, G = p->c.grid_size, L = p->c.wlayer_count;
     const p9idg_plan::View& v = active_view(p);
     const std::vector<WorkItem> items =
-        make_items(v.meta, v.order, p->C, p->use_queue ? p->grid_chunk : 0);
+        make_items(v.meta, v.order, p->C, queue_on(p) ? p->grid_chunk : 0);
     const size_t need = items.size() * (size_t)S * S;
     P9_HIP(hipStreamSynchronize(p->stream));  // queued launches may still use the old buffers
     if (p->alloc_scratch != need) {
@@ -1174,6 +1183,7 @@ int p9idg_set_launch(p9idg_plan* p, int32_t queue, int32_t grid_chunk, int32_t d
     if (grid_chunk < 0 || degrid_chunk < 0 || workgroups < 0)
         return fail(P9IDG_ERR_ARGUMENT, "negative launch parameter");
     p->use_queue = queue != 0;
+    p->launch_chosen = true;
     p->grid_chunk = grid_chunk;
     p->degrid_chunk = degrid_chunk;
     p->workgroups = workgroups;
@@ -1586,6 +1596,7 @@ int p9idg_autotune(p9idg_plan* p, int32_t reps, float* grid_ms, float* degrid_ms
     Cand pick[2] = {{p->use_queue, p->grid_chunk, p->workgroups},
                     {p->use_queue, p->degrid_chunk, p->workgroups_degrid}};
     const int32_t q0 = p->use_queue, g0 = p->grid_chunk, d0 = p->degrid_chunk, w0 = p->workgroups;
+    p->launch_chosen = true;
     for (const Cand& c : cands) {
         p->use_queue = c.queue;
         p->grid_chunk = c.chunk;
