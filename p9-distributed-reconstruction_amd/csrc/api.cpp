@@ -111,6 +111,11 @@ struct p9idg_plan {
     int32_t n_fp[3] = {0, 0, 0};
     Box fp_union[3] = {};                         // bounding box of each mode's boxes
     float2* d_lsum = nullptr;                     // layer sum for the w-stacked ToImage
+    // line transforms (kernels_fft.hip), where the grid size has them
+    LinePlan line{};
+    bool have_line = false;
+    float2* d_line_tw = nullptr;
+    float2* d_line_mid = nullptr;
     int32_t use_queue = 1;
     bool launch_chosen = false;  // by p9idg_set_launch or p9idg_autotune
     int32_t grid_chunk = 2048;
@@ -430,7 +435,7 @@ int zero_target(p9idg_plan* p, int mode, float2* target, size_t n) {
     } else if (fp >= 0) {
         P9_HIP(launch_zero_boxes(target, p->d_fp[fp], p->n_fp[fp], p->c.grid_size, p->stream));
     }
-    clean = !p->capturing;
+    clean = true;  // while capturing: until p9idg_capture_cycle ends
     fp = mode;
     return P9IDG_OK;
 }
@@ -440,6 +445,22 @@ int ensure_fft_one(p9idg_plan* p) {
     P9_FFT(hipfftPlan2d(&p->fft_one, p->c.grid_size, p->c.grid_size, HIPFFT_C2C));
     P9_FFT(hipfftSetStream(p->fft_one, p->stream));
     p->have_fft_one = true;
+    return P9IDG_OK;
+}
+
+// The line transforms' twiddles and buffer (allocated once: a recorded graph
+// may hold them).
+int ensure_line(p9idg_plan* p) {
+    if (p->d_line_tw && p->d_line_mid) return P9IDG_OK;
+    const int G = p->c.grid_size;
+    std::vector<float2> tw(G);
+    for (int k = 0; k < G; k++) {
+        const double a = 2.0 * M_PI * (double)k / (double)G;
+        tw[k] = make_float2((float)std::cos(a), (float)std::sin(a));
+    }
+    if (int st = dev_alloc(&p->d_line_mid, (size_t)G * std::max(G, line_pitch(G)))) return st;
+    if (int st = dev_alloc(&p->d_line_tw, (size_t)G)) return st;
+    P9_HIP(hipMemcpy(p->d_line_tw, tw.data(), G * sizeof(float2), hipMemcpyHostToDevice));
     return P9IDG_OK;
 }
 
@@ -851,28 +872,27 @@ int do_exec_degrid(p9idg_plan* p, int mode, bool direct = false) {
 // FFT.WStackIFFTFloat (FFT.cs:188-215): sum over layers of
 // (float)(Re(IFFT(layer)) / N).  The inverse FFT is linear and applies no
 // per-layer w-screen, so it runs once on the sum of the layers (identical up
-// to the per-layer float rounding).  The layers are left as they are; when
-// their footprint is known only the union of the footprint boxes is summed.
+// to the per-layer float rounding).  The layers are left as they are.
 int layers_image(p9idg_plan* p, double inv_n, int shift) {
     const int G = p->c.grid_size;
-    const int W = P9IDG_GRID_WSTACK;
     if (int st = dev_alloc(&p->d_lsum, grid_elems(p))) return st;
     if (int st = ensure_fft_one(p)) return st;
-    if (p->layers_clean && p->layers_dirty_fp == W && !p->capturing) {
-        P9_HIP(launch_fill_zero(p->d_lsum, grid_elems(p), p->stream));
-        if (p->n_fp[W] > 0)
-            P9_HIP(launch_sum_layer_boxes(p->d_layers, p->d_fp[W], p->n_fp[W], G, p->fp_union[W], p->d_lsum,
-                                          p->stream));
-    } else {
-        P9_HIP(launch_sum_layers(p->d_layers, p->c.wlayer_count, grid_elems(p), p->d_lsum, p->stream));
-    }
+    P9_HIP(launch_sum_layers(p->d_layers, p->c.wlayer_count, grid_elems(p), p->d_lsum, p->stream));
     P9_FFT(hipfftExecC2C(p->fft_one, reinterpret_cast<hipfftComplex*>(p->d_lsum),
                          reinterpret_cast<hipfftComplex*>(p->d_lsum), HIPFFT_BACKWARD));
     P9_HIP(launch_layers_to_image(p->d_lsum, 1, G, inv_n, shift, p->d_image, p->stream));
     return P9IDG_OK;
 }
 
-// Inverse FFT of the grid buffer(s) followed by the image extraction.
+// Whether the buffer of `mode` is known to be zero outside that mode's boxes.
+bool footprint_known(const p9idg_plan* p, int mode) {
+    return p->n_fp[mode] > 0 && (mode == P9IDG_GRID_WSTACK ? p->layers_clean && p->layers_dirty_fp == mode
+                                                           : p->grid_clean && p->grid_dirty_fp == mode);
+}
+
+// Inverse FFT of the grid buffer(s) and the image extraction: over the
+// subgrids' bounding box when it is known (kernels_fft.hip; the buffers are
+// left as they are), else over the whole grid.
 int do_grid_to_image(p9idg_plan* p, int mode) {
     if (int st = check_obs(p)) return st;
     DeviceGuard dg(p->device);
@@ -880,8 +900,18 @@ int do_grid_to_image(p9idg_plan* p, int mode) {
     const double inv_n = 1.0 / (double)p->c.visibilities_count;
     if (int st = span_begin(p, P9IDG_STAGE_TO_IMAGE)) return st;
     if (int st_ = record(p, 5)) return st_;
-    if (mode == P9IDG_GRID_WSTACK) {
-        if (!p->d_layers) return fail(P9IDG_ERR_STATE, "no layers gridded");
+    const bool wstack = mode == P9IDG_GRID_WSTACK;
+    if (wstack && !p->d_layers) return fail(P9IDG_ERR_STATE, "no layers gridded");
+    if (p->have_line && mode >= P9IDG_GRID_PLAIN && mode <= P9IDG_GRID_WSUM && footprint_known(p, mode)) {
+        if (int st = ensure_line(p)) return st;
+        const Box u = p->fp_union[mode];
+        if (wstack) {
+            if (int st = dev_alloc(&p->d_lsum, grid_elems(p))) return st;
+            P9_HIP(launch_sum_boxes(p->d_layers, p->d_fp[mode], p->n_fp[mode], G, u, p->d_lsum, p->stream));
+        }
+        P9_HIP(launch_line_image(wstack ? p->d_lsum : p->d_grid, wstack, u, p->line, p->d_line_tw, p->d_line_mid, inv_n,
+                                 p->d_image, p->stream));
+    } else if (wstack) {
         if (int st = layers_image(p, inv_n, 1)) return st;
     } else {
         p->grid_clean = false;
@@ -896,9 +926,16 @@ int do_grid_to_image(p9idg_plan* p, int mode) {
     return P9IDG_OK;
 }
 
-int do_image_to_grid(p9idg_plan* p) {
+// library: the 2-D library transform also where line transforms exist.
+int do_image_to_grid(p9idg_plan* p, bool library = false) {
     if (int st = check_obs(p)) return st;
     DeviceGuard dg(p->device);
+    if (p->have_line && !library) {
+        if (int st = ensure_line(p)) return st;
+        if (int st = span_begin(p, P9IDG_STAGE_TO_UVW)) return st;
+        P9_HIP(launch_line_grid(p->d_image, p->line, p->d_line_tw, p->d_line_mid, p->d_model_grid, p->stream));
+        return span_end(p);
+    }
     if (int st = ensure_fft_one(p)) return st;
     if (int st = span_begin(p, P9IDG_STAGE_TO_UVW)) return st;
     P9_HIP(launch_image_to_grid(p->d_image, p->c.grid_size, 1, p->d_model_grid, p->stream));
@@ -1068,6 +1105,7 @@ int p9idg_create(const p9idg_constants* c, int32_t device, p9idg_plan** plan) {
     }
     for (int i = 0; i < 8; i++) p->mark[i] = p->ev[i];
     const int S = c->subgrid_size, G = c->grid_size;
+    p->have_line = line_plan(G, p->line);
     // tables: twiddles exp(+2 pi i m / S) and the adder phasor
     // exp(i pi (x + y - S) / S) (Adder.cs:37-40, AdderWStack.cs:17-25), FP64 -> float
     std::vector<float2> tw(S), ph((size_t)S * S);
@@ -1128,6 +1166,8 @@ int p9idg_destroy(p9idg_plan* p) {
     dev_free(p->d_image);
     dev_free(p->d_image64);
     dev_free(p->d_lsum);
+    dev_free(p->d_line_tw);
+    dev_free(p->d_line_mid);
     dev_free(p->d_twiddle);
     dev_free(p->d_phasor);
     dev_free(p->d_rtab);
@@ -1389,7 +1429,7 @@ int p9idg_image_to_vis(p9idg_plan* p, const float* img, double* vis_out) {
     DeviceGuard dg(p->device);
     P9_HIP(hipMemcpyAsync(p->d_image, img, grid_elems(p) * sizeof(float), hipMemcpyHostToDevice,
                           p->stream));
-    if (int st = do_image_to_grid(p)) return st;
+    if (int st = do_image_to_grid(p, true)) return st;
     if (int st = do_exec_degrid(p, P9IDG_DEGRID_WSTACK, true)) return st;
     return download_c128(p, p->d_model_vis, vis_out, vis_elems(p));
 }

@@ -204,9 +204,23 @@ hipError_t launch_resample_tables(const ResamplePair* pairs, int npairs, float* 
 // rows -> visibilities of every covered timestep.
 hipError_t launch_resample_gather(const Resample& r, int C, const float2* vis, float2* out, hipStream_t st);
 hipError_t launch_resample_spread(const Resample& r, int C, const float2* rows, float2* vis, hipStream_t st);
+// LDS line transforms of length n = 2^a 3^b 5^c (even, at most kMaxLine).
+constexpr int kMaxLine = 4096, kMaxPasses = 8;
+struct LinePlan {
+    int32_t n, passes, radix[kMaxPasses];
+};
+bool line_plan(int n, LinePlan& p);
+constexpr int line_pitch(int n) { return n / 2 + 8; }  // mid's row pitch in launch_line_grid
+// The w-layers summed over the union u of their boxes, dense.
+hipError_t launch_sum_boxes(const float2* layers, const Box* boxes, int nboxes, int G, Box u, float2* out, hipStream_t st);
+// Quadrant-swapped real image x inv_n of a grid that is zero outside u: src is
+// that box (dense) or the quadrant-swapped grid; mid: G x (u.x1 - u.x0).
+hipError_t launch_line_image(const float2* src, bool dense, Box u, const LinePlan& p, const float2* tw, float2* mid,
+                             double inv_n, float* img, hipStream_t st);
+// Forward transform of the quadrant-swapped image; mid: G x line_pitch(G).
+hipError_t launch_line_grid(const float* img, const LinePlan& p, const float2* tw, float2* mid, float2* grid,
+                            hipStream_t st);
 hipError_t launch_sum_layers(const float2* layers, int L, size_t GG, float2* out, hipStream_t st);
-hipError_t launch_sum_layer_boxes(const float2* layers, const Box* boxes, int nboxes, int G, Box u,
-                                  float2* out, hipStream_t st);
 hipError_t launch_scale_c64(float2* p, size_t n, double inv_norm, hipStream_t st);
 
 }  // namespace p9idg
