@@ -11,43 +11,36 @@ namespace cd {
 
 constexpr int kTile = 32;  // edge of the argmax tiles (pixels)
 
-// A candidate update: |x - prox|, pixel index y * W + x, new and old value.
-struct Cand {
-    float diff;
-    int32_t idx;
-    float xnew;
-    float xold;
-};
+// A candidate update as an ordered word (kernels_cd.hip); 0: none.
+using Key = unsigned long long;
 
-// Deconvolution state on the device, read by every kernel of an iteration.
-// The call's parameters live here too, so a recorded graph of iterations
-// serves any lambda, alpha, epsilon and iteration limit.
+// Results of the deconvolver's kernels.
 struct State {
-    int32_t done;       // no further updates (converged or iteration limit)
+    int32_t done;       // no further updates
     int32_t converged;  // the last selected |diff| was below epsilon
-    int32_t iters;      // updates made
-    int32_t updated;    // the last selection changed a pixel
-    Cand last;          // that change
-    float absmax;       // the last selected |diff|
-    float lambda, alpha, epsilon;
-    int32_t max_iter;
+    int32_t updates;    // pixels changed by the launch
+    int32_t stalled;    // the workgroups could not exchange their selections
+    float absmax;       // GetAbsMaxDiff
     int32_t pad[3];
 };
 
 // All tiles of the table for lambda / alpha.
 hipError_t launch_tiles_all(const float* x, const float* g, const float* amap, int H, int W, float lambda,
-                            float alpha, Cand* tiles, hipStream_t st);
+                            float alpha, Key* tiles, hipStream_t st);
 // GetAbsMaxDiff: the best |diff| of the tile table into state->absmax.
-hipError_t launch_absmax(const Cand* tiles, int ntiles, State* state, hipStream_t st);
+hipError_t launch_absmax(const Key* tiles, int ntiles, State* state, hipStream_t st);
 
-// The row table (best tile per tile row) and the first selection after
-// launch_tiles_all; then launch_iteration repeatedly: the window tiles take
-// the gradient change and are re-evaluated, and one workgroup refreshes the
-// rows the window spans and selects the next update.
-// lambda, alpha, epsilon and the iteration limit come from the state.
-hipError_t launch_first_select(const Cand* tiles, Cand* rows, int H, int W, State* state, float* x, hipStream_t st);
-hipError_t launch_iteration(float* x, float* g, const float* amap, const float* psf2, int p2h, int p2w, int H, int W,
-                            Cand* tiles, Cand* rows, State* state, hipStream_t st);
+// The descent's workgroups: OH x OW of them on the current device, `local`
+// tiles each at most.
+struct DescentShape {
+    int OH = 0, OW = 0, local = 0;
+};
+hipError_t descent_shape(int H, int W, DescentShape* shape);
+// Up to `limit` (> 0) iterations on x and g.  slots: 2 OH OW words; tiles:
+// OH OW local words.
+hipError_t launch_descent(float* x, float* g, const float* amap, const float* psf2, int p2h, int p2w, int H, int W,
+                          const DescentShape& shape, float lambda, float alpha, float epsilon, int limit, Key* slots,
+                          Key* tiles, State* state, hipStream_t st);
 
 // PaddedConvolver / CalcPaddedFourierCorrelation pieces (complex double
 // buffers of N0 x N1).

@@ -332,25 +332,18 @@ struct p9cd {
     hipStream_t stream = nullptr;
     float* d_amap = nullptr;
     float* d_psf2 = nullptr;
-    cd::Cand* d_tiles = nullptr;
-    cd::Cand* d_rows = nullptr;
+    cd::DescentShape shape;
+    cd::Key* d_tiles = nullptr;
+    cd::Key* d_slots = nullptr;
     cd::State* d_state = nullptr;
     cd::State* h_state = nullptr;  // pinned host copy of the state (hipHostMalloc)
 
     float* d_io = nullptr;  // [2][H][W] staging for host-array calls
-
-    // kBatch iterations recorded as a graph for one (x, gradients) buffer
-    // pair; the parameters are read from the device state, so every call on
-    // the same buffers replays it
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t graph_exec = nullptr;
-    const float* graph_x = nullptr;
-    const float* graph_g = nullptr;
 };
 
 namespace {
 
-constexpr int kBatch = 128;  // iterations enqueued between host checks of the state
+constexpr int kPerLaunch = 1 << 14;  // iterations of one launch: some 50 ms at most
 
 int cd_abs_max(p9cd* c, const float* d_x, const float* d_g, float lambda, float alpha, float* out) {
     P9_HIP(cd::launch_tiles_all(d_x, d_g, c->d_amap, c->H, c->W, lambda, alpha, c->d_tiles, c->stream));
@@ -361,67 +354,22 @@ int cd_abs_max(p9cd* c, const float* d_x, const float* d_g, float lambda, float 
     return P9IDG_OK;
 }
 
-void cd_drop_graph(p9cd* c) {
-    if (c->graph_exec) (void)hipGraphExecDestroy(c->graph_exec);
-    if (c->graph) (void)hipGraphDestroy(c->graph);
-    c->graph_exec = nullptr;
-    c->graph = nullptr;
-    c->graph_x = c->graph_g = nullptr;
-}
-
-// Records kBatch iterations on (d_x, d_g) as a graph, unless the recorded
-// one already works on these buffers.  Called with the stream idle.
-int cd_graph(p9cd* c, float* d_x, float* d_g) {
-    if (c->graph_exec && c->graph_x == d_x && c->graph_g == d_g) return P9IDG_OK;
-    cd_drop_graph(c);
-    P9_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-    hipError_t e = hipSuccess;
-    for (int k = 0; k < kBatch && e == hipSuccess; k++)
-        e = cd::launch_iteration(d_x, d_g, c->d_amap, c->d_psf2, c->p2h, c->p2w, c->H, c->W, c->d_tiles, c->d_rows,
-                                 c->d_state, c->stream);
-    hipGraph_t graph = nullptr;
-    const hipError_t e_end = hipStreamEndCapture(c->stream, &graph);
-    if (e == hipSuccess) e = e_end;
-    hipGraphExec_t exec = nullptr;
-    if (e == hipSuccess) e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
-    if (e != hipSuccess) {
-        if (graph) (void)hipGraphDestroy(graph);
-        return hip_fail(e, "deconvolution graph");
-    }
-    c->graph = graph;
-    c->graph_exec = exec;
-    c->graph_x = d_x;
-    c->graph_g = d_g;
-    return P9IDG_OK;
-}
-
-// The first selection, then the recorded iterations replayed until the state
-// says done (launches after that return at once).  The state travels through
-// pinned host memory.
+// The state travels through pinned host memory.
 int cd_run(p9cd* c, float* d_x, float* d_g, float lambda, float alpha, int32_t max_iter, float eps, int32_t* conv,
            int32_t* iters) {
     cd::State& s = *c->h_state;
     s = cd::State{};
-    s.done = max_iter <= 0;
-    s.lambda = lambda;
-    s.alpha = alpha;
-    s.epsilon = eps;
-    s.max_iter = max_iter;
-    P9_HIP(hipMemcpyAsync(c->d_state, &s, sizeof(s), hipMemcpyHostToDevice, c->stream));
-    P9_HIP(cd::launch_tiles_all(d_x, d_g, c->d_amap, c->H, c->W, lambda, alpha, c->d_tiles, c->stream));
-    P9_HIP(cd::launch_first_select(c->d_tiles, c->d_rows, c->H, c->W, c->d_state, d_x, c->stream));
-    P9_HIP(hipMemcpyAsync(&s, c->d_state, sizeof(s), hipMemcpyDeviceToHost, c->stream));
-    P9_HIP(hipStreamSynchronize(c->stream));
-    if (!(s.done && !s.updated)) {
-        if (int st = cd_graph(c, d_x, d_g)) return st;
-        while (!s.done || s.updated) {
-            P9_HIP(hipGraphLaunch(c->graph_exec, c->stream));
-            P9_HIP(hipMemcpyAsync(&s, c->d_state, sizeof(s), hipMemcpyDeviceToHost, c->stream));
-            P9_HIP(hipStreamSynchronize(c->stream));
-        }
+    int32_t made = 0;
+    while (!s.done && made < max_iter) {
+        P9_HIP(cd::launch_descent(d_x, d_g, c->d_amap, c->d_psf2, c->p2h, c->p2w, c->H, c->W, c->shape, lambda, alpha, eps,
+                                  std::min(max_iter - made, kPerLaunch), c->d_slots, c->d_tiles, c->d_state, c->stream));
+        P9_HIP(hipMemcpyAsync(&s, c->d_state, sizeof(s), hipMemcpyDeviceToHost, c->stream));
+        P9_HIP(hipStreamSynchronize(c->stream));
+        if (s.stalled) return fail(P9IDG_ERR_HIP, "the deconvolution's workgroups did not all become resident");
+        made += s.updates;
     }
     if (conv) *conv = s.converged;
-    if (iters) *iters = s.iters;
+    if (iters) *iters = made;
     return P9IDG_OK;
 }
 
@@ -448,10 +396,12 @@ int p9cd_create(int32_t device, int32_t height, int32_t width, const float* psf,
         return st;
     };
     if (hipStreamCreate(&c->stream) != hipSuccess) return bail(fail(P9IDG_ERR_HIP, "stream creation failed"));
+    if (hipError_t e = cd::descent_shape(height, width, &c->shape)) return bail(hip_fail(e, "deconvolution launch shape"));
+    const size_t workgroups = (size_t)c->shape.OH * c->shape.OW;
     int st;
     if ((st = alloc(&c->d_amap, (size_t)height * width)) || (st = alloc(&c->d_psf2, (size_t)c->p2h * c->p2w)) ||
-        (st = alloc(&c->d_tiles, (size_t)c->ntiles)) || (st = alloc(&c->d_state, 1)) ||
-        (st = alloc(&c->d_rows, (size_t)(height + cd::kTile - 1) / cd::kTile)) ||
+        (st = alloc(&c->d_tiles, std::max((size_t)c->ntiles, workgroups * c->shape.local))) ||
+        (st = alloc(&c->d_slots, 2 * workgroups)) || (st = alloc(&c->d_state, 1)) ||
         (st = alloc(&c->d_io, 2 * (size_t)height * width)))
         return bail(st);
     if (hipHostMalloc(reinterpret_cast<void**>(&c->h_state), sizeof(cd::State), hipHostMallocDefault) != hipSuccess) {
@@ -476,12 +426,11 @@ int p9cd_destroy(p9cd* c) {
     if (!c) return P9IDG_OK;
     Guard g(c->device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
-    cd_drop_graph(c);
     if (c->h_state) (void)hipHostFree(c->h_state);
     release(c->d_amap);
     release(c->d_psf2);
     release(c->d_tiles);
-    release(c->d_rows);
+    release(c->d_slots);
     release(c->d_state);
     release(c->d_io);
     if (c->stream) (void)hipStreamDestroy(c->stream);

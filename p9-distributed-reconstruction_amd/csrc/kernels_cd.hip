@@ -4,12 +4,11 @@
 // FastSerialCD picks, per iteration, the pixel whose elastic-net proximal
 // update changes it most (first row, then first column on ties), writes it
 // and adds psf2 * (old - new) to the gradients in the PSF^2 window.  Only the
-// window's pixels change, so the argmax is kept as a table of per-tile bests:
-// an iteration re-evaluates the tiles the window touches and reduces the
-// table.  Float expressions use one rounding per operation (no contraction),
-// as the reference's float code does (this file is built with
-// -ffp-contract=off).
-#include <climits>
+// window's pixels change, so the argmax is kept as a table of per-tile bests.
+// Float expressions use one rounding per operation (no contraction), as the
+// reference's float code does (this file is built with -ffp-contract=off).
+#include <algorithm>
+#include <cmath>
 
 #include "cd_internal.h"
 
@@ -30,104 +29,96 @@ __device__ __forceinline__ float prox(float x, float lipschitz, float lambda, fl
     return __fdiv_rn(num, den);
 }
 
-// Larger |diff| wins; equal nonzero |diff|: the smaller pixel index (the
-// reference's row-then-column scan keeps the first maximum).
-__device__ __forceinline__ bool better(const Cand& a, const Cand& b) {
-    return a.diff > b.diff || (a.diff == b.diff && a.diff > 0.f && a.idx < b.idx);
+// A candidate update as one ordered word: |old - new| above the complement of
+// the pixel index (equal changes: the smaller index wins, as the reference's
+// row-then-column scan keeps the first maximum), the sign of old - new in bit
+// 0.  0: no update.  Bit 63 is free: a finite or infinite |change| has no sign.
+__device__ __forceinline__ Key make_key(float d, int idx) {
+    const float m = fabsf(d);
+    if (!(m > 0.f)) return 0;
+    return ((Key)__float_as_uint(m) << 32) | ((Key)(unsigned)(INT32_MAX - idx) << 1) | (d < 0.f ? 1u : 0u);
 }
+__device__ __forceinline__ float key_diff(Key k) { return __uint_as_float((unsigned)(k >> 32)); }
+__device__ __forceinline__ float key_change(Key k) { return (k & 1) ? -key_diff(k) : key_diff(k); }
+__device__ __forceinline__ int key_index(Key k) { return INT32_MAX - (int)((unsigned)k >> 1); }
+__device__ __forceinline__ Key max_key(Key a, Key b) { return a > b ? a : b; }
 
-
-// One step of a wave-wide best over DPP lane routes: each lane compares with
-// the candidate CTRL routes to it; lanes outside ROW_MASK (rows of 16 lanes)
+// One step of a wave-wide maximum over DPP lane routes: each lane compares
+// with the key CTRL routes to it; lanes outside ROW_MASK (rows of 16 lanes)
 // keep their own.
 template <int CTRL, int ROW_MASK>
-__device__ __forceinline__ Cand dpp_best(const Cand& c) {
-    Cand o;
-    o.diff = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, c.diff),
-                                                                   __builtin_bit_cast(int, c.diff), CTRL, ROW_MASK,
-                                                                   0xF, false));
-    o.idx = __builtin_amdgcn_update_dpp(c.idx, c.idx, CTRL, ROW_MASK, 0xF, false);
-    o.xnew = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, c.xnew),
-                                                                   __builtin_bit_cast(int, c.xnew), CTRL, ROW_MASK,
-                                                                   0xF, false));
-    o.xold = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, c.xold),
-                                                                   __builtin_bit_cast(int, c.xold), CTRL, ROW_MASK,
-                                                                   0xF, false));
-    return better(o, c) ? o : c;
+__device__ __forceinline__ Key dpp_max(Key k) {
+    const int lo = (int)(unsigned)k, hi = (int)(unsigned)(k >> 32);
+    const unsigned l = (unsigned)__builtin_amdgcn_update_dpp(lo, lo, CTRL, ROW_MASK, 0xF, false);
+    const unsigned h = (unsigned)__builtin_amdgcn_update_dpp(hi, hi, CTRL, ROW_MASK, 0xF, false);
+    return max_key(k, ((Key)h << 32) | l);
 }
-// The wave's best candidate, in every lane: lane pairs, quads (quad
-// permutes), 8 and 16 lanes (half-row and row mirrors), then rows 0 + 1 into
-// row 1 and rows 2 + 3 into row 3 (row_bcast15), and rows 0-1 into rows 2-3
-// (row_bcast31), so lane 63 holds the best of all 64.  better() orders every
-// candidate with a positive difference strictly, so that best does not depend
-// on the order of the comparisons.
-__device__ __forceinline__ Cand wave_reduce(Cand c) {
-    c = dpp_best<0xB1, 0xF>(c);   // quad_perm [1, 0, 3, 2]
-    c = dpp_best<0x4E, 0xF>(c);   // quad_perm [2, 3, 0, 1]
-    c = dpp_best<0x141, 0xF>(c);  // row_half_mirror
-    c = dpp_best<0x140, 0xF>(c);  // row_mirror
-    c = dpp_best<0x142, 0xA>(c);  // row_bcast15
-    c = dpp_best<0x143, 0xC>(c);  // row_bcast31
-    Cand r;
-    r.diff = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, c.diff), 63));
-    r.idx = __builtin_amdgcn_readlane(c.idx, 63);
-    r.xnew = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, c.xnew), 63));
-    r.xold = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, c.xold), 63));
-    return r;
+// The wave's largest key, in every lane: lane pairs, quads (quad permutes), 8
+// and 16 lanes (half-row and row mirrors), then rows 0 + 1 into row 1 and rows
+// 2 + 3 into row 3 (row_bcast15), and rows 0-1 into rows 2-3 (row_bcast31), so
+// lane 63 holds the largest of all 64.
+__device__ __forceinline__ Key wave_max(Key k) {
+    k = dpp_max<0xB1, 0xF>(k);   // quad_perm [1, 0, 3, 2]
+    k = dpp_max<0x4E, 0xF>(k);   // quad_perm [2, 3, 0, 1]
+    k = dpp_max<0x141, 0xF>(k);  // row_half_mirror
+    k = dpp_max<0x140, 0xF>(k);  // row_mirror
+    k = dpp_max<0x142, 0xA>(k);  // row_bcast15
+    k = dpp_max<0x143, 0xC>(k);  // row_bcast31
+    const unsigned l = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)k, 63);
+    const unsigned h = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(k >> 32), 63);
+    return ((Key)h << 32) | l;
 }
-template <int NT>
-__device__ Cand block_best(Cand c, Cand* sh) {
-    c = wave_reduce(c);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    if (lane == 0) sh[wave] = c;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int w = 1; w < NT / 64; w++)
-            if (better(sh[w], c)) c = sh[w];
-        sh[0] = c;
-    }
-    __syncthreads();
-    return sh[0];
+template <int WAVES>
+__device__ __forceinline__ Key max_of(const Key* v) {
+    Key k = v[0];
+#pragma unroll
+    for (int w = 1; w < WAVES; w++) k = max_key(k, v[w]);
+    return k;
 }
 
-__device__ __forceinline__ Cand none() { return Cand{0.f, INT_MAX, 0.f, 0.f}; }
-
-// FastSerialCD.cs:150-162 for one pixel
-__device__ __forceinline__ Cand eval(const float* x, const float* g, const float* amap, int idx, float lambda,
-                                     float alpha) {
-    const float a = amap[idx], old = x[idx];
-    const float t = prox(__fadd_rn(__fmul_rn(old, a), g[idx]), a, lambda, alpha);
-    return Cand{fabsf(__fsub_rn(old, t)), idx, t, old};
+// FastSerialCD.cs:150-162 for one pixel: the proximal value
+__device__ __forceinline__ float update_of(float old, float g, float a, float lambda, float alpha) {
+    return prox(__fadd_rn(__fmul_rn(old, a), g), a, lambda, alpha);
 }
 
-__device__ void tile_best(const float* x, const float* g, const float* amap, int H, int W, int ty, int tx,
-                          float lambda, float alpha, Cand* tiles, int ntx) {
-    __shared__ Cand sh[kThreads / 64];
-    Cand best = none();
-    for (int p = threadIdx.x; p < kTile * kTile; p += kThreads) {
-        const int y = ty * kTile + p / kTile, xx = tx * kTile + p % kTile;
-        if (y < H && xx < W) {
-            const Cand c = eval(x, g, amap, y * W + xx, lambda, alpha);
-            if (better(c, best)) best = c;
+// The best update of tile (ty, tx), by one wave.
+__device__ __forceinline__ Key tile_best(const float* __restrict__ x, const float* __restrict__ g,
+                                         const float* __restrict__ amap, int H, int W, int ty, int tx, float lambda,
+                                         float alpha) {
+    const int lane = threadIdx.x & 63;
+    const int j = tx * kTile + lane % kTile;
+    Key best = 0;
+    if (j < W)
+#pragma unroll 4
+        for (int r = lane / kTile; r < kTile; r += 64 / kTile) {
+            const int i = ty * kTile + r;
+            if (i >= H) break;
+            const int idx = i * W + j;
+            const float old = x[idx];
+            best = max_key(best, make_key(__fsub_rn(old, update_of(old, g[idx], amap[idx], lambda, alpha)), idx));
         }
-    }
-    best = block_best<kThreads>(best, sh);
-    if (threadIdx.x == 0) tiles[ty * ntx + tx] = best;
+    return wave_max(best);
 }
 
+// One tile per wave.
 __global__ __launch_bounds__(kThreads) void tiles_all_kernel(const float* x, const float* g, const float* amap,
-                                                             int H, int W, float lambda, float alpha, Cand* tiles) {
-    tile_best(x, g, amap, H, W, blockIdx.y, blockIdx.x, lambda, alpha, tiles, gridDim.x);
+                                                             int H, int W, float lambda, float alpha, Key* tiles,
+                                                             int ntx, int ntiles) {
+    const int t = (int)(blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6));
+    if (t >= ntiles) return;
+    const Key k = tile_best(x, g, amap, H, W, t / ntx, t % ntx, lambda, alpha);
+    if ((threadIdx.x & 63) == 0) tiles[t] = k;
 }
 
 // FastSerialCD.cs:132-135 (GetAbsMaxDiff): the best |diff| of the tile table.
-__global__ __launch_bounds__(kSelectThreads) void absmax_kernel(const Cand* tiles, int ntiles, State* st) {
-    __shared__ Cand sh[kSelectThreads / 64];
-    Cand best = none();
-    for (int i = threadIdx.x; i < ntiles; i += kSelectThreads)
-        if (better(tiles[i], best)) best = tiles[i];
-    best = block_best<kSelectThreads>(best, sh);
-    if (threadIdx.x == 0) st->absmax = best.diff;
+__global__ __launch_bounds__(kSelectThreads) void absmax_kernel(const Key* tiles, int ntiles, State* st) {
+    __shared__ Key sh[kSelectThreads / 64];
+    Key best = 0;
+    for (int i = threadIdx.x; i < ntiles; i += kSelectThreads) best = max_key(best, tiles[i]);
+    best = wave_max(best);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = best;
+    __syncthreads();
+    if (threadIdx.x == 0) st->absmax = key_diff(max_of<kSelectThreads / 64>(sh));
 }
 
 // Common.cs:146-160: flipped PSF at (y + ypad/2 + 1, x + xpad/2 + 1), then
@@ -211,155 +202,152 @@ __global__ void amap_kernel(const double* s, int ph, int pw, int H, int W, float
     }
 }
 
-// --- one launch per iteration ------------------------------------------------
-// Best of tiles[first .. first + n) by one wave (64 lanes).
-__device__ Cand wave_best(const Cand* v, int n, int lane) {
-    Cand b = none();
-    for (int i = lane; i < n; i += 64)
-        if (better(v[i], b)) b = v[i];
-    return wave_reduce(b);
+// --- the descent ----------------------------------------------------------------
+// All iterations of a call in one cooperative launch.  Tile (ty, tx) belongs to
+// workgroup (ty % OH, tx % OW) of an OH x OW arrangement, so the tiles of a
+// window fall on different workgroups, and each workgroup keeps the bests of
+// its tiles.  An iteration is one exchange: every workgroup publishes its best
+// update, reads all of them and finds the same maximum; the owners of the
+// window's tiles then add psf2 * (old - new) to their gradients
+// (FastSerialCD.cs:219-238) and re-evaluate them.  A pixel is only ever touched
+// by one thread of its tile's workgroup.
+//
+// A published word holds the key and, in bit 63, the turn's tag, so one 64-bit
+// store hands over both and nothing else needs ordering.  Turn n uses buffer
+// n & 1 with tag (n >> 1) & 1: a workgroup writes turn n + 2 only after it has
+// read turn n + 1 from all, each of which had then finished reading turn n.
+//
+// What bounds it is the latency of that exchange over the XCDs and of the
+// window's loads.  A launch pair per iteration (window, then a one-workgroup
+// selection) spent most of its time between launches.
+struct Descent {
+    float* x;
+    float* g;
+    const float* amap;
+    const float* psf2;
+    int p2h, p2w, H, W, OH, OW;
+    float lambda, alpha, epsilon;
+    int limit;    // updates of this launch
+    Key* slots;   // [2][OH * OW]
+    Key* tiles;   // [OH * OW][local]: the tile tables where they don't fit LDS
+    int local;
+    State* st;
+};
+constexpr int kLdsTiles = 1024;
+constexpr Key kStalled = ~(Key)0;
+// Polls of one slot before the exchange is given up (seconds: only if the
+// launch's workgroups could not all become resident).
+constexpr int kMaxPolls = 1 << 25;
+
+// The slots' tags before turn 0: neither buffer holds its first turn.
+__global__ void reset_slots_kernel(Key* slots, int n) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) slots[i] = (Key)1 << 63;
 }
 
-// Rows [ty0, ty1] of the row table from the tile table, then the overall best
-// (4 waves), and the selection of FastSerialCD.cs:84-97 by thread 0.
-// A wave takes rows ty0 + wave, + 4, + 8, ...; four of its rows at a time have
-// their tiles loaded before any is reduced, so the loads overlap (the
-// comparisons run in the same order as one row at a time).
-__device__ __forceinline__ void rows_and_select(const Cand* __restrict__ tiles, Cand* __restrict__ rows, int ntx, int nty, int ty0,
-                                int ty1, State* st, float* x) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    constexpr int kWaves = kThreads / 64, kBatch = 4;
-    for (int ty = ty0 + wave; ty <= ty1; ty += kWaves * kBatch) {
-        Cand b[kBatch];
-        if (ntx <= 128) {  // two tiles per lane at most: all loads first
-            Cand v0[kBatch], v1[kBatch];
-#pragma unroll
-            for (int r = 0; r < kBatch; r++) {
-                const int t = ty + r * kWaves;
-                const Cand* row = tiles + (size_t)t * ntx;
-                v0[r] = t <= ty1 && lane < ntx ? row[lane] : none();
-                v1[r] = t <= ty1 && lane + 64 < ntx ? row[lane + 64] : none();
-            }
-#pragma unroll
-            for (int r = 0; r < kBatch; r++) {
-                b[r] = none();
-                if (better(v0[r], b[r])) b[r] = v0[r];
-                if (better(v1[r], b[r])) b[r] = v1[r];
-            }
-        } else {
-#pragma unroll
-            for (int r = 0; r < kBatch; r++) {
-                const int t = ty + r * kWaves;
-                b[r] = none();
-                if (t <= ty1)
-                    for (int i = lane; i < ntx; i += 64)
-                        if (better(tiles[(size_t)t * ntx + i], b[r])) b[r] = tiles[(size_t)t * ntx + i];
-            }
-        }
-#pragma unroll
-        for (int r = 0; r < kBatch; r++) {
-            b[r] = wave_reduce(b[r]);
-            const int t = ty + r * kWaves;
-            if (lane == 0 && t <= ty1) rows[t] = b[r];
-        }
+__device__ __forceinline__ Key await_slot(const Key* slot, unsigned tag) {
+    for (int i = 0; i < kMaxPolls; i++) {
+        const Key v = __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if ((unsigned)(v >> 63) == tag) return v & ~((Key)1 << 63);
+    }
+    return kStalled;
+}
+
+template <bool LDS>
+__global__ __launch_bounds__(kThreads) void descent_kernel(Descent a) {
+    constexpr int kWaves = kThreads / 64, kPer = kTile * kTile / kThreads;
+    __shared__ Key s_table[LDS ? kLdsTiles : 1];
+    __shared__ Key s_turn[2][kWaves], s_tile[2][kWaves];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int H = a.H, W = a.W, OH = a.OH, OW = a.OW, me = blockIdx.x, nwg = OH * OW;
+    const int ntx = (W + kTile - 1) / kTile, nty = (H + kTile - 1) / kTile;
+    const int oy = me / OW, ox = me - oy * OW;
+    const int nrow = (nty - oy + OH - 1) / OH, ncol = (ntx - ox + OW - 1) / OW, nlocal = nrow * ncol;
+    Key* const table = LDS ? s_table : a.tiles + (size_t)me * a.local;
+    for (int l = wave; l < nlocal; l += kWaves) {
+        const Key k = tile_best(a.x, a.g, a.amap, H, W, oy + l / ncol * OH, ox + l % ncol * OW, a.lambda, a.alpha);
+        if (lane == 0) table[l] = k;
     }
     __threadfence_block();
     __syncthreads();
-    if (wave != 0) return;
-    const Cand best = wave_best(rows, nty, lane);
-    if (lane != 0) return;
-    const float epsilon = st->epsilon;
-    st->absmax = best.diff;
-    if (best.diff < epsilon || best.idx == INT_MAX) {
-        st->converged = best.diff < epsilon;
-        st->done = 1;
-        st->updated = 0;
-        return;
-    }
-    x[best.idx] = best.xnew;
-    st->last = best;
-    st->updated = 1;
-    st->iters += 1;
-    if (st->iters >= st->max_iter) st->done = 1;
-}
-
-// All rows and the first selection (after tiles_all_kernel).
-__global__ __launch_bounds__(kThreads) void first_select_kernel(const Cand* tiles, Cand* rows, int ntx, int nty,
-                                                                State* st, float* x) {
-    if (st->done) return;
-    rows_and_select(tiles, rows, ntx, nty, 0, nty - 1, st, x);
-}
-
-// Window half of an iteration: each block owns one tile of the PSF^2 window
-// of the last update, adds psf2 * (old - new) to its gradients
-// (FastSerialCD.cs:219-238) and re-evaluates the tile.  The change of the
-// last selection is applied even when that selection reached the iteration
-// limit (the reference updates before it stops).
-__global__ __launch_bounds__(kThreads) void window_kernel(float* __restrict__ x, float* __restrict__ g,
-                                                          const float* __restrict__ amap,
-                                                          const float* __restrict__ psf2, int p2h, int p2w, int H,
-                                                          int W, Cand* __restrict__ tiles, const State* st) {
-    __shared__ Cand sh[kThreads / 64];
-    if (!st->updated) return;  // uniform
-    const float lambda = st->lambda, alpha = st->alpha;
-    const int ntx = (W + kTile - 1) / kTile;
-    const int y0 = st->last.idx / W, x0 = st->last.idx % W;
-    const float d = __fsub_rn(st->last.xold, st->last.xnew);
-    const int yh = p2h / 2, xh = p2w / 2;
-    const int r0 = max(y0 - yh, 0), r1 = min(y0 - yh + p2h, H);
-    const int c0 = max(x0 - xh, 0), c1 = min(x0 - xh + p2w, W);
-    const int ty = r0 / kTile + (int)blockIdx.y, tx = c0 / kTile + (int)blockIdx.x;
-    if (ty > (r1 - 1) / kTile || tx > (c1 - 1) / kTile) return;
-    // this thread's pixels: every load first, then the updates and
-    // evaluations in pixel order (x is written only by the select kernel,
-    // each gradient by its own thread)
-    constexpr int kPer = kTile * kTile / kThreads;
-    int idx[kPer];
-    bool in[kPer], win[kPer];
-    float gv[kPer], pv[kPer], xv[kPer], av[kPer];
-#pragma unroll
-    for (int k = 0; k < kPer; k++) {
-        const int p = (int)threadIdx.x + k * kThreads;
-        const int i = ty * kTile + p / kTile, j = tx * kTile + p % kTile;
-        in[k] = i < H && j < W;
-        win[k] = in[k] && i >= r0 && i < r1 && j >= c0 && j < c1;
-        idx[k] = in[k] ? i * W + j : 0;
-        gv[k] = in[k] ? g[idx[k]] : 0.f;
-        xv[k] = in[k] ? x[idx[k]] : 0.f;
-        av[k] = in[k] ? amap[idx[k]] : 0.f;
-        pv[k] = win[k] ? psf2[(i - y0 + yh) * p2w + (j - x0 + xh)] : 0.f;
-    }
-    Cand best = none();
-#pragma unroll
-    for (int k = 0; k < kPer; k++) {
-        if (!in[k]) continue;
-        if (win[k]) {
-            gv[k] = __fadd_rn(gv[k], __fmul_rn(pv[k], d));
-            g[idx[k]] = gv[k];
+    const int yh = a.p2h / 2, xh = a.p2w / 2;
+    Key mine = 0, best = 0;
+    bool changed = true;  // of this workgroup's tiles
+    int updates = 0;
+    for (unsigned turn = 0;; turn++) {
+        if (wave == 0) {
+            if (changed) {
+                mine = 0;
+                for (int l = lane; l < nlocal; l += 64) mine = max_key(mine, table[l]);
+                mine = wave_max(mine);
+            }
+            if (lane == 0)
+                __hip_atomic_store(a.slots + (turn & 1) * nwg + me, mine | ((Key)((turn >> 1) & 1) << 63), __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
         }
-        // FastSerialCD.cs:150-162 (as eval)
-        const float t = prox(__fadd_rn(__fmul_rn(xv[k], av[k]), gv[k]), av[k], lambda, alpha);
-        const Cand c{fabsf(__fsub_rn(xv[k], t)), idx[k], t, xv[k]};
-        if (better(c, best)) best = c;
-    }
-    best = block_best<kThreads>(best, sh);
-    if (threadIdx.x == 0) tiles[ty * ntx + tx] = best;
-}
-
-// Selection half: refresh the rows the window spans and select the next
-// update (one workgroup).
-__global__ __launch_bounds__(kThreads) void row_select_kernel(const Cand* tiles, Cand* rows, int p2h, int H, int W,
-                                                              State* st, float* x) {
-    if (!st->updated) return;  // uniform
-    if (st->done) {
+        Key v = 0;
+        for (int s = t; s < nwg; s += kThreads)
+            v = max_key(v, await_slot(a.slots + (turn & 1) * nwg + s, (turn >> 1) & 1));
+        v = wave_max(v);
+        if (lane == 0) s_turn[turn & 1][wave] = v;
         __syncthreads();
-        if (threadIdx.x == 0) st->updated = 0;
-        return;
+        best = max_of<kWaves>(s_turn[turn & 1]);
+        // FastSerialCD.cs:84-97
+        if (best == kStalled || best == 0 || key_diff(best) < a.epsilon) break;
+        updates++;
+        const int at = key_index(best), y0 = at / W, x0 = at - y0 * W;
+        const float d = key_change(best);
+        const int r0 = max(y0 - yh, 0), r1 = min(y0 - yh + a.p2h, H);
+        const int c0 = max(x0 - xh, 0), c1 = min(x0 - xh + a.p2w, W);
+        const int tya = r0 / kTile, txa = c0 / kTile, tyb = (r1 - 1) / kTile, txb = (c1 - 1) / kTile;
+        int q = 0;
+        // the first own tile at or after (tya, txa) in each direction
+        for (int ty = tya + (oy + OH - tya % OH) % OH; ty <= tyb; ty += OH)
+            for (int tx = txa + (ox + OW - txa % OW) % OW; tx <= txb; tx += OW, q++) {
+                int idx[kPer];
+                bool in[kPer], win[kPer];
+                float gv[kPer], pv[kPer], xv[kPer], av[kPer];
+#pragma unroll
+                for (int k = 0; k < kPer; k++) {
+                    const int p = t + k * kThreads, i = ty * kTile + p / kTile, j = tx * kTile + p % kTile;
+                    in[k] = i < H && j < W;
+                    win[k] = in[k] && i >= r0 && i < r1 && j >= c0 && j < c1;
+                    idx[k] = in[k] ? i * W + j : 0;
+                    gv[k] = in[k] ? a.g[idx[k]] : 0.f;
+                    xv[k] = in[k] ? a.x[idx[k]] : 0.f;
+                    av[k] = in[k] ? a.amap[idx[k]] : 0.f;
+                    pv[k] = win[k] ? a.psf2[(i - y0 + yh) * a.p2w + (j - x0 + xh)] : 0.f;
+                }
+                Key b = 0;
+#pragma unroll
+                for (int k = 0; k < kPer; k++) {
+                    if (!in[k]) continue;
+                    if (idx[k] == at) {  // the update itself
+                        xv[k] = update_of(xv[k], gv[k], av[k], a.lambda, a.alpha);
+                        a.x[at] = xv[k];
+                    }
+                    if (win[k]) {
+                        gv[k] = __fadd_rn(gv[k], __fmul_rn(pv[k], d));
+                        a.g[idx[k]] = gv[k];
+                    }
+                    b = max_key(b, make_key(__fsub_rn(xv[k], update_of(xv[k], gv[k], av[k], a.lambda, a.alpha)), idx[k]));
+                }
+                b = wave_max(b);
+                if (lane == 0) s_tile[q & 1][wave] = b;
+                __syncthreads();
+                if (t == 0) table[(ty / OH) * ncol + tx / OW] = max_of<kWaves>(s_tile[q & 1]);
+            }
+        changed = q > 0;
+        if (changed) __threadfence_block();  // wave 0 reads what its lane 0 wrote
+        if (updates >= a.limit) break;
     }
-    const int y0 = st->last.idx / W;
-    const int r0 = max(y0 - p2h / 2, 0), r1 = min(y0 - p2h / 2 + p2h, H);
-    __syncthreads();  // every thread has read the state before thread 0 rewrites it
-    rows_and_select(tiles, rows, (W + kTile - 1) / kTile, (H + kTile - 1) / kTile, r0 / kTile, (r1 - 1) / kTile, st, x);
+    if (me == 0 && t == 0) {
+        const bool stop = updates < a.limit || best == 0 || key_diff(best) < a.epsilon;
+        a.st->stalled = best == kStalled;
+        a.st->updates = updates;
+        a.st->done = stop;
+        a.st->converged = stop && key_diff(best) < a.epsilon;
+    }
 }
 
 __global__ void zero_u32_kernel(unsigned* p) { *p = 0u; }
@@ -381,13 +369,14 @@ unsigned blocks(size_t n) {
 }  // namespace
 
 hipError_t launch_tiles_all(const float* x, const float* g, const float* amap, int H, int W, float lambda,
-                            float alpha, Cand* tiles, hipStream_t st) {
-    const dim3 grid((W + kTile - 1) / kTile, (H + kTile - 1) / kTile);
-    hipLaunchKernelGGL(tiles_all_kernel, grid, dim3(kThreads), 0, st, x, g, amap, H, W, lambda, alpha, tiles);
+                            float alpha, Key* tiles, hipStream_t st) {
+    const int ntx = (W + kTile - 1) / kTile, n = ntx * ((H + kTile - 1) / kTile);
+    hipLaunchKernelGGL(tiles_all_kernel, dim3((n + kThreads / 64 - 1) / (kThreads / 64)), dim3(kThreads), 0, st, x, g, amap,
+                       H, W, lambda, alpha, tiles, ntx, n);
     return hipGetLastError();
 }
 
-hipError_t launch_absmax(const Cand* tiles, int ntiles, State* state, hipStream_t st) {
+hipError_t launch_absmax(const Key* tiles, int ntiles, State* state, hipStream_t st) {
     hipLaunchKernelGGL(absmax_kernel, dim3(1), dim3(kSelectThreads), 0, st, tiles, ntiles, state);
     return hipGetLastError();
 }
@@ -424,18 +413,36 @@ hipError_t launch_extract(const double2* buf, int N1, int yh, int xh, double nor
     return hipGetLastError();
 }
 
-hipError_t launch_first_select(const Cand* tiles, Cand* rows, int H, int W, State* state, float* x, hipStream_t st) {
-    hipLaunchKernelGGL(first_select_kernel, dim3(1), dim3(kThreads), 0, st, tiles, rows, (W + kTile - 1) / kTile,
-                       (H + kTile - 1) / kTile, state, x);
-    return hipGetLastError();
+hipError_t descent_shape(int H, int W, DescentShape* shape) {
+    int dev = 0, cus = 0, per = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+    if (e == hipSuccess)
+        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, reinterpret_cast<const void*>(descent_kernel<true>), kThreads, 0);
+    if (e != hipSuccess) return e;
+    // one workgroup per CU at most: the exchange grows with their number
+    const int most = cus * std::min(per, 1);
+    if (most < 1) return hipErrorInvalidConfiguration;
+    const int ntx = (W + kTile - 1) / kTile, nty = (H + kTile - 1) / kTile;
+    const int side = std::max(1, (int)std::sqrt((double)most));
+    shape->OW = std::min(side, ntx);
+    shape->OH = std::min(nty, most / shape->OW);
+    shape->OW = std::min(ntx, most / shape->OH);
+    shape->local = ((nty + shape->OH - 1) / shape->OH) * ((ntx + shape->OW - 1) / shape->OW);
+    return hipSuccess;
 }
 
-hipError_t launch_iteration(float* x, float* g, const float* amap, const float* psf2, int p2h, int p2w, int H, int W,
-                            Cand* tiles, Cand* rows, State* state, hipStream_t st) {
-    const dim3 grid((p2w + kTile - 1) / kTile + 1, (p2h + kTile - 1) / kTile + 1);
-    hipLaunchKernelGGL(window_kernel, grid, dim3(kThreads), 0, st, x, g, amap, psf2, p2h, p2w, H, W, tiles, state);
-    hipLaunchKernelGGL(row_select_kernel, dim3(1), dim3(kThreads), 0, st, tiles, rows, p2h, H, W, state, x);
-    return hipGetLastError();
+hipError_t launch_descent(float* x, float* g, const float* amap, const float* psf2, int p2h, int p2w, int H, int W,
+                          const DescentShape& shape, float lambda, float alpha, float epsilon, int limit, Key* slots,
+                          Key* tiles, State* state, hipStream_t st) {
+    const int n = shape.OH * shape.OW;
+    hipLaunchKernelGGL(reset_slots_kernel, dim3((2 * n + kThreads - 1) / kThreads), dim3(kThreads), 0, st, slots, 2 * n);
+    if (hipError_t e = hipGetLastError()) return e;
+    Descent a{x, g, amap, psf2, p2h, p2w, H, W, shape.OH, shape.OW, lambda, alpha, epsilon, limit, slots, tiles, shape.local, state};
+    void* args[] = {&a};
+    const void* kernel = shape.local <= kLdsTiles ? reinterpret_cast<const void*>(descent_kernel<true>)
+                                                  : reinterpret_cast<const void*>(descent_kernel<false>);
+    return hipLaunchCooperativeKernel(kernel, dim3(n), dim3(kThreads), args, 0, st);
 }
 
 hipError_t launch_amap(const double* scan, int ph, int pw, int H, int W, float* amap, hipStream_t st) {
