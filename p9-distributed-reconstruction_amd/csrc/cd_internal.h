@@ -19,7 +19,7 @@ struct State {
     int32_t done;       // no further updates
     int32_t converged;  // the last selected |diff| was below epsilon
     int32_t updates;    // pixels changed by the launch
-    int32_t stalled;    // the workgroups could not exchange their selections
+    int32_t stalled;    // the workgroups were not all resident (1: nothing was changed)
     float absmax;       // GetAbsMaxDiff
     int32_t pad[3];
 };
@@ -35,12 +35,13 @@ hipError_t launch_absmax(const Key* tiles, int ntiles, State* state, hipStream_t
 struct DescentShape {
     int OH = 0, OW = 0, local = 0;
 };
-hipError_t descent_shape(int H, int W, DescentShape* shape);
-// Up to `limit` (> 0) iterations on x and g.  slots: 2 OH OW words; tiles:
-// OH OW local words.
+hipError_t descent_shape(int H, int W, int p2h, int p2w, DescentShape* shape);
+size_t descent_slots(const DescentShape& shape);  // words
+// Up to `limit` (> 0) iterations on x and g.  resident: with the gradients in
+// LDS where they fit, one workgroup per CU.  tiles: OH OW local words.
 hipError_t launch_descent(float* x, float* g, const float* amap, const float* psf2, int p2h, int p2w, int H, int W,
-                          const DescentShape& shape, float lambda, float alpha, float epsilon, int limit, Key* slots,
-                          Key* tiles, State* state, hipStream_t st);
+                          const DescentShape& shape, bool resident, float lambda, float alpha, float epsilon, int limit,
+                          Key* slots, Key* tiles, State* state, hipStream_t st);
 
 // PaddedConvolver / CalcPaddedFourierCorrelation pieces (complex double
 // buffers of N0 x N1).

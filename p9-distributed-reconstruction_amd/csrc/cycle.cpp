@@ -360,11 +360,19 @@ int cd_run(p9cd* c, float* d_x, float* d_g, float lambda, float alpha, int32_t m
     cd::State& s = *c->h_state;
     s = cd::State{};
     int32_t made = 0;
+    bool resident = true;
     while (!s.done && made < max_iter) {
-        P9_HIP(cd::launch_descent(d_x, d_g, c->d_amap, c->d_psf2, c->p2h, c->p2w, c->H, c->W, c->shape, lambda, alpha, eps,
-                                  std::min(max_iter - made, kPerLaunch), c->d_slots, c->d_tiles, c->d_state, c->stream));
+        P9_HIP(cd::launch_descent(d_x, d_g, c->d_amap, c->d_psf2, c->p2h, c->p2w, c->H, c->W, c->shape, resident, lambda,
+                                  alpha, eps, std::min(max_iter - made, kPerLaunch), c->d_slots, c->d_tiles, c->d_state,
+                                  c->stream));
         P9_HIP(hipMemcpyAsync(&s, c->d_state, sizeof(s), hipMemcpyDeviceToHost, c->stream));
         P9_HIP(hipStreamSynchronize(c->stream));
+        if (s.stalled == 1 && resident) {
+            // another program holds part of the CUs' LDS: the form that shares them
+            resident = false;
+            s = cd::State{};
+            continue;
+        }
         if (s.stalled) return fail(P9IDG_ERR_HIP, "the deconvolution's workgroups did not all become resident");
         made += s.updates;
     }
@@ -396,12 +404,12 @@ int p9cd_create(int32_t device, int32_t height, int32_t width, const float* psf,
         return st;
     };
     if (hipStreamCreate(&c->stream) != hipSuccess) return bail(fail(P9IDG_ERR_HIP, "stream creation failed"));
-    if (hipError_t e = cd::descent_shape(height, width, &c->shape)) return bail(hip_fail(e, "deconvolution launch shape"));
+    if (hipError_t e = cd::descent_shape(height, width, c->p2h, c->p2w, &c->shape)) return bail(hip_fail(e, "deconvolution launch shape"));
     const size_t workgroups = (size_t)c->shape.OH * c->shape.OW;
     int st;
     if ((st = alloc(&c->d_amap, (size_t)height * width)) || (st = alloc(&c->d_psf2, (size_t)c->p2h * c->p2w)) ||
         (st = alloc(&c->d_tiles, std::max((size_t)c->ntiles, workgroups * c->shape.local))) ||
-        (st = alloc(&c->d_slots, 2 * workgroups)) || (st = alloc(&c->d_state, 1)) ||
+        (st = alloc(&c->d_slots, cd::descent_slots(c->shape))) || (st = alloc(&c->d_state, 1)) ||
         (st = alloc(&c->d_io, 2 * (size_t)height * width)))
         return bail(st);
     if (hipHostMalloc(reinterpret_cast<void**>(&c->h_state), sizeof(cd::State), hipHostMallocDefault) != hipSuccess) {

@@ -19,6 +19,8 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kSelectThreads = 1024;
+constexpr int kDescent = 512;  // threads of a descent workgroup: 3072^2 3.5 us per iteration, 256 3.7, 1024 4.4
+constexpr int kCopies = 8;     // of the exchanged words
 static_assert(kTile * kTile % kThreads == 0, "whole pixels per thread");
 
 // Common.cs:27-29; Math.Max(v, 0f) gives +0 for -0
@@ -81,22 +83,40 @@ __device__ __forceinline__ float update_of(float old, float g, float a, float la
     return prox(__fadd_rn(__fmul_rn(old, a), g), a, lambda, alpha);
 }
 
-// The best update of tile (ty, tx), by one wave.
+// What a tile holds besides its best update: whether all its x are +0, and
+// whether its Lipschitz values are all `amap`.
+struct TileKind {
+    float amap;
+    bool zero, flat;
+};
+
+// The best update of tile (ty, tx), by one wave; own: the tile's gradients
+// (p = row * kTile + column), if not NULL.
 __device__ __forceinline__ Key tile_best(const float* __restrict__ x, const float* __restrict__ g,
                                          const float* __restrict__ amap, int H, int W, int ty, int tx, float lambda,
-                                         float alpha) {
+                                         float alpha, float* own, TileKind* kind) {
     const int lane = threadIdx.x & 63;
     const int j = tx * kTile + lane % kTile;
+    const float first = amap[(size_t)ty * kTile * W + tx * kTile];
     Key best = 0;
+    bool zero = true, flat = true;
     if (j < W)
-#pragma unroll 4
+#pragma unroll 8
         for (int r = lane / kTile; r < kTile; r += 64 / kTile) {
             const int i = ty * kTile + r;
             if (i >= H) break;
             const int idx = i * W + j;
-            const float old = x[idx];
-            best = max_key(best, make_key(__fsub_rn(old, update_of(old, g[idx], amap[idx], lambda, alpha)), idx));
+            const float old = x[idx], grad = g[idx], a = amap[idx];
+            best = max_key(best, make_key(__fsub_rn(old, update_of(old, grad, a, lambda, alpha)), idx));
+            if (own) own[r * kTile + lane % kTile] = grad;
+            zero = zero && __float_as_uint(old) == 0u;
+            flat = flat && __float_as_uint(a) == __float_as_uint(first);
         }
+    if (kind) {
+        kind->amap = first;
+        kind->zero = __all(zero);
+        kind->flat = __all(flat);
+    }
     return wave_max(best);
 }
 
@@ -106,7 +126,7 @@ __global__ __launch_bounds__(kThreads) void tiles_all_kernel(const float* x, con
                                                              int ntx, int ntiles) {
     const int t = (int)(blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6));
     if (t >= ntiles) return;
-    const Key k = tile_best(x, g, amap, H, W, t / ntx, t % ntx, lambda, alpha);
+    const Key k = tile_best(x, g, amap, H, W, t / ntx, t % ntx, lambda, alpha, nullptr, nullptr);
     if ((threadIdx.x & 63) == 0) tiles[t] = k;
 }
 
@@ -212,14 +232,22 @@ __global__ void amap_kernel(const double* s, int ph, int pw, int H, int W, float
 // (FastSerialCD.cs:219-238) and re-evaluate them.  A pixel is only ever touched
 // by one thread of its tile's workgroup.
 //
+// What bounds it is latency: 2 to 2.6 us of an iteration are the exchange over
+// the XCDs, the rest are the window's loads.  A launch pair per iteration
+// (window, then a one-workgroup selection) took 9.7 us, most of it between the
+// launches.  3072^2, PSF 192^2, 3000 iterations: 29.2 -> 10.5 ms.
+//
 // A published word holds the key and, in bit 63, the turn's tag, so one 64-bit
 // store hands over both and nothing else needs ordering.  Turn n uses buffer
 // n & 1 with tag (n >> 1) & 1: a workgroup writes turn n + 2 only after it has
 // read turn n + 1 from all, each of which had then finished reading turn n.
+// Every buffer has kCopies copies, each polled by every kCopies-th workgroup
+// (one copy: 3.3 us per exchange of 256 workgroups instead of 2.6).
 //
-// What bounds it is the latency of that exchange over the XCDs and of the
-// window's loads.  A launch pair per iteration (window, then a one-workgroup
-// selection) spent most of its time between launches.
+// RES: the tiles' gradients stay in LDS between the first and the last turn.
+// x and the Lipschitz map are read only where a tile's are not all zero or all
+// equal, so that a window's tile usually waits for nothing but psf2 (16.5 ->
+// 11.1 ms together with the copies).
 struct Descent {
     float* x;
     float* g;
@@ -228,66 +256,100 @@ struct Descent {
     int p2h, p2w, H, W, OH, OW;
     float lambda, alpha, epsilon;
     int limit;    // updates of this launch
-    Key* slots;   // [2][OH * OW]
+    Key* slots;   // [2][kCopies][OH * OW], then the gate's two words
     Key* tiles;   // [OH * OW][local]: the tile tables where they don't fit LDS
     int local;
     State* st;
 };
 constexpr int kLdsTiles = 1024;
+constexpr int kResTiles = 38;  // 4 KB each
 constexpr Key kStalled = ~(Key)0;
-// Polls of one slot before the exchange is given up (seconds: only if the
-// launch's workgroups could not all become resident).
-constexpr int kMaxPolls = 1 << 25;
+constexpr int kGatePolls = 1 << 19;  // a fraction of a second
+constexpr int kMaxPolls = 1 << 28;
 
-// The slots' tags before turn 0: neither buffer holds its first turn.
+// The slots' tags before turn 0 (neither buffer holds its first turn) and the
+// gate: arrivals, verdict.
 __global__ void reset_slots_kernel(Key* slots, int n) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) slots[i] = (Key)1 << 63;
+    if (i < n + 2) slots[i] = i < n ? (Key)1 << 63 : 0;
 }
 
+__device__ __forceinline__ Key poll(const Key* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
 __device__ __forceinline__ Key await_slot(const Key* slot, unsigned tag) {
     for (int i = 0; i < kMaxPolls; i++) {
-        const Key v = __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const Key v = poll(slot);
         if ((unsigned)(v >> 63) == tag) return v & ~((Key)1 << 63);
     }
     return kStalled;
 }
+// Whether all workgroups of the launch are resident: the last to arrive opens
+// the gate, the first to lose patience shuts it, and the first verdict holds
+// for all.  Nothing has been changed before it.
+__device__ __forceinline__ bool all_resident(Key* gate, Key nwg) {
+    if (__hip_atomic_fetch_add(gate, (Key)1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 == nwg) atomicCAS(gate + 1, (Key)0, (Key)1);
+    for (int i = 0; i < kGatePolls; i++)
+        if (const Key v = poll(gate + 1)) return v == 1;
+    const Key before = atomicCAS(gate + 1, (Key)0, (Key)2);
+    return before == 1;
+}
 
-template <bool LDS>
-__global__ __launch_bounds__(kThreads) void descent_kernel(Descent a) {
-    constexpr int kWaves = kThreads / 64, kPer = kTile * kTile / kThreads;
-    __shared__ Key s_table[LDS ? kLdsTiles : 1];
+template <bool LDS, bool RES>
+__global__ __launch_bounds__(kDescent) void descent_kernel(Descent a) {
+    static_assert(LDS || !RES, "resident tiles have their table in LDS");
+    constexpr int kWaves = kDescent / 64, kPer = kTile * kTile / kDescent, kTiles = RES ? kResTiles : LDS ? kLdsTiles : 1;
+    __shared__ float s_g[RES ? kResTiles * kTile * kTile : 1];
+    __shared__ Key s_table[kTiles];
+    __shared__ float s_amap[kTiles];
+    __shared__ unsigned char s_zero[kTiles], s_flat[kTiles];
     __shared__ Key s_turn[2][kWaves], s_tile[2][kWaves];
+    __shared__ int s_go;
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int H = a.H, W = a.W, OH = a.OH, OW = a.OW, me = blockIdx.x, nwg = OH * OW;
+    if (t == 0) s_go = all_resident(a.slots + 2 * kCopies * nwg, nwg);
     const int ntx = (W + kTile - 1) / kTile, nty = (H + kTile - 1) / kTile;
     const int oy = me / OW, ox = me - oy * OW;
     const int nrow = (nty - oy + OH - 1) / OH, ncol = (ntx - ox + OW - 1) / OW, nlocal = nrow * ncol;
     Key* const table = LDS ? s_table : a.tiles + (size_t)me * a.local;
     for (int l = wave; l < nlocal; l += kWaves) {
-        const Key k = tile_best(a.x, a.g, a.amap, H, W, oy + l / ncol * OH, ox + l % ncol * OW, a.lambda, a.alpha);
-        if (lane == 0) table[l] = k;
+        TileKind kind;
+        const Key k = tile_best(a.x, a.g, a.amap, H, W, oy + l / ncol * OH, ox + l % ncol * OW, a.lambda, a.alpha,
+                                RES ? s_g + l * kTile * kTile : nullptr, LDS ? &kind : nullptr);
+        if (lane == 0) {
+            table[l] = k;
+            if (LDS) {
+                s_amap[l] = kind.amap;
+                s_zero[l] = kind.zero;
+                s_flat[l] = kind.flat;
+            }
+        }
     }
     __threadfence_block();
     __syncthreads();
+    if (!s_go) {
+        if (me == 0 && t == 0) a.st->stalled = 1;
+        return;  // every workgroup
+    }
     const int yh = a.p2h / 2, xh = a.p2w / 2;
     Key mine = 0, best = 0;
     bool changed = true;  // of this workgroup's tiles
     int updates = 0;
     for (unsigned turn = 0;; turn++) {
+        Key* const slots = a.slots + (turn & 1) * kCopies * nwg;
+        const unsigned tag = (turn >> 1) & 1;
         if (wave == 0) {
             if (changed) {
                 mine = 0;
                 for (int l = lane; l < nlocal; l += 64) mine = max_key(mine, table[l]);
                 mine = wave_max(mine);
             }
-            if (lane == 0)
-                __hip_atomic_store(a.slots + (turn & 1) * nwg + me, mine | ((Key)((turn >> 1) & 1) << 63), __ATOMIC_RELAXED,
+            if (lane < kCopies)
+                __hip_atomic_store(slots + lane * nwg + me, mine | ((Key)tag << 63), __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_AGENT);
         }
         Key v = 0;
-        for (int s = t; s < nwg; s += kThreads)
-            v = max_key(v, await_slot(a.slots + (turn & 1) * nwg + s, (turn >> 1) & 1));
+        for (int s = t; s < nwg; s += kDescent) v = max_key(v, await_slot(slots + me % kCopies * nwg + s, tag));
         v = wave_max(v);
         if (lane == 0) s_turn[turn & 1][wave] = v;
         __syncthreads();
@@ -304,19 +366,22 @@ __global__ __launch_bounds__(kThreads) void descent_kernel(Descent a) {
         // the first own tile at or after (tya, txa) in each direction
         for (int ty = tya + (oy + OH - tya % OH) % OH; ty <= tyb; ty += OH)
             for (int tx = txa + (ox + OW - txa % OW) % OW; tx <= txb; tx += OW, q++) {
+                const int l = (ty / OH) * ncol + tx / OW;
+                const bool zero = LDS && s_zero[l], flat = LDS && s_flat[l];  // uniform but for the update's own clearing of zero
+                const float amap = LDS ? s_amap[l] : 0.f;
                 int idx[kPer];
                 bool in[kPer], win[kPer];
                 float gv[kPer], pv[kPer], xv[kPer], av[kPer];
 #pragma unroll
                 for (int k = 0; k < kPer; k++) {
-                    const int p = t + k * kThreads, i = ty * kTile + p / kTile, j = tx * kTile + p % kTile;
+                    const int p = t + k * kDescent, i = ty * kTile + p / kTile, j = tx * kTile + p % kTile;
                     in[k] = i < H && j < W;
                     win[k] = in[k] && i >= r0 && i < r1 && j >= c0 && j < c1;
                     idx[k] = in[k] ? i * W + j : 0;
-                    gv[k] = in[k] ? a.g[idx[k]] : 0.f;
-                    xv[k] = in[k] ? a.x[idx[k]] : 0.f;
-                    av[k] = in[k] ? a.amap[idx[k]] : 0.f;
                     pv[k] = win[k] ? a.psf2[(i - y0 + yh) * a.p2w + (j - x0 + xh)] : 0.f;
+                    gv[k] = RES ? s_g[l * kTile * kTile + p] : in[k] ? a.g[idx[k]] : 0.f;
+                    xv[k] = !zero && in[k] ? a.x[idx[k]] : 0.f;
+                    av[k] = flat ? amap : in[k] ? a.amap[idx[k]] : 0.f;
                 }
                 Key b = 0;
 #pragma unroll
@@ -325,25 +390,37 @@ __global__ __launch_bounds__(kThreads) void descent_kernel(Descent a) {
                     if (idx[k] == at) {  // the update itself
                         xv[k] = update_of(xv[k], gv[k], av[k], a.lambda, a.alpha);
                         a.x[at] = xv[k];
+                        if (LDS) s_zero[l] = 0;
                     }
                     if (win[k]) {
                         gv[k] = __fadd_rn(gv[k], __fmul_rn(pv[k], d));
-                        a.g[idx[k]] = gv[k];
+                        if (RES)
+                            s_g[l * kTile * kTile + t + k * kDescent] = gv[k];
+                        else
+                            a.g[idx[k]] = gv[k];
                     }
                     b = max_key(b, make_key(__fsub_rn(xv[k], update_of(xv[k], gv[k], av[k], a.lambda, a.alpha)), idx[k]));
                 }
                 b = wave_max(b);
                 if (lane == 0) s_tile[q & 1][wave] = b;
                 __syncthreads();
-                if (t == 0) table[(ty / OH) * ncol + tx / OW] = max_of<kWaves>(s_tile[q & 1]);
+                if (t == 0) table[l] = max_of<kWaves>(s_tile[q & 1]);
             }
         changed = q > 0;
         if (changed) __threadfence_block();  // wave 0 reads what its lane 0 wrote
         if (updates >= a.limit) break;
     }
+    if (RES)
+        for (int l = 0; l < nlocal; l++)
+#pragma unroll
+            for (int k = 0; k < kPer; k++) {
+                const int p = t + k * kDescent;  // this thread's own elements, after a barrier in any case
+                const int i = (oy + l / ncol * OH) * kTile + p / kTile, j = (ox + l % ncol * OW) * kTile + p % kTile;
+                if (i < H && j < W) a.g[i * W + j] = s_g[l * kTile * kTile + p];
+            }
     if (me == 0 && t == 0) {
         const bool stop = updates < a.limit || best == 0 || key_diff(best) < a.epsilon;
-        a.st->stalled = best == kStalled;
+        a.st->stalled = best == kStalled ? 2 : 0;
         a.st->updates = updates;
         a.st->done = stop;
         a.st->converged = stop && key_diff(best) < a.epsilon;
@@ -413,36 +490,51 @@ hipError_t launch_extract(const double2* buf, int N1, int yh, int xh, double nor
     return hipGetLastError();
 }
 
-hipError_t descent_shape(int H, int W, DescentShape* shape) {
-    int dev = 0, cus = 0, per = 0;
+namespace {
+
+const void* descent_of(int local, bool resident) {
+    return resident && local <= kResTiles ? reinterpret_cast<const void*>(descent_kernel<true, true>)
+           : local <= kLdsTiles           ? reinterpret_cast<const void*>(descent_kernel<true, false>)
+                                          : reinterpret_cast<const void*>(descent_kernel<false, false>);
+}
+
+}  // namespace
+
+hipError_t descent_shape(int H, int W, int p2h, int p2w, DescentShape* shape) {
+    int dev = 0, cus = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    if (e == hipSuccess)
-        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, reinterpret_cast<const void*>(descent_kernel<true>), kThreads, 0);
     if (e != hipSuccess) return e;
-    // one workgroup per CU at most: the exchange grows with their number
-    const int most = cus * std::min(per, 1);
-    if (most < 1) return hipErrorInvalidConfiguration;
     const int ntx = (W + kTile - 1) / kTile, nty = (H + kTile - 1) / kTile;
-    const int side = std::max(1, (int)std::sqrt((double)most));
-    shape->OW = std::min(side, ntx);
-    shape->OH = std::min(nty, most / shape->OW);
-    shape->OW = std::min(ntx, most / shape->OH);
-    shape->local = ((nty + shape->OH - 1) / shape->OH) * ((ntx + shape->OW - 1) / shape->OW);
+    auto arrange = [&](int side) {
+        shape->OW = std::min(side, ntx);
+        shape->OH = std::min(nty, side * side / shape->OW);
+        shape->OW = std::min(ntx, side * side / shape->OH);
+        shape->local = ((nty + shape->OH - 1) / shape->OH) * ((ntx + shape->OW - 1) / shape->OW);
+    };
+    // The exchange is faster among fewer workgroups, so no more than the
+    // window's tiles, unless only more of them hold all gradients in LDS.  us
+    // per iteration, 8 x 8 / 11 x 11 / 16 x 16: 512^2 with a 64^2 window 3.1 /
+    // 3.3 / 3.8, 1500^2 with 200^2 3.3 / 3.5 / 3.8, 3072^2 with 384^2 (too
+    // large for LDS below 16 x 16) 6.3 / 6.4 / 3.5.
+    const int most = std::max(1, (int)std::sqrt((double)std::max(cus, 1)));  // one workgroup per CU at most
+    const int window = std::max(p2h, p2w) / kTile + 1;
+    arrange(std::min(most, std::max(8, window)));
+    if (shape->local > kResTiles) arrange(most);
     return hipSuccess;
 }
 
+size_t descent_slots(const DescentShape& shape) { return 2 * kCopies * (size_t)shape.OH * shape.OW + 2; }
+
 hipError_t launch_descent(float* x, float* g, const float* amap, const float* psf2, int p2h, int p2w, int H, int W,
-                          const DescentShape& shape, float lambda, float alpha, float epsilon, int limit, Key* slots,
-                          Key* tiles, State* state, hipStream_t st) {
-    const int n = shape.OH * shape.OW;
-    hipLaunchKernelGGL(reset_slots_kernel, dim3((2 * n + kThreads - 1) / kThreads), dim3(kThreads), 0, st, slots, 2 * n);
+                          const DescentShape& shape, bool resident, float lambda, float alpha, float epsilon, int limit,
+                          Key* slots, Key* tiles, State* state, hipStream_t st) {
+    const int n = shape.OH * shape.OW, words = 2 * kCopies * n;
+    hipLaunchKernelGGL(reset_slots_kernel, dim3((words + 2 + kThreads - 1) / kThreads), dim3(kThreads), 0, st, slots, words);
     if (hipError_t e = hipGetLastError()) return e;
     Descent a{x, g, amap, psf2, p2h, p2w, H, W, shape.OH, shape.OW, lambda, alpha, epsilon, limit, slots, tiles, shape.local, state};
     void* args[] = {&a};
-    const void* kernel = shape.local <= kLdsTiles ? reinterpret_cast<const void*>(descent_kernel<true>)
-                                                  : reinterpret_cast<const void*>(descent_kernel<false>);
-    return hipLaunchCooperativeKernel(kernel, dim3(n), dim3(kThreads), args, 0, st);
+    return hipLaunchCooperativeKernel(descent_of(shape.local, resident), dim3(n), dim3(kDescent), args, 0, st);
 }
 
 hipError_t launch_amap(const double* scan, int ph, int pw, int H, int W, float* amap, hipStream_t st) {

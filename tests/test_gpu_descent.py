@@ -37,7 +37,8 @@ def _compare(O, shape, n, x, g, lam, alpha, iters, eps):
 @pytest.mark.parametrize("shape,n,iters", [
     ((1, 1), 1, 3), ((32, 32), 4, 40), ((33, 31), 8, 40), ((16, 700), 10, 60), ((515, 40), 12, 60),
     ((640, 640), 300, 25),       # windows of 600 pixels: two tiles per workgroup and direction
-    ((513, 545), 33, 60),        # 17 x 18 tiles: one more than the workgroups' arrangement
+    ((513, 545), 33, 60),        # 17 x 18 tiles on 8 x 8 workgroups
+    ((256 * 32 * 39 + 5, 1), 4, 12),  # 40 tiles per workgroup: gradients not in LDS
     ((1, 5000), 3, 30), ((9000, 1), 3, 30),
 ])
 def test_descent_matches_the_oracle(O, shape, n, iters):
