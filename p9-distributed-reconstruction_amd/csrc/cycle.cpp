@@ -76,12 +76,45 @@ struct p9conv {
     bool have_plan = false;
     double2* d_kernel = nullptr;
     double2* d_buf = nullptr;
+    // line transforms (kernels_conv.hip) where the padded size is even (FFT.Shift
+    // leaves an odd size's last row and column in place) and a line length
+    // reaches it: d_kernel is the spectrum, d_buf their intermediate
+    bool lines = false;
+    LinePlan line{};
+    double2* d_tw = nullptr;
     float* d_io = nullptr;  // [2][H][W] staging for host-array calls
 };
 
 namespace {
 
+// Spectrum and buffers of the line transforms.
+int conv_lines(p9conv* c, const float* psf) {
+    const int n = c->line.n;
+    std::vector<double2> tw(n);
+    for (int k = 0; k < n; k++) {
+        const double a = 2.0 * M_PI * (double)k / (double)n;
+        tw[k] = make_double2(std::cos(a), std::sin(a));
+    }
+    if (int st = alloc(&c->d_kernel, (size_t)(n / 2 + 1) * n)) return st;
+    if (int st = alloc(&c->d_buf, (size_t)(n / 2 + 2) * (std::max(c->H, c->ph) + 1))) return st;
+    if (int st = alloc(&c->d_tw, (size_t)n)) return st;
+    if (int st = alloc(&c->d_io, 2 * (size_t)std::max(c->H, c->ph) * std::max(c->W, c->pw))) return st;
+    P9_HIP(hipMemcpyAsync(c->d_tw, tw.data(), n * sizeof(double2), hipMemcpyHostToDevice, c->stream));
+    P9_HIP(hipMemcpyAsync(c->d_io, psf, sizeof(float) * c->ph * c->pw, hipMemcpyHostToDevice, c->stream));
+    // Common.cs:146-160: the turned PSF at H / 2 + 1 before the quadrant swap
+    const int yoff = c->H / 2 + 1 - c->N0 / 2, xoff = c->W / 2 + 1 - c->N1 / 2;
+    P9_HIP(launch_conv_spectrum(c->d_io, c->ph, c->pw, (yoff + n) % n, (xoff + n) % n, c->line, c->d_tw, c->d_buf, c->d_kernel,
+                                c->stream));
+    P9_HIP(hipStreamSynchronize(c->stream));
+    return P9IDG_OK;
+}
+
 int conv_run(p9conv* c, const float* d_in, float* d_out) {
+    if (c->lines) {
+        P9_HIP(launch_conv(d_in, c->H, c->W, c->line, c->d_tw, c->d_buf, c->d_kernel, d_out, c->stream));
+        P9_HIP(hipStreamSynchronize(c->stream));
+        return P9IDG_OK;
+    }
     const size_t n = (size_t)c->N0 * c->N1;
     P9_HIP(cd::launch_insert_image(d_in, c->H, c->W, c->ph / 2, c->pw / 2, c->N0, c->N1, c->d_buf, c->stream));
     P9_FFT(hipfftExecZ2Z(c->plan, reinterpret_cast<hipfftDoubleComplex*>(c->d_buf),
@@ -120,6 +153,12 @@ int p9conv_create_correlation(int32_t device, const float* psf, int32_t rows, in
         return st;
     };
     if (hipStreamCreate(&c->stream) != hipSuccess) return bail(fail(P9IDG_ERR_HIP, "stream creation failed"));
+    c->lines = c->N0 % 2 == 0 && conv_line_plan(c->N0, c->line);
+    if (c->lines) {
+        if (int st = conv_lines(c, psf)) return bail(st);
+        *out = c;
+        return P9IDG_OK;
+    }
     if (hipfftPlan2d(&c->plan, c->N0, c->N1, HIPFFT_Z2Z) != HIPFFT_SUCCESS)
         return bail(fail(P9IDG_ERR_HIP, "hipFFT plan failed"));
     c->have_plan = true;
@@ -150,6 +189,7 @@ int p9conv_destroy(p9conv* c) {
     if (c->have_plan) (void)hipfftDestroy(c->plan);
     release(c->d_kernel);
     release(c->d_buf);
+    release(c->d_tw);
     release(c->d_io);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;

@@ -209,7 +209,7 @@ constexpr int kMaxLine = 4096, kMaxPasses = 8;
 struct LinePlan {
     int32_t n, passes, radix[kMaxPasses];
 };
-bool line_plan(int n, LinePlan& p);
+bool line_plan(int n, LinePlan& p, bool nine = false);  // nine: radix 9 too (FP64)
 constexpr int line_pitch(int n) { return n / 2 + 8; }  // mid's row pitch in launch_line_grid
 // The w-layers summed over the union u of their boxes, dense.
 hipError_t launch_sum_boxes(const float2* layers, const Box* boxes, int nboxes, int G, Box u, float2* out, hipStream_t st);
@@ -220,6 +220,15 @@ hipError_t launch_line_image(const float2* src, bool dense, Box u, const LinePla
 // Forward transform of the quadrant-swapped image; mid: G x line_pitch(G).
 hipError_t launch_line_grid(const float* img, const LinePlan& p, const float2* tw, float2* mid, float2* grid,
                             hipStream_t st);
+// The padded correlation (kernels_conv.hip).  conv_line_plan: the line length
+// for at least `least` points.  mid: (n / 2 + 2) x (rows + 1) values at most;
+// spectrum: (n / 2 + 1) x n.  yoff, xoff: where the turned PSF's first row and
+// column lie (modulo n).
+bool conv_line_plan(int least, LinePlan& p);
+hipError_t launch_conv_spectrum(const float* psf, int rows, int cols, int yoff, int xoff, const LinePlan& p,
+                                const double2* tw, double2* mid, double2* spectrum, hipStream_t st);
+hipError_t launch_conv(const float* img, int rows, int cols, const LinePlan& p, const double2* tw, double2* mid,
+                       const double2* spectrum, float* out, hipStream_t st);
 hipError_t launch_sum_layers(const float2* layers, int L, size_t GG, float2* out, hipStream_t st);
 hipError_t launch_scale_c64(float2* p, size_t n, double inv_norm, hipStream_t st);
 
