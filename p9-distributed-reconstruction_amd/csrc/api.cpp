@@ -98,6 +98,8 @@ struct p9idg_plan {
     int32_t grid_src = P9IDG_SRC_VIS;
     // captured major-cycle step
     bool capturing = false;
+    int32_t cycle_mode = 0;    // the recorded cycle's grid mode
+    bool cycle_keeps = false;  // and whether its ToImage leaves the grid as gridded
     hipGraph_t graph = nullptr;
     hipGraphExec_t graph_exec = nullptr;
     // Zero state of the gridder targets.  A buffer is "clean" when it is zero
@@ -422,6 +424,18 @@ int build_resample(p9idg_plan* p, int T, int C, const double* freq) {
     p->rs.nchunks = (int32_t)nc;
     p->have_rs = true;
     return P9IDG_OK;
+}
+
+// After work that cleared the whole target of `mode` and gridded into it
+// without zero_target's knowledge (a replayed graph, a batch).
+void mark_gridded(p9idg_plan* p, int mode) {
+    if (mode == P9IDG_GRID_WSTACK) {
+        p->layers_clean = true;
+        p->layers_dirty_fp = mode;
+    } else {
+        p->grid_clean = true;
+        p->grid_dirty_fp = mode;
+    }
 }
 
 // Brings the gridder target of `mode` to all-zero: the previous footprint
@@ -1570,6 +1584,9 @@ int p9idg_capture_cycle(p9idg_plan* p, int32_t grid_mode) {
     p->capturing = true;
     int st = cycle_step(p, grid_mode);
     p->capturing = false;
+    p->cycle_mode = grid_mode;
+    // what the last call leaves in a plain grid is what each replay leaves
+    p->cycle_keeps = grid_mode == P9IDG_GRID_WSTACK || p->grid_clean;
     mark_unknown(p);
     hipGraph_t g = nullptr;
     hipError_t e = hipStreamEndCapture(p->stream, &g);
@@ -1592,6 +1609,11 @@ int p9idg_launch_cycle(p9idg_plan* p) {
     if (!p->graph_exec) return fail(P9IDG_ERR_STATE, "no captured cycle (p9idg_capture_cycle)");
     DeviceGuard dg(p->device);
     P9_HIP(hipGraphLaunch(p->graph_exec, p->stream));
+    if (p->cycle_keeps)
+        mark_gridded(p, p->cycle_mode);
+    else
+        p->grid_clean = false;
+    p->model_vis_clean = true;
     return P9IDG_OK;
 }
 
@@ -1861,6 +1883,7 @@ struct p9idg_batch {
     std::vector<Group> groups;
     int grid_mode = P9IDG_GRID_WSTACK, degrid_mode = P9IDG_DEGRID_WSTACK;
     bool prepared = false;
+    int graph_what = 0;  // directions that the recorded graph runs
     hipGraph_t graph = nullptr;
     hipGraphExec_t graph_exec = nullptr;
     hipEvent_t ev[5] = {};
@@ -1926,33 +1949,48 @@ int batch_order_out(p9idg_batch* b) {
     return P9IDG_OK;
 }
 
-// One persistent launch per group, on the batch stream or fanned out over the
-// groups' streams.
-int batch_launch_groups(p9idg_batch* b, bool grid) {
+hipError_t batch_zero_grid(const p9idg_batch* b, const p9idg_plan* p, hipStream_t st) {
+    const bool wstack = b->grid_mode == P9IDG_GRID_WSTACK;
+    return launch_fill_zero(wstack ? p->d_layers : p->d_grid, grid_elems(p) * (wstack ? p->c.wlayer_count : 1), st);
+}
+
+// One group's launches of one direction; zero: with the members' zero fills.
+int batch_launch_group(p9idg_batch* b, p9idg_batch::Group& g, bool grid, bool zero, hipStream_t st) {
+    for (size_t m = 0; m < g.members.size(); m++) {
+        const p9idg_plan* p = b->plans[g.members[m]];
+        if (grid) {
+            if (zero) P9_HIP(batch_zero_grid(b, p, st));
+            if (g.resampled[m]) P9_HIP(launch_resample_gather(p->rs, p->C, p->d_vis, p->d_rs_vis, st));
+        } else if (zero) {
+            P9_HIP(launch_fill_zero(p->d_model_vis, vis_elems(p), st));
+        }
+    }
+    if (grid) {
+        BatchArgs ba{g.d_args_grid, g.d_items_grid, g.n_grid, g.d_counter};
+        const hipError_t e = launch_grid_batch(ba, g.S, g.kernel, g.workgroups, st);
+        return e == hipSuccess ? P9IDG_OK : hip_fail(e, "batched gridder launch");
+    }
+    BatchArgs ba{g.d_args_degrid, g.d_items_degrid, g.n_degrid, g.d_counter};
+    hipError_t e = launch_degrid_batch(ba, g.S, g.kernel, g.workgroups_degrid, st);
+    for (size_t m = 0; m < g.members.size(); m++) {
+        const p9idg_plan* p = b->plans[g.members[m]];
+        if (g.resampled[m] && e == hipSuccess) e = launch_resample_spread(p->rs, p->C, p->d_rs_vis, p->d_model_vis, st);
+    }
+    return e == hipSuccess ? P9IDG_OK : hip_fail(e, "batched degridder launch");
+}
+
+// The groups' launches for `what`, on the batch stream or fanned out over the
+// groups' streams.  Each group passes from its zero fills through both
+// directions without waiting for the others.
+int batch_launch_groups(p9idg_batch* b, int what, bool zero) {
     const bool fan = b->side.size() == b->groups.size() && b->groups.size() > 1;
     if (fan) P9_HIP(hipEventRecord(b->fork, b->stream));
     for (size_t i = 0; i < b->groups.size(); i++) {
-        auto& g = b->groups[i];
         hipStream_t st = fan ? b->side[i] : b->stream;
         if (fan) P9_HIP(hipStreamWaitEvent(st, b->fork, 0));
-        hipError_t e = hipSuccess;
-        if (grid) {
-            for (size_t m = 0; m < g.members.size(); m++) {
-                const p9idg_plan* p = b->plans[g.members[m]];
-                if (g.resampled[m]) P9_HIP(launch_resample_gather(p->rs, p->C, p->d_vis, p->d_rs_vis, st));
-            }
-            BatchArgs ba{g.d_args_grid, g.d_items_grid, g.n_grid, g.d_counter};
-            e = launch_grid_batch(ba, g.S, g.kernel, g.workgroups, st);
-        } else {
-            BatchArgs ba{g.d_args_degrid, g.d_items_degrid, g.n_degrid, g.d_counter};
-            e = launch_degrid_batch(ba, g.S, g.kernel, g.workgroups_degrid, st);
-            for (size_t m = 0; m < g.members.size(); m++) {
-                const p9idg_plan* p = b->plans[g.members[m]];
-                if (g.resampled[m] && e == hipSuccess)
-                    e = launch_resample_spread(p->rs, p->C, p->d_rs_vis, p->d_model_vis, st);
-            }
-        }
-        if (e != hipSuccess) return hip_fail(e, grid ? "batched gridder launch" : "batched degridder launch");
+        for (int dir : {1, 2})
+            if (what & dir)
+                if (int s = batch_launch_group(b, b->groups[i], dir == 1, zero, st)) return s;
         if (fan) P9_HIP(hipEventRecord(b->side_done[i], st));
     }
     if (fan)
@@ -1960,30 +1998,34 @@ int batch_launch_groups(p9idg_batch* b, bool grid) {
     return P9IDG_OK;
 }
 
-// Zero fills and one persistent launch per (subgrid size, kernel) group.
-int batch_run(p9idg_batch* b, int what, bool capturing) {
+// The plans' buffers after a run of `what`: cleared as a whole and gridded.
+void batch_mark(p9idg_batch* b, int what) {
+    for (p9idg_plan* p : b->plans) {
+        if (what & 1) mark_gridded(p, b->grid_mode);
+        if (what & 2) p->model_vis_clean = true;
+    }
+}
+
+// Eager: zero fills and one persistent launch per (subgrid size, kernel) group,
+// direction after direction with the timing events between them.
+int batch_run(p9idg_batch* b, int what) {
     if (int st = batch_check(b)) return st;
     for (p9idg_plan* p : b->plans) mark_unknown(p);
-    if (!capturing) P9_HIP(hipEventRecord(b->ev[0], b->stream));
+    P9_HIP(hipEventRecord(b->ev[0], b->stream));
     if (what & 1) {
-        for (p9idg_plan* p : b->plans) {
-            float2* target = b->grid_mode == P9IDG_GRID_WSTACK ? p->d_layers : p->d_grid;
-            size_t n = grid_elems(p) * (b->grid_mode == P9IDG_GRID_WSTACK ? p->c.wlayer_count : 1);
-            P9_HIP(launch_fill_zero(target, n, b->stream));
-        }
-        if (!capturing) P9_HIP(hipEventRecord(b->ev[1], b->stream));
-        if (int st = batch_launch_groups(b, true)) return st;
+        for (p9idg_plan* p : b->plans) P9_HIP(batch_zero_grid(b, p, b->stream));
+        P9_HIP(hipEventRecord(b->ev[1], b->stream));
+        if (int st = batch_launch_groups(b, 1, false)) return st;
     }
-    if (!capturing) P9_HIP(hipEventRecord(b->ev[2], b->stream));
+    P9_HIP(hipEventRecord(b->ev[2], b->stream));
     if (what & 2) {
         for (p9idg_plan* p : b->plans) P9_HIP(launch_fill_zero(p->d_model_vis, vis_elems(p), b->stream));
-        if (!capturing) P9_HIP(hipEventRecord(b->ev[3], b->stream));
-        if (int st = batch_launch_groups(b, false)) return st;
+        P9_HIP(hipEventRecord(b->ev[3], b->stream));
+        if (int st = batch_launch_groups(b, 2, false)) return st;
     }
-    if (!capturing) {
-        P9_HIP(hipEventRecord(b->ev[4], b->stream));
-        b->timed = (what & 1) && (what & 2);
-    }
+    P9_HIP(hipEventRecord(b->ev[4], b->stream));
+    b->timed = (what & 1) && (what & 2);
+    batch_mark(b, what);
     return P9IDG_OK;
 }
 
@@ -2132,7 +2174,7 @@ int p9idg_batch_exec(p9idg_batch* b, int32_t what) {
     DeviceGuard dg(b->device);
     if (int st = batch_check(b)) return st;
     if (int st = batch_order_in(b)) return st;
-    if (int st = batch_run(b, what, false)) return st;
+    if (int st = batch_run(b, what)) return st;
     return batch_order_out(b);
 }
 
@@ -2145,10 +2187,10 @@ int p9idg_batch_capture(p9idg_batch* b, int32_t what) {
     b->graph = nullptr;
     if (int st = batch_check(b)) return st;
     if (int st = batch_order_in(b)) return st;
-    if (int st = batch_run(b, what, false)) return st;  // warm: occupancy figures, first launches
+    if (int st = batch_run(b, what)) return st;  // warm: occupancy figures, first launches
     P9_HIP(hipStreamSynchronize(b->stream));
     P9_HIP(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
-    int st = batch_run(b, what, true);
+    int st = batch_launch_groups(b, what, true);
     hipGraph_t g = nullptr;
     hipError_t e = hipStreamEndCapture(b->stream, &g);
     if (st) {
@@ -2157,6 +2199,7 @@ int p9idg_batch_capture(p9idg_batch* b, int32_t what) {
     }
     if (e != hipSuccess) return hip_fail(e, "hipStreamEndCapture");
     b->graph = g;
+    b->graph_what = what;
     e = hipGraphInstantiate(&b->graph_exec, g, nullptr, nullptr, 0);
     if (e != hipSuccess) return hip_fail(e, "hipGraphInstantiate");
     return P9IDG_OK;
@@ -2169,6 +2212,7 @@ int p9idg_batch_launch(p9idg_batch* b) {
     if (int st = batch_check(b)) return st;
     if (int st = batch_order_in(b)) return st;
     P9_HIP(hipGraphLaunch(b->graph_exec, b->stream));
+    batch_mark(b, b->graph_what);
     return batch_order_out(b);
 }
 
