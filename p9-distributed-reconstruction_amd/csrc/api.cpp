@@ -1659,6 +1659,7 @@ int p9idg_autotune(p9idg_plan* p, int32_t reps, float* grid_ms, float* degrid_ms
                     {p->use_queue, p->degrid_chunk, p->workgroups_degrid}};
     const int32_t q0 = p->use_queue, g0 = p->grid_chunk, d0 = p->degrid_chunk, w0 = p->workgroups;
     p->launch_chosen = true;
+    bool warm = false;
     for (const Cand& c : cands) {
         p->use_queue = c.queue;
         p->grid_chunk = c.chunk;
@@ -1666,6 +1667,15 @@ int p9idg_autotune(p9idg_plan* p, int32_t reps, float* grid_ms, float* degrid_ms
         p->workgroups = c.wg;
         p->workgroups_degrid = c.wg;
         if (int st = upload_items(p)) return st;
+        // the first launches of a plan run on low clocks: not the first candidate's time
+        for (int dir = 0; dir < 2 && !warm; dir++) {
+            float ms = 0.f;
+            if (int st = time_direction(p, dir, 4, &ms)) {
+                p->collect = collect;
+                return st;
+            }
+        }
+        warm = true;
         for (int dir = 0; dir < 2; dir++) {
             float ms = 0.f;
             if (int st = time_direction(p, dir, reps, &ms)) {
