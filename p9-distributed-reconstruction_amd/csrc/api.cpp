@@ -472,7 +472,7 @@ int ensure_line(p9idg_plan* p) {
         const double a = 2.0 * M_PI * (double)k / (double)G;
         tw[k] = make_float2((float)std::cos(a), (float)std::sin(a));
     }
-    if (int st = dev_alloc(&p->d_line_mid, (size_t)G * std::max(G, line_pitch(G)))) return st;
+    if (int st = dev_alloc(&p->d_line_mid, (size_t)G * G)) return st;
     if (int st = dev_alloc(&p->d_line_tw, (size_t)G)) return st;
     P9_HIP(hipMemcpy(p->d_line_tw, tw.data(), G * sizeof(float2), hipMemcpyHostToDevice));
     return P9IDG_OK;

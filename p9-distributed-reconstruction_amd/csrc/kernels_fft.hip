@@ -5,9 +5,9 @@
 //   ToImage  transforms only the box's columns (v -> y), then pairs of rows
 //            (u -> x) whose Hermitian parts share one complex transform:
 //            Re(IFFT) of two rows at once, written as whole image rows;
-//   ToUVW    transforms pairs of real image rows with one complex transform,
-//            keeps the G / 2 + 1 columns that determine the rest, transforms
-//            them and writes each with its conjugate mirror.
+//   ToUVW    transforms pairs of real image columns with one complex transform,
+//            keeps the G / 2 + 1 rows that determine the rest, transforms them
+//            and writes each with its conjugate mirror.
 // A 2-D library transform moves the complex grid four times (read + write per
 // pass, 75 MB each way at 3072^2) besides the real <-> complex copies.
 #include "device_linefft.h"
@@ -37,8 +37,9 @@ __global__ void sum_boxes_kernel(const float2* layers, const Box* boxes, int nbo
 // ToImage, columns: column u.x0 + c of the box (dense array, or the
 // quadrant-swapped grid) over v; mid[y][c] for every storage row y.
 template <int MAXN, int LINES>
-__global__ __launch_bounds__(kLine * LINES) void image_columns_kernel(const float2* src, bool dense, Box u, LinePlan plan,
-                                                                      const float2* tw, float2* mid) {
+__global__ __launch_bounds__(kLine * LINES) void image_columns_kernel(const float2* src, bool dense, Box u,
+                                                                                   LinePlan plan, const float2* tw,
+                                                                                   float2* mid) {
     __shared__ float2 s_line[LINES][line_slots(MAXN)];
     const int t = threadIdx.x % kLine, l = threadIdx.x / kLine, G = plan.n, h = G / 2;
     const int w = u.x1 - u.x0, c = blockIdx.x * LINES + l;
@@ -64,8 +65,8 @@ __global__ __launch_bounds__(kLine * LINES) void image_columns_kernel(const floa
 // ToImage, rows: storage rows 2 b and 2 b + 1 over u; image rows scaled by
 // inv_n, quadrant-swapped.
 template <int MAXN>
-__global__ __launch_bounds__(kLine) void image_rows_kernel(const float2* mid, Box u, LinePlan plan, const float2* tw,
-                                                           double inv_n, float* img) {
+__global__ __launch_bounds__(kLine) void image_rows_kernel(const float2* mid, Box u, LinePlan plan,
+                                                                        const float2* tw, double inv_n, float* img) {
     __shared__ float2 line[line_slots(MAXN)];
     const int t = threadIdx.x, G = plan.n, h = G / 2, w = u.x1 - u.x0;
     const int y0 = 2 * blockIdx.x, y1 = y0 + 1;  // G is even
@@ -98,51 +99,59 @@ __global__ __launch_bounds__(kLine) void image_rows_kernel(const float2* mid, Bo
     }
 }
 
-// ToUVW, rows: storage rows 2 b and 2 b + 1 of the quadrant-swapped image;
-// mid[y][f] for f = 0 .. G / 2 (row pitch `pitch`).
-template <int MAXN>
-__global__ __launch_bounds__(kLine) void grid_rows_kernel(const float* img, LinePlan plan, const float2* tw, int pitch,
-                                                          float2* mid) {
-    __shared__ float2 line[line_slots(MAXN)];
-    const int t = threadIdx.x, G = plan.n, h = G / 2;
-    const int y0 = 2 * blockIdx.x, y1 = y0 + 1;
-    const float* i0 = img + (size_t)(y0 >= h ? y0 - h : y0 + h) * G;
-    const float* i1 = img + (size_t)(y1 >= h ? y1 - h : y1 + h) * G;
-    for (int x = t; x < G; x += kLine) {
-        const int at = x >= h ? x - h : x + h;
-        line[slot(x)] = make_float2(i0[at], i1[at]);
-    }
-    __syncthreads();
-    line_fft<-1, MAXN, kLine>(line, plan, tw, t);
-    for (int f = t; f <= h; f += kLine) {
-        const float2 z = line[slot(f)], c = line[slot(f ? G - f : 0)];
-        mid[(size_t)y0 * pitch + f] = make_float2(0.5f * (z.x + c.x), 0.5f * (z.y - c.y));
-        mid[(size_t)y1 * pitch + f] = make_float2(0.5f * (z.y + c.y), 0.5f * (c.x - z.x));
-    }
-}
-// ToUVW, columns: columns f and their mirrors G - f.
+// ToUVW, columns: LINES pairs of real columns of the quadrant-swapped image, a
+// pair as one complex line; mid[f][x] for f = 0 .. G / 2.  The grid's rows are
+// then written whole: with the rows first, the columns' 32-byte pieces of the
+// grid and of its mirror were the larger half of the time (4096^2 182 -> 133
+// us, 3072^2 87 -> 76, 2048^2 59 -> 45).
 template <int MAXN, int LINES>
-__global__ __launch_bounds__(kLine * LINES) void grid_columns_kernel(const float2* mid, int pitch, LinePlan plan,
-                                                                     const float2* tw, float2* grid) {
+__global__ __launch_bounds__(kLine * LINES) void grid_columns_kernel(const float* img, LinePlan plan,
+                                                                                  const float2* tw, float2* mid) {
     __shared__ float2 s_line[LINES][line_slots(MAXN)];
     const int G = plan.n, h = G / 2;
     // workgroups go round robin over the 8 XCDs: give each XCD neighbouring
     // columns, whose lines its L2 then holds for all of them
     const int per = (gridDim.x + 7) / 8, blk = (blockIdx.x % 8) * per + blockIdx.x / 8;
-    const int f0 = blk * LINES, cols = min(LINES, h + 1 - f0);
-    if (cols <= 0) return;  // whole workgroups
+    const int c0 = blk * LINES, lines = min(LINES, h - c0);  // column pairs
+    if (lines <= 0) return;  // whole workgroups
     for (int i = threadIdx.x; i < G * LINES; i += kLine * LINES) {
-        const int y = i / LINES, k = i % LINES;
-        s_line[k][slot(y)] = k < cols ? mid[(size_t)y * pitch + f0 + k] : make_float2(0.f, 0.f);
+        const int y = i / LINES, k = i % LINES, x = 2 * (c0 + k);
+        float2 e = make_float2(0.f, 0.f);
+        if (k < lines) {
+            const float* row = img + (size_t)(y >= h ? y - h : y + h) * G;
+            e.x = row[x >= h ? x - h : x + h];
+            e.y = row[x + 1 >= h ? x + 1 - h : x + 1 + h];
+        }
+        s_line[k][slot(y)] = e;
     }
     __syncthreads();
     line_fft<-1, MAXN, kLine>(s_line[threadIdx.x / kLine], plan, tw, threadIdx.x % kLine);
-    for (int i = threadIdx.x; i < G * LINES; i += kLine * LINES) {
-        const int v = i / LINES, k = i % LINES, f = f0 + k;
-        if (k >= cols) continue;
-        const float2 e = s_line[k][slot(v)];
-        grid[(size_t)v * G + f] = e;
-        if (f > 0 && f < h) grid[(size_t)(v ? G - v : 0) * G + G - f] = make_float2(e.x, -e.y);
+    for (int i = threadIdx.x; i < (h + 1) * LINES; i += kLine * LINES) {
+        const int f = i / LINES, k = i % LINES;
+        if (k >= lines) continue;
+        const float2 z = s_line[k][slot(f)], c = s_line[k][slot(f ? G - f : 0)];
+        float2* o = mid + (size_t)f * G + 2 * (c0 + k);
+        o[0] = make_float2(0.5f * (z.x + c.x), 0.5f * (z.y - c.y));
+        o[1] = make_float2(0.5f * (z.y + c.y), 0.5f * (c.x - z.x));
+    }
+}
+// ToUVW, rows: grid row f and its conjugate mirror G - f.
+template <int MAXN>
+__global__ __launch_bounds__(kLine) void grid_rows_kernel(const float2* mid, LinePlan plan, const float2* tw,
+                                                                       float2* grid) {
+    __shared__ float2 line[line_slots(MAXN)];
+    const int t = threadIdx.x, G = plan.n, h = G / 2, f = blockIdx.x;
+    const float2* in = mid + (size_t)f * G;
+    for (int x = t; x < G; x += kLine) line[slot(x)] = in[x];
+    __syncthreads();
+    line_fft<-1, MAXN, kLine>(line, plan, tw, t);
+    float2* o = grid + (size_t)f * G;
+    for (int u = t; u < G; u += kLine) o[u] = line[slot(u)];
+    if (f == 0 || f == h) return;
+    float2* m = grid + (size_t)(G - f) * G;
+    for (int u = t; u < G; u += kLine) {
+        const float2 e = line[slot(u ? G - u : 0)];
+        m[u] = make_float2(e.x, -e.y);
     }
 }
 
@@ -184,16 +193,14 @@ hipError_t launch_line_image(const float2* src, bool dense, Box u, const LinePla
 }
 
 hipError_t launch_line_grid(const float* img, const LinePlan& p, const float2* tw, float2* mid, float2* grid, hipStream_t st) {
-    constexpr int L = 4;
-    const int pitch = line_pitch(p.n);
-#define P9_ROWS(N) \
-    hipLaunchKernelGGL((dev::grid_rows_kernel<N>), dim3(p.n / 2), dim3(dev::kLine), 0, st, img, p, tw, pitch, mid)
-#define P9_COLS(N)                                                                                                           \
-    hipLaunchKernelGGL((dev::grid_columns_kernel<N, L>), dim3(((p.n / 2 + 1 + L - 1) / L + 7) / 8 * 8), dim3(dev::kLine * L), 0, \
-                       st, mid, pitch, p, tw, grid)
-    P9_LINE(P9_ROWS);
-    if (hipError_t e = hipGetLastError()) return e;
+    constexpr int L = 2;  // 3072^2: as many workgroups as the chip holds; 4: 88 us
+    const unsigned blocks = ((p.n / 2 + L - 1) / L + 7) / 8 * 8;
+#define P9_COLS(N) \
+    hipLaunchKernelGGL((dev::grid_columns_kernel<N, L>), dim3(blocks), dim3(dev::kLine * L), 0, st, img, p, tw, mid)
+#define P9_ROWS(N) hipLaunchKernelGGL((dev::grid_rows_kernel<N>), dim3(p.n / 2 + 1), dim3(dev::kLine), 0, st, mid, p, tw, grid)
     P9_LINE(P9_COLS);
+    if (hipError_t e = hipGetLastError()) return e;
+    P9_LINE(P9_ROWS);
 #undef P9_COLS
 #undef P9_ROWS
     return hipGetLastError();

@@ -210,14 +210,13 @@ struct LinePlan {
     int32_t n, passes, radix[kMaxPasses];
 };
 bool line_plan(int n, LinePlan& p, bool nine = false);  // nine: radix 9 too (FP64)
-constexpr int line_pitch(int n) { return n / 2 + 8; }  // mid's row pitch in launch_line_grid
 // The w-layers summed over the union u of their boxes, dense.
 hipError_t launch_sum_boxes(const float2* layers, const Box* boxes, int nboxes, int G, Box u, float2* out, hipStream_t st);
 // Quadrant-swapped real image x inv_n of a grid that is zero outside u: src is
 // that box (dense) or the quadrant-swapped grid; mid: G x (u.x1 - u.x0).
 hipError_t launch_line_image(const float2* src, bool dense, Box u, const LinePlan& p, const float2* tw, float2* mid,
                              double inv_n, float* img, hipStream_t st);
-// Forward transform of the quadrant-swapped image; mid: G x line_pitch(G).
+// Forward transform of the quadrant-swapped image; mid: (G / 2 + 1) x G.
 hipError_t launch_line_grid(const float* img, const LinePlan& p, const float2* tw, float2* mid, float2* grid,
                             hipStream_t st);
 // The padded correlation (kernels_conv.hip).  conv_line_plan: the line length
