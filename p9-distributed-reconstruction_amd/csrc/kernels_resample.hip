@@ -168,17 +168,17 @@ __global__ __launch_bounds__(kMaxLen) void analyse_kernel(const ResampleChunk* c
 }
 
 // Weights of one (len, nodes) pair per workgroup, FP64 rounded to float, in
-// both orders: to[j][t] for the degridder's interpolation behind from[t][j]
-// for the gridder's sums.
+// both orders: [t][j] for the degridder's interpolation, [j][t] behind it for
+// the gridder's sums.
 __global__ void weights_kernel(const ResamplePair* pairs, float* weights) {
     const ResamplePair p = pairs[blockIdx.x];
-    float* from = weights + p.offset;
-    float* to = from + (size_t)p.len * p.nodes;
+    float* tj = weights + p.offset;
+    float* jt = tj + (size_t)p.len * p.nodes;
     for (int i = threadIdx.x; i < p.len * p.nodes; i += blockDim.x) {
         const int t = i / p.nodes, j = i - t * p.nodes;
         const float w = (float)cardinal(angle_of((double)t, p.len), node_angle(j, p.nodes), p.nodes);
-        from[i] = w;
-        to[(size_t)j * p.len + t] = w;
+        tj[i] = w;
+        jt[(size_t)j * p.len + t] = w;
     }
 }
 
@@ -207,124 +207,221 @@ __global__ __launch_bounds__(kMaxLen) void node_track_kernel(const ResampleChunk
     }
 }
 
-// Rows of one chunk copied as they are (16 floats per column tile).
-__device__ __forceinline__ void copy_rows(const float* in, float* out, int rows, int width, int n, int g, bool col) {
-    if (!col) return;
-    for (int r = g; r < rows; r += 4) out[(size_t)r * width + n] = in[(size_t)r * width + n];
+// Four consecutive floats, 4-byte aligned.
+__device__ __forceinline__ rs_f32x4 load4(const float* p) {
+    rs_f32x4 v;
+    __builtin_memcpy(&v, p, sizeof(v));
+    return v;
 }
 
-// One chunk's 16 columns for up to 16 Q nodes, in one sweep over the timesteps.
-template <int Q>
+// The `count` (even) floats of a chunk that is kept as it is, by wave `w` of
+// `waves`, four vectors in flight per lane.
+__device__ __forceinline__ void copy_rows(const float* in, float* out, int count, int lane, int w, int waves) {
+    constexpr int U = 4;
+    const int step = 256 * waves;
+    for (int i = (64 * w + lane) * 4; i < count; i += U * step) {
+        rs_f32x4 v[U];
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (i + u * step + 3 < count) v[u] = load4(in + i + u * step);
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int at = i + u * step;
+            if (at + 3 < count)
+                __builtin_memcpy(out + at, &v[u], sizeof(v[u]));
+            else if (at < count)
+                for (int k = 0; k < 2; k++) out[at + k] = in[at + k];
+        }
+    }
+}
+
+// A lane's four neighbouring columns c .. c + 3 of a row of `width` (even).
+__device__ __forceinline__ void store4(float* row, int c, int width, rs_f32x4 v) {
+    if (c + 3 < width)
+        __builtin_memcpy(row + c, &v, sizeof(v));
+    else if (c < width)
+        __builtin_memcpy(row + c, &v, 2 * sizeof(float));
+}
+
+// One chunk's 16 columns for up to 16 Q nodes, in one sweep over the timesteps
+// (steps of 16; SPLIT waves take turns), two steps in flight.  MFMA k of a step
+// takes timestep 4 g + k from lane group g, so that a lane's four weights of a
+// node lie side by side in w[j][t].  sum: LDS of [SPLIT - 1][16][64] floats.
+template <int Q, int SPLIT>
 __device__ __forceinline__ void gather_chunk(const float* src, const float* w, float* dst, int len, int J, int width, int n,
-                                             int nc, int m, int g, bool col) {
+                                             int nc, int m, int g, int part, float* sum) {
     rs_f32x4 acc[Q];
-    int jq[Q];
+    const float* row[Q];
 #pragma unroll
     for (int q = 0; q < Q; q++) {
         acc[q] = (rs_f32x4){};
-        jq[q] = min(16 * q + m, J - 1);
+        row[q] = w + (size_t)min(16 * q + m, J - 1) * len + 4 * g;
     }
-    for (int t0 = 0; t0 < len; t0 += 16) {
-        float v[4], wt[4][Q];
+    const int full = len & ~15;
+    const float* in = src + (size_t)(4 * g) * width + nc;
+    constexpr int D = 2, kStep = 16 * SPLIT;
+    float v[D][4];
+    rs_f32x4 wt[D][Q];
+    auto load = [&](int d, int t0) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) v[d][k] = in[(size_t)(t0 + k) * width];
+#pragma unroll
+        for (int q = 0; q < Q; q++) wt[d][q] = load4(row[q] + t0);
+    };
+#pragma unroll
+    for (int d = 0; d < D; d++)
+        if (16 * part + kStep * d < full) load(d, 16 * part + kStep * d);
+    for (int t1 = 16 * part; t1 < full; t1 += kStep * D)
+#pragma unroll
+        for (int d = 0; d < D; d++) {
+            const int t0 = t1 + kStep * d;
+            if (t0 >= full) break;
+            float b[4];
+            rs_f32x4 a[Q];
+#pragma unroll
+            for (int k = 0; k < 4; k++) b[k] = v[d][k];
+#pragma unroll
+            for (int q = 0; q < Q; q++) a[q] = wt[d][q];
+            if (t0 + kStep * D < full) load(d, t0 + kStep * D);
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+#pragma unroll
+                for (int q = 0; q < Q; q++)
+                    acc[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[k], a[q][k], acc[q], 0, 0, 0);
+        }
+    if (full < len && full / 16 % SPLIT == part) {
+        float b[4], a[4][Q];
 #pragma unroll
         for (int k = 0; k < 4; k++) {
-            const int t = t0 + 4 * k + g, tt = min(t, len - 1);
-            v[k] = src[(size_t)tt * width + nc];
+            const int t = full + 4 * g + k, tt = min(t, len - 1);
+            const float x = src[(size_t)tt * width + nc];
+            b[k] = t < len ? x : 0.f;
 #pragma unroll
-            for (int q = 0; q < Q; q++) wt[k][q] = w[(size_t)tt * J + jq[q]];
+            for (int q = 0; q < Q; q++) a[k][q] = row[q][tt - 4 * g];
         }
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
-            const float b = t0 + 4 * k + g < len ? v[k] : 0.f;
+        for (int k = 0; k < 4; k++)
 #pragma unroll
-            for (int q = 0; q < Q; q++) acc[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(wt[k][q], b, acc[q], 0, 0, 0);
-        }
+            for (int q = 0; q < Q; q++) acc[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[k], a[k][q], acc[q], 0, 0, 0);
+    }
+    if (SPLIT > 1) {
+        const int lane = 16 * g + m;
+        if (part > 0)
+#pragma unroll
+            for (int q = 0; q < Q; q++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) sum[((part - 1) * 16 + 4 * q + r) * 64 + lane] = acc[q][r];
+        __syncthreads();
+        if (part > 0) return;
+#pragma unroll
+        for (int p = 0; p < SPLIT - 1; p++)
+#pragma unroll
+            for (int q = 0; q < Q; q++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) acc[q][r] += sum[(p * 16 + 4 * q + r) * 64 + lane];
     }
 #pragma unroll
     for (int q = 0; q < Q; q++)
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const int j = 16 * q + 4 * g + r;
-            if (j < J && col) dst[(size_t)j * width + n] = acc[q][r];
-        }
+        if (16 * q + m < J) store4(dst + (size_t)(16 * q + m) * width, n - m + 4 * g, width, acc[q]);
 }
 
 // out[j][n] = sum_t W[t][j] in[t][n] for every chunk, n over the real columns
 // of a row of channels, on v_mfma_f32_16x16x4_f32: FP32 products and sums on
 // the matrix cores, so the visibilities and weights keep 24 bits.  A wave owns
-// a chunk and 16 columns (8 channels): A = W (16 nodes x 4 timesteps), B = 4
-// rows of visibilities straight from HBM (256 contiguous bytes per load at 8
-// channels).
+// a chunk and 16 columns (8 channels); with SPLIT 4 the workgroup's waves share
+// them.  Bound by the reads of the visibilities: 134 MB (3072^2) in 37 us, 47
+// with one weight per load and one step in flight.
+template <int SPLIT>
 __global__ __launch_bounds__(256) void gather_rows_kernel(const ResampleChunk* chunks, int nchunks, int ntiles,
                                                           const float* weights, int width, const float* in, float* out) {
-    const int unit = (int)(blockIdx.x * 4 + (threadIdx.x >> 6));
+    __shared__ float s_sum[SPLIT > 1 ? (SPLIT - 1) * 16 * 64 : 1];
+    const int wave = threadIdx.x >> 6, part = SPLIT > 1 ? wave : 0;
+    const int unit = SPLIT > 1 ? (int)blockIdx.x : (int)(blockIdx.x * 4 + wave);
     const int ci = unit / ntiles;
-    if (ci >= nchunks) return;  // whole waves
+    if (ci >= nchunks) return;  // whole waves, or workgroups where they share
     const ResampleChunk c = chunks[ci];
     const int lane = threadIdx.x & 63, m = lane & 15, g = lane >> 4;
     const int n = (unit - ci * ntiles) * 16 + m;
     const bool col = n < width;
     const float* src = in + (size_t)c.src * width;
     float* dst = out + (size_t)c.dst * width;
-    if (c.nodes == 0) return copy_rows(src, dst, c.len, width, n, g, col);
-    const float* w = weights + c.weights;
+    if (c.nodes == 0) return copy_rows(src, dst, c.len * width, lane, (unit - ci * ntiles) * SPLIT + part, ntiles * SPLIT);
     const int J = c.nodes, len = c.len, nc = col ? n : 0;
+    const float* w = weights + c.weights + (size_t)len * J;  // [j][t]
     switch ((J + 15) >> 4) {  // uniform
-        case 1: return gather_chunk<1>(src, w, dst, len, J, width, n, nc, m, g, col);
-        case 2: return gather_chunk<2>(src, w, dst, len, J, width, n, nc, m, g, col);
-        case 3: return gather_chunk<3>(src, w, dst, len, J, width, n, nc, m, g, col);
-        default: return gather_chunk<4>(src, w, dst, len, J, width, n, nc, m, g, col);
+        case 1: return gather_chunk<1, SPLIT>(src, w, dst, len, J, width, n, nc, m, g, part, s_sum);
+        case 2: return gather_chunk<2, SPLIT>(src, w, dst, len, J, width, n, nc, m, g, part, s_sum);
+        case 3: return gather_chunk<3, SPLIT>(src, w, dst, len, J, width, n, nc, m, g, part, s_sum);
+        default: return gather_chunk<4, SPLIT>(src, w, dst, len, J, width, n, nc, m, g, part, s_sum);
     }
 }
 
-// One chunk's 16 columns from up to 16 Q node rows, held in registers.
+// One chunk's 16 columns from up to 16 Q node rows, held in registers, the next
+// 16 timesteps' weights in flight (the four waves take turns).  MFMA k of quad q
+// takes node 16 q + 4 g + k from lane group g: four weights side by side in
+// w[t][j] (J is a multiple of 4).
 template <int Q>
 __device__ __forceinline__ void spread_chunk(const float* src, const float* w, float* dst, int len, int J, int width, int n,
-                                             int nc, int m, int g, bool col) {
-    float b[4 * Q];
+                                             int nc, int m, int g, int part) {
+    float b[Q][4];
+    int at[Q];
 #pragma unroll
-    for (int k = 0; k < 4 * Q; k++) b[k] = src[(size_t)min(4 * k + g, J - 1) * width + nc];
-    for (int t0 = 0; t0 < len; t0 += 16) {
-        const int ta = min(t0 + m, len - 1);
-        float a[4 * Q];
+    for (int q = 0; q < Q; q++) {
+        const int j = 16 * q + 4 * g;
+        at[q] = min(j, J - 4);
 #pragma unroll
-        for (int k = 0; k < 4 * Q; k++) {
-            const float wt = w[(size_t)min(4 * k + g, J - 1) * len + ta];
-            a[k] = 4 * k + g < J ? wt : 0.f;
+        for (int k = 0; k < 4; k++) {
+            const float x = src[(size_t)(at[q] + k) * width + nc];
+            b[q][k] = j < J ? x : 0.f;
         }
+    }
+    rs_f32x4 wt[Q];
+    auto load = [&](int t0) {
+        const float* row = w + (size_t)min(t0 + m, len - 1) * J;
+#pragma unroll
+        for (int q = 0; q < Q; q++) wt[q] = load4(row + at[q]);
+    };
+    load(16 * part);
+    for (int t0 = 16 * part; t0 < len; t0 += 64) {
+        rs_f32x4 a[Q];
+#pragma unroll
+        for (int q = 0; q < Q; q++) a[q] = wt[q];
+        if (t0 + 64 < len) load(t0 + 64);
         rs_f32x4 acc[2] = {(rs_f32x4){}, (rs_f32x4){}};
 #pragma unroll
-        for (int k = 0; k < 4 * Q; k++) acc[k & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[k], b[k], acc[k & 1], 0, 0, 0);
+        for (int q = 0; q < Q; q++)
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const int t = t0 + 4 * g + r;
-            if (t < len && col) dst[(size_t)t * width + n] = acc[0][r] + acc[1][r];
-        }
+            for (int k = 0; k < 4; k++)
+                acc[k & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[q][k], a[q][k], acc[k & 1], 0, 0, 0);
+        rs_f32x4 sum;
+#pragma unroll
+        for (int r = 0; r < 4; r++) sum[r] = acc[0][r] + acc[1][r];
+        if (t0 + m < len) store4(dst + (size_t)(t0 + m) * width, n - m + 4 * g, width, sum);
     }
 }
 
 // out[t][n] = sum_j W[t][j] in[j][n]: the degridded nodes interpolated to the
-// timesteps, 16 timesteps x 16 columns per MFMA tile, the chunk's node rows
-// held in registers as the B operands.
-__global__ __launch_bounds__(256) void spread_rows_kernel(const ResampleChunk* chunks, int nchunks, int ntiles,
+// timesteps, 16 timesteps x 16 columns per MFMA tile, a workgroup per chunk and
+// 16 columns (one wave each: 46 us at 3072^2).  Bound by the writes: 134 MB
+// (3072^2) in 35 us, 50 with one weight per load and one float per store.
+__global__ __launch_bounds__(256) void spread_rows_kernel(const ResampleChunk* chunks, int ntiles,
                                                           const float* weights, int width, const float* in, float* out) {
-    const int unit = (int)(blockIdx.x * 4 + (threadIdx.x >> 6));
+    const int part = threadIdx.x >> 6, unit = blockIdx.x;
     const int ci = unit / ntiles;
-    if (ci >= nchunks) return;
     const ResampleChunk c = chunks[ci];
     const int lane = threadIdx.x & 63, m = lane & 15, g = lane >> 4;
     const int n = (unit - ci * ntiles) * 16 + m;
     const bool col = n < width;
     const float* src = in + (size_t)c.dst * width;
     float* dst = out + (size_t)c.src * width;
-    if (c.nodes == 0) return copy_rows(src, dst, c.len, width, n, g, col);
+    if (c.nodes == 0) return copy_rows(src, dst, c.len * width, lane, (unit - ci * ntiles) * 4 + part, ntiles * 4);
     const int J = c.nodes, len = c.len, nc = col ? n : 0;
-    const float* w = weights + c.weights + (size_t)len * J;  // [j][t]
+    const float* w = weights + c.weights;  // [t][j]
     switch ((J + 15) >> 4) {  // uniform
-        case 1: return spread_chunk<1>(src, w, dst, len, J, width, n, nc, m, g, col);
-        case 2: return spread_chunk<2>(src, w, dst, len, J, width, n, nc, m, g, col);
-        case 3: return spread_chunk<3>(src, w, dst, len, J, width, n, nc, m, g, col);
-        default: return spread_chunk<4>(src, w, dst, len, J, width, n, nc, m, g, col);
+        case 1: return spread_chunk<1>(src, w, dst, len, J, width, n, nc, m, g, part);
+        case 2: return spread_chunk<2>(src, w, dst, len, J, width, n, nc, m, g, part);
+        case 3: return spread_chunk<3>(src, w, dst, len, J, width, n, nc, m, g, part);
+        default: return spread_chunk<4>(src, w, dst, len, J, width, n, nc, m, g, part);
     }
 }
 
@@ -347,21 +444,25 @@ hipError_t launch_resample_tables(const ResamplePair* pairs, int npairs, float* 
     return hipGetLastError();
 }
 namespace {
-unsigned row_blocks(const Resample& r, int C) {
-    const int64_t units = (int64_t)r.nchunks * ((2 * C + 15) / 16);
-    return (unsigned)((units + 3) / 4);
-}
+// (chunk, column tile) units; below kSplitUnits of them, a quarter of the waves
+// the chip holds, four waves share each in the gather: 1327 units 11.1 -> 9.5 us,
+// but 3424 units 12.5 -> 13.8 and 10674 45 -> 55.
+constexpr int64_t kSplitUnits = 2048;
+int64_t row_units(const Resample& r, int C) { return (int64_t)r.nchunks * ((2 * C + 15) / 16); }
 }  // namespace
 hipError_t launch_resample_gather(const Resample& r, int C, const float2* vis, float2* out, hipStream_t st) {
     if (r.nchunks <= 0) return hipSuccess;
-    hipLaunchKernelGGL(dev::gather_rows_kernel, dim3(row_blocks(r, C)), dim3(256), 0, st, r.chunks, r.nchunks,
+    const int64_t units = row_units(r, C);
+    const bool split = units < kSplitUnits;
+    hipLaunchKernelGGL(split ? dev::gather_rows_kernel<4> : dev::gather_rows_kernel<1>,
+                       dim3((unsigned)(split ? units : (units + 3) / 4)), dim3(256), 0, st, r.chunks, r.nchunks,
                        (2 * C + 15) / 16, r.weights, 2 * C, reinterpret_cast<const float*>(vis),
                        reinterpret_cast<float*>(out));
     return hipGetLastError();
 }
 hipError_t launch_resample_spread(const Resample& r, int C, const float2* rows, float2* vis, hipStream_t st) {
     if (r.nchunks <= 0) return hipSuccess;
-    hipLaunchKernelGGL(dev::spread_rows_kernel, dim3(row_blocks(r, C)), dim3(256), 0, st, r.chunks, r.nchunks,
+    hipLaunchKernelGGL(dev::spread_rows_kernel, dim3((unsigned)row_units(r, C)), dim3(256), 0, st, r.chunks,
                        (2 * C + 15) / 16, r.weights, 2 * C, reinterpret_cast<const float*>(rows),
                        reinterpret_cast<float*>(vis));
     return hipGetLastError();

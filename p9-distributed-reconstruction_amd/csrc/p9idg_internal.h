@@ -97,7 +97,7 @@ struct ResampleChunk {
     int32_t dst, len, nodes, pad;
 };
 struct ResamplePair {
-    int64_t offset;  // from[len][nodes], then to[nodes][len]
+    int64_t offset;  // [len][nodes], then [nodes][len]
     int32_t len, nodes;
 };
 // The device tables of a plan's resampled observation.
