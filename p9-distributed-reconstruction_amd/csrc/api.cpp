@@ -191,6 +191,8 @@ namespace {
 constexpr int64_t kResampleMinVis = 1 << 14;
 constexpr int64_t kResampleMinVisMfma = 1 << 18;
 constexpr double kResamplePays = 0.6;
+// Chunks up to this length are not halved any more.
+constexpr int kResampleSplitLen = 64;
 
 size_t padded(size_t bytes) { return (bytes + 255) & ~(size_t)255; }
 
@@ -328,22 +330,32 @@ bool want_resample(const p9idg_plan* p) {
 }
 
 // Splits the subgrids' timesteps into chunks, measures which of them can be
-// resampled and, where that pays, builds the resampled observation.  Called
-// with the plan's stream idle and the tracks' upload queued.
+// resampled (a chunk that cannot as a whole is tried in halves) and, where that
+// pays, builds the resampled observation.  Called with the plan's stream idle
+// and the tracks' upload queued.
 int build_resample(p9idg_plan* p, int T, int C, const double* freq) {
     p->have_rs = p->resampled = false;
     std::vector<p9idg_subgrid> meta = p->direct.meta;
     const int S = p->c.subgrid_size;
     const float image_size = p->c.scale_arcsec * (float)p->c.grid_size;
-    std::vector<ResampleChunk> chunks;
+    // a chunk and its place in the subgrids' order
+    struct Piece {
+        ResampleChunk c;
+        int64_t at;
+    };
+    std::vector<Piece> pending, done;
+    auto cut = [&](int64_t src, int64_t at, int len, int n) {
+        const int step = ((len + n - 1) / n + 15) / 16 * 16;
+        for (int t = 0; t < len; t += step) {
+            const int k = std::min(step, len - t);
+            pending.push_back({{src + t, 0, 0, k, 0, (k + 15) / 16 * 16}, at + t});
+        }
+    };
     int64_t rows = 0;
     for (const p9idg_subgrid& m : meta) {
-        const int nt = m.time_sample_count, n = (nt + kResampleMaxLen - 1) / kResampleMaxLen;
-        // multiples of 16 up to the last chunk, so few weight tables serve all
-        const int step = n > 0 ? ((nt + n - 1) / n + 15) / 16 * 16 : 1;
-        for (int t = 0; t < nt; t += step)
-            chunks.push_back({(int64_t)m.baseline_idx * T + m.time_sample_start + t, 0, 0, std::min(step, nt - t), 0, 0});
-        rows += nt;
+        const int nt = m.time_sample_count;
+        if (nt > 0) cut((int64_t)m.baseline_idx * T + m.time_sample_start, rows, nt, (nt + kResampleMaxLen - 1) / kResampleMaxLen);
+        rows += std::max(nt, 0);
     }
     if (rows * C < kResampleMinVis || rows > INT32_MAX) return P9IDG_OK;
     // corner pixel and highest wavenumber (Gridder.cs:163-174; n in double: an upper estimate suffices)
@@ -351,22 +363,43 @@ int build_resample(p9idg_plan* p, int T, int C, const double* freq) {
     for (int i = 0; i < C; i++) fmax = std::max(fmax, std::fabs(freq[i]));
     const double l = (0.5 * S - 0.5) * (double)image_size / S, t = 2.0 * l * l;
     const double kl = fmax / 299792458.0 * l, kn = fmax / 299792458.0 * (t < 1.0 ? t / (t + std::sqrt(1.0 - t)) : 1.0);
+    std::vector<ResampleChunk> chunks;
+    std::vector<int32_t> nodes;
+    for (int pass = 0; pass < 3 && !pending.empty(); pass++) {
+        const size_t n = pending.size(), nodes_at = padded(n * sizeof(ResampleChunk));
+        if (int st = dev_reserve(p->d_rs_chunks, p->alloc_rs_chunks, nodes_at + n * sizeof(int32_t))) return st;
+        ResampleChunk* const d_chunks = reinterpret_cast<ResampleChunk*>(p->d_rs_chunks);
+        int32_t* const d_nodes = reinterpret_cast<int32_t*>(p->d_rs_chunks + nodes_at);
+        chunks.clear();
+        for (const Piece& x : pending) chunks.push_back(x.c);
+        nodes.resize(n);
+        P9_HIP(hipMemcpyAsync(d_chunks, chunks.data(), n * sizeof(ResampleChunk), hipMemcpyHostToDevice, p->stream));
+        P9_HIP(launch_resample_analyse(d_chunks, (int)n, p->d_uvw, kl, kn, d_nodes, p->stream));
+        P9_HIP(hipMemcpyAsync(nodes.data(), d_nodes, n * sizeof(int32_t), hipMemcpyDeviceToHost, p->stream));
+        P9_HIP(hipStreamSynchronize(p->stream));
+        std::vector<Piece> tried;
+        tried.swap(pending);
+        for (size_t i = 0; i < n; i++) {
+            Piece& x = tried[i];
+            x.c.nodes = nodes[i];
+            if (x.c.nodes == 0 && x.c.len > kResampleSplitLen && pass < 2)
+                cut(x.c.src, x.at, x.c.len, 2);
+            else
+                done.push_back(x);
+        }
+    }
+    std::sort(done.begin(), done.end(), [](const Piece& a, const Piece& b) { return a.at < b.at; });
+    chunks.clear();
+    for (const Piece& x : done) chunks.push_back(x.c);
     const size_t nc = chunks.size();
-    const size_t nodes_at = padded(nc * sizeof(ResampleChunk));
-    if (int st = dev_reserve(p->d_rs_chunks, p->alloc_rs_chunks, nodes_at + nc * sizeof(int32_t))) return st;
-    p->rs.chunks = reinterpret_cast<ResampleChunk*>(p->d_rs_chunks);
-    int32_t* const d_nodes = reinterpret_cast<int32_t*>(p->d_rs_chunks + nodes_at);
-    P9_HIP(hipMemcpyAsync(p->rs.chunks, chunks.data(), nc * sizeof(ResampleChunk), hipMemcpyHostToDevice, p->stream));
-    P9_HIP(launch_resample_analyse(p->rs.chunks, (int)nc, p->d_uvw, kl, kn, d_nodes, p->stream));
-    std::vector<int32_t> nodes(nc);
-    P9_HIP(hipMemcpyAsync(nodes.data(), d_nodes, nc * sizeof(int32_t), hipMemcpyDeviceToHost, p->stream));
-    P9_HIP(hipStreamSynchronize(p->stream));
     int64_t kept = 0;
-    for (size_t i = 0; i < nc; i++) kept += nodes[i] > 0 ? nodes[i] : chunks[i].len;
+    for (const ResampleChunk& c : chunks) kept += c.nodes > 0 ? c.nodes : c.len;
     if ((double)kept > kResamplePays * (double)rows) return P9IDG_OK;
-    // rows in subgrid order, one weight table per (len, nodes) pair
+    if (int st = dev_reserve(p->d_rs_chunks, p->alloc_rs_chunks, nc * sizeof(ResampleChunk))) return st;
+    p->rs.chunks = reinterpret_cast<ResampleChunk*>(p->d_rs_chunks);
+    // rows in subgrid order, one weight table per (span, nodes) pair
     constexpr int kNodeSteps = kResampleMaxNodes / 4 + 1;
-    std::vector<int64_t> table((size_t)(kResampleMaxLen + 1) * kNodeSteps, -1);
+    std::vector<int64_t> table((size_t)(kResampleMaxLen / 16 + 1) * kNodeSteps, -1);
     std::vector<ResamplePair> pairs;
     int64_t weights = 0;
     int32_t dst = 0;
@@ -375,16 +408,15 @@ int build_resample(p9idg_plan* p, int T, int C, const double* freq) {
         const int32_t row0 = dst;
         for (int t = 0; t < m.time_sample_count; i++) {
             ResampleChunk& c = chunks[i];
-            c.nodes = nodes[i];
             c.dst = dst;
             dst += c.nodes > 0 ? c.nodes : c.len;
             t += c.len;
             if (c.nodes == 0) continue;
-            int64_t& at = table[(size_t)c.len * kNodeSteps + c.nodes / 4];
+            int64_t& at = table[(size_t)(c.span / 16) * kNodeSteps + c.nodes / 4];
             if (at < 0) {
                 at = weights;
-                pairs.push_back({weights, c.len, c.nodes});
-                weights += 2 * (int64_t)c.len * c.nodes;
+                pairs.push_back({weights, c.span, c.nodes});
+                weights += 2 * (int64_t)c.span * c.nodes;
             }
             c.weights = at;
         }

@@ -20,12 +20,19 @@
 // track itself, and takes the smallest number of nodes whose error is below
 // kResampleTol everywhere.  A track with a jump, noise or a gap fails the test
 // and keeps its rows as they are.
+//
+// Long chunks need fewer nodes in all (they grow with the phase that a chunk
+// covers, with some ten on top for each), but more weights and products per
+// row.  3072^2, subgrid 32, at most 256 / 512 / 1024 timesteps: gridder 141 / 132
+// / 124 us, gather 45 / 50 / 66; images at 1024^2 with FP32 106 / 93 us, three
+// uneven observations 646 / 597.  A chunk that would need more than 64 nodes is
+// halved.
 #include "device_common.h"
 
 namespace p9idg {
 namespace dev {
 
-constexpr int kMaxLen = kResampleMaxLen;
+constexpr int kAnalyse = 256;  // threads of analyse_kernel
 constexpr int kMaxNodes = kResampleMaxNodes;
 // samples that the track itself is interpolated from (degree 11: exact to
 // ~1e-14 of the track for chunks of an hour)
@@ -33,10 +40,10 @@ constexpr int kBase = 12;
 
 typedef float rs_f32x4 __attribute__((ext_vector_type(4)));
 
-// Angle of timestep t in a chunk of `len` (x = cos(angle) runs from 1 to -1)
-// and of Chebyshev node j of J.
-__device__ __forceinline__ double angle_of(double t, int len) {
-    const double x = 1.0 - 2.0 * t / (double)(len - 1);
+// Angle of timestep t in an interval of `span` (x = cos(angle) runs from 1 to
+// -1) and of Chebyshev node j of J.
+__device__ __forceinline__ double angle_of(double t, int span) {
+    const double x = 1.0 - 2.0 * t / (double)(span - 1);
     return acos(fmin(1.0, fmax(-1.0, x)));
 }
 __device__ __forceinline__ double node_angle(int j, int J) { return (kTwoPi / 4.0) * (double)(2 * j + 1) / (double)J; }
@@ -79,19 +86,19 @@ __device__ __forceinline__ double block_max_d(double v, double* red) {
     return fmax(fmax(red[0], red[1]), fmax(red[2], red[3]));
 }
 
-// One workgroup per chunk (thread t: timestep t): the smallest multiple of
-// four nodes whose interpolant reproduces the corner phasors of every
-// timestep to kResampleTol, or 0.  kl, kn: highest wavenumber / 2 pi times the
-// corner pixel's l and n.
-__global__ __launch_bounds__(kMaxLen) void analyse_kernel(const ResampleChunk* chunks, const double* uvw, double kl,
-                                                          double kn, int32_t* nodes_out) {
-    static_assert(kMaxLen == 256, "four waves reduce");
+// One workgroup per chunk (thread t: timesteps t, t + 256, ...): the smallest
+// multiple of four nodes whose interpolant reproduces the corner phasors of
+// every timestep to kResampleTol, or 0.  kl, kn: highest wavenumber / 2 pi times
+// the corner pixel's l and n.
+__global__ __launch_bounds__(kAnalyse) void analyse_kernel(const ResampleChunk* chunks, const double* uvw, double kl,
+                                                           double kn, int32_t* nodes_out) {
+    static_assert(kAnalyse == 256, "four waves reduce");
     __shared__ double s_base[kBase][3];
     __shared__ int s_bt[kBase];
     __shared__ double2 s_node[kMaxNodes][4];
     __shared__ double s_red[4];
     const ResampleChunk c = chunks[blockIdx.x];
-    const int tid = threadIdx.x, len = c.len;
+    const int tid = threadIdx.x, len = c.len, span = c.span;
     const int nb = min(kBase, len);
     const double* track = uvw + (size_t)c.src * 3;
     if (tid < nb) {
@@ -100,25 +107,29 @@ __global__ __launch_bounds__(kMaxLen) void analyse_kernel(const ResampleChunk* c
         for (int k = 0; k < 3; k++) s_base[tid][k] = track[(size_t)t * 3 + k];
     }
     __syncthreads();
-    // this timestep's corner phases relative to the chunk's first sample, in turns
-    const int tc = min(tid, len - 1);
+    // a timestep's corner phasors relative to the chunk's first sample; the largest phase in turns
     const double u0 = s_base[0][0], v0 = s_base[0][1], w0 = s_base[0][2];
-    const double du = (track[(size_t)tc * 3] - u0) * kl, dv = (track[(size_t)tc * 3 + 1] - v0) * kl;
-    const double dw = (track[(size_t)tc * 3 + 2] - w0) * kn;
-    double2 own[4];
-    double span = 0.0;
+    auto corners = [&](double u, double v, double w, double2* out) {
+        const double du = (u - u0) * kl, dv = (v - v0) * kl, dw = (w - w0) * kn;
+        double most = 0.0;
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
-        const double ph = ((q & 1) ? -du : du) + ((q & 2) ? -dv : dv) + dw;
-        sincospi(2.0 * ph, &own[q].y, &own[q].x);
-        span = fmax(span, fabs(ph));
+        for (int q = 0; q < 4; q++) {
+            const double ph = ((q & 1) ? -du : du) + ((q & 2) ? -dv : dv) + dw;
+            sincospi(2.0 * ph, &out[q].y, &out[q].x);
+            most = fmax(most, fabs(ph));
+        }
+        // not finite: fails every test below
+        return fabs(du) < 1e12 && fabs(dv) < 1e12 && fabs(dw) < 1e12 ? most : 1e9;
+    };
+    double phase = 0.0;
+    for (int t = tid; t < len; t += kAnalyse) {
+        double2 own[4];
+        phase = fmax(phase, corners(track[(size_t)t * 3], track[(size_t)t * 3 + 1], track[(size_t)t * 3 + 2], own));
     }
-    // not finite: fails every test below
-    const bool bad = !(fabs(du) < 1e12 && fabs(dv) < 1e12 && fabs(dw) < 1e12);
     // start where the Chebyshev coefficients 2 (z / 2)^J / J! of exp(i z s) fall
     // below the tolerance for z of half the span from the first sample
-    span = block_max_d(bad ? 1e9 : span, s_red);
-    const double z = (kTwoPi / 2.0) * span;
+    phase = block_max_d(phase, s_red);
+    const double z = (kTwoPi / 2.0) * phase;
     int start = 1;
     double term = 2.0 * (0.5 * z);
     while (start < kMaxNodes && (term > kResampleTol || (double)start < 0.5 * z)) {
@@ -127,37 +138,37 @@ __global__ __launch_bounds__(kMaxLen) void analyse_kernel(const ResampleChunk* c
     }
     const int limit = min(kMaxNodes, (int)(kResampleKeep * (double)len)) & ~3;
     int found = 0;
-    const double th = angle_of((double)tc, len);
     for (int J = (start + 3) & ~3; J <= limit; J += 4) {  // uniform
         __syncthreads();  // the previous candidate's nodes are read
         if (tid < J) {
             double p[3];
-            track_at(0.5 * (double)(len - 1) * (1.0 - cos(node_angle(tid, J))), s_base, s_bt, nb, p);
-            const double nu = (p[0] - u0) * kl, nv = (p[1] - v0) * kl, nw = (p[2] - w0) * kn;
+            track_at(0.5 * (double)(span - 1) * (1.0 - cos(node_angle(tid, J))), s_base, s_bt, nb, p);
+            double2 n[4];
+            corners(p[0], p[1], p[2], n);
 #pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const double ph = ((q & 1) ? -nu : nu) + ((q & 2) ? -nv : nv) + nw;
-                sincospi(2.0 * ph, &s_node[tid][q].y, &s_node[tid][q].x);
-            }
+            for (int q = 0; q < 4; q++) s_node[tid][q] = n[q];
         }
         __syncthreads();
-        double2 e[4];
+        double err = 0.0;
+        for (int t = tid; t < len && err <= kResampleTol; t += kAnalyse) {
+            double2 e[4];
+            corners(track[(size_t)t * 3], track[(size_t)t * 3 + 1], track[(size_t)t * 3 + 2], e);
+            const double th = angle_of((double)t, span);
+            for (int j = 0; j < J; j++) {
+                const double w = cardinal(th, node_angle(j, J), J);
 #pragma unroll
-        for (int q = 0; q < 4; q++) e[q] = own[q];
-        for (int j = 0; j < J; j++) {
-            const double w = cardinal(th, node_angle(j, J), J);
+                for (int q = 0; q < 4; q++) {
+                    e[q].x -= w * s_node[j][q].x;
+                    e[q].y -= w * s_node[j][q].y;
+                }
+            }
 #pragma unroll
             for (int q = 0; q < 4; q++) {
-                e[q].x -= w * s_node[j][q].x;
-                e[q].y -= w * s_node[j][q].y;
+                const double m = fmax(fabs(e[q].x), fabs(e[q].y));
+                // fmax passes over a NaN, so both parts are looked at
+                err = m <= kResampleTol && e[q].x == e[q].x && e[q].y == e[q].y ? fmax(err, m) : 1e9;
+                if (err > kResampleTol) break;
             }
-        }
-        double err = 0.0;
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const double m = fmax(fabs(e[q].x), fabs(e[q].y));
-            err = m <= kResampleTol ? fmax(err, m) : 1e9;  // NaN counts as a failure
-            if (err > kResampleTol) break;
         }
         if (block_max_d(err, s_red) <= kResampleTol) {
             found = J;
@@ -167,24 +178,24 @@ __global__ __launch_bounds__(kMaxLen) void analyse_kernel(const ResampleChunk* c
     if (tid == 0) nodes_out[blockIdx.x] = found;
 }
 
-// Weights of one (len, nodes) pair per workgroup, FP64 rounded to float, in
+// Weights of one (span, nodes) pair per workgroup, FP64 rounded to float, in
 // both orders: [t][j] for the degridder's interpolation, [j][t] behind it for
 // the gridder's sums.
 __global__ void weights_kernel(const ResamplePair* pairs, float* weights) {
     const ResamplePair p = pairs[blockIdx.x];
     float* tj = weights + p.offset;
-    float* jt = tj + (size_t)p.len * p.nodes;
-    for (int i = threadIdx.x; i < p.len * p.nodes; i += blockDim.x) {
+    float* jt = tj + (size_t)p.span * p.nodes;
+    for (int i = threadIdx.x; i < p.span * p.nodes; i += blockDim.x) {
         const int t = i / p.nodes, j = i - t * p.nodes;
-        const float w = (float)cardinal(angle_of((double)t, p.len), node_angle(j, p.nodes), p.nodes);
+        const float w = (float)cardinal(angle_of((double)t, p.span), node_angle(j, p.nodes), p.nodes);
         tj[i] = w;
-        jt[(size_t)j * p.len + t] = w;
+        jt[(size_t)j * p.span + t] = w;
     }
 }
 
 // Track rows of the resampled observation: the track at the nodes, or the
 // chunk's own rows where it is not resampled.
-__global__ __launch_bounds__(kMaxLen) void node_track_kernel(const ResampleChunk* chunks, const double* uvw, double* out) {
+__global__ __launch_bounds__(kAnalyse) void node_track_kernel(const ResampleChunk* chunks, const double* uvw, double* out) {
     __shared__ double s_base[kBase][3];
     __shared__ int s_bt[kBase];
     const ResampleChunk c = chunks[blockIdx.x];
@@ -202,7 +213,7 @@ __global__ __launch_bounds__(kMaxLen) void node_track_kernel(const ResampleChunk
     __syncthreads();
     if (tid < c.nodes) {
         double p[3];
-        track_at(0.5 * (double)(c.len - 1) * (1.0 - cos(node_angle(tid, c.nodes))), s_base, s_bt, nb, p);
+        track_at(0.5 * (double)(c.span - 1) * (1.0 - cos(node_angle(tid, c.nodes))), s_base, s_bt, nb, p);
         for (int k = 0; k < 3; k++) out[((size_t)c.dst + tid) * 3 + k] = p[k];
     }
 }
@@ -248,14 +259,14 @@ __device__ __forceinline__ void store4(float* row, int c, int width, rs_f32x4 v)
 // takes timestep 4 g + k from lane group g, so that a lane's four weights of a
 // node lie side by side in w[j][t].  sum: LDS of [SPLIT - 1][16][64] floats.
 template <int Q, int SPLIT>
-__device__ __forceinline__ void gather_chunk(const float* src, const float* w, float* dst, int len, int J, int width, int n,
-                                             int nc, int m, int g, int part, float* sum) {
+__device__ __forceinline__ void gather_chunk(const float* src, const float* w, float* dst, int len, int span, int J,
+                                             int width, int n, int nc, int m, int g, int part, float* sum) {
     rs_f32x4 acc[Q];
     const float* row[Q];
 #pragma unroll
     for (int q = 0; q < Q; q++) {
         acc[q] = (rs_f32x4){};
-        row[q] = w + (size_t)min(16 * q + m, J - 1) * len + 4 * g;
+        row[q] = w + (size_t)min(16 * q + m, J - 1) * span + 4 * g;
     }
     const int full = len & ~15;
     const float* in = src + (size_t)(4 * g) * width + nc;
@@ -289,20 +300,21 @@ __device__ __forceinline__ void gather_chunk(const float* src, const float* w, f
                 for (int q = 0; q < Q; q++)
                     acc[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[k], a[q][k], acc[q], 0, 0, 0);
         }
-    if (full < len && full / 16 % SPLIT == part) {
-        float b[4], a[4][Q];
+    if (full < len && full / 16 % SPLIT == part) {  // the weights' rows reach to span
+        float b[4];
+        rs_f32x4 a[Q];
 #pragma unroll
         for (int k = 0; k < 4; k++) {
-            const int t = full + 4 * g + k, tt = min(t, len - 1);
-            const float x = src[(size_t)tt * width + nc];
+            const int t = full + 4 * g + k;
+            const float x = src[(size_t)min(t, len - 1) * width + nc];
             b[k] = t < len ? x : 0.f;
-#pragma unroll
-            for (int q = 0; q < Q; q++) a[k][q] = row[q][tt - 4 * g];
         }
+#pragma unroll
+        for (int q = 0; q < Q; q++) a[q] = load4(row[q] + full);
 #pragma unroll
         for (int k = 0; k < 4; k++)
 #pragma unroll
-            for (int q = 0; q < Q; q++) acc[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[k], a[k][q], acc[q], 0, 0, 0);
+            for (int q = 0; q < Q; q++) acc[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[k], a[q][k], acc[q], 0, 0, 0);
     }
     if (SPLIT > 1) {
         const int lane = 16 * g + m;
@@ -347,12 +359,12 @@ __global__ __launch_bounds__(256) void gather_rows_kernel(const ResampleChunk* c
     float* dst = out + (size_t)c.dst * width;
     if (c.nodes == 0) return copy_rows(src, dst, c.len * width, lane, (unit - ci * ntiles) * SPLIT + part, ntiles * SPLIT);
     const int J = c.nodes, len = c.len, nc = col ? n : 0;
-    const float* w = weights + c.weights + (size_t)len * J;  // [j][t]
+    const float* w = weights + c.weights + (size_t)c.span * J;  // [j][t]
     switch ((J + 15) >> 4) {  // uniform
-        case 1: return gather_chunk<1, SPLIT>(src, w, dst, len, J, width, n, nc, m, g, part, s_sum);
-        case 2: return gather_chunk<2, SPLIT>(src, w, dst, len, J, width, n, nc, m, g, part, s_sum);
-        case 3: return gather_chunk<3, SPLIT>(src, w, dst, len, J, width, n, nc, m, g, part, s_sum);
-        default: return gather_chunk<4, SPLIT>(src, w, dst, len, J, width, n, nc, m, g, part, s_sum);
+        case 1: return gather_chunk<1, SPLIT>(src, w, dst, len, c.span, J, width, n, nc, m, g, part, s_sum);
+        case 2: return gather_chunk<2, SPLIT>(src, w, dst, len, c.span, J, width, n, nc, m, g, part, s_sum);
+        case 3: return gather_chunk<3, SPLIT>(src, w, dst, len, c.span, J, width, n, nc, m, g, part, s_sum);
+        default: return gather_chunk<4, SPLIT>(src, w, dst, len, c.span, J, width, n, nc, m, g, part, s_sum);
     }
 }
 
@@ -430,7 +442,7 @@ __global__ __launch_bounds__(256) void spread_rows_kernel(const ResampleChunk* c
 hipError_t launch_resample_analyse(const ResampleChunk* chunks, int nchunks, const double* uvw, double kl, double kn,
                                    int32_t* nodes, hipStream_t st) {
     if (nchunks <= 0) return hipSuccess;
-    hipLaunchKernelGGL(dev::analyse_kernel, dim3(nchunks), dim3(kResampleMaxLen), 0, st, chunks, uvw, kl, kn, nodes);
+    hipLaunchKernelGGL(dev::analyse_kernel, dim3(nchunks), dim3(dev::kAnalyse), 0, st, chunks, uvw, kl, kn, nodes);
     return hipGetLastError();
 }
 hipError_t launch_resample_tables(const ResamplePair* pairs, int npairs, float* weights, const ResampleChunk* chunks,
@@ -440,14 +452,14 @@ hipError_t launch_resample_tables(const ResamplePair* pairs, int npairs, float* 
         if (hipError_t e = hipGetLastError()) return e;
     }
     if (nchunks > 0)
-        hipLaunchKernelGGL(dev::node_track_kernel, dim3(nchunks), dim3(kResampleMaxLen), 0, st, chunks, uvw, out);
+        hipLaunchKernelGGL(dev::node_track_kernel, dim3(nchunks), dim3(dev::kAnalyse), 0, st, chunks, uvw, out);
     return hipGetLastError();
 }
 namespace {
-// (chunk, column tile) units; below kSplitUnits of them, a quarter of the waves
-// the chip holds, four waves share each in the gather: 1327 units 11.1 -> 9.5 us,
+// (chunk, column tile) units; below kSplitUnits of them, fewer waves than the
+// chip holds, four waves share each in the gather: 1327 units 11.1 -> 9.5 us,
 // but 3424 units 12.5 -> 13.8 and 10674 45 -> 55.
-constexpr int64_t kSplitUnits = 2048;
+constexpr int64_t kSplitUnits = 8192;
 int64_t row_units(const Resample& r, int C) { return (int64_t)r.nchunks * ((2 * C + 15) / 16); }
 }  // namespace
 hipError_t launch_resample_gather(const Resample& r, int C, const float2* vis, float2* out, hipStream_t st) {

@@ -83,9 +83,11 @@ struct SlotCorner {
 
 // Time resampling (kernels_resample.hip): `len` consecutive rows (timesteps x
 // C channels) of the observation from row `src` become `nodes` rows from row
-// `dst` of the resampled observation; nodes 0: the rows are copied.  weights:
-// float offset of the (len, nodes) pair's tables.
-constexpr int kResampleMaxLen = 256;
+// `dst` of the resampled observation; nodes 0: the rows are copied.  The nodes
+// are those of an interval of `span` >= len timesteps (a multiple of 16), so
+// that few weight tables serve all; weights: float offset of the (span, nodes)
+// pair's tables.
+constexpr int kResampleMaxLen = 512;
 constexpr int kResampleMaxNodes = 64;
 // Largest interpolation error of a unit phasor: below the rounding of the
 // FP32 weights and sums (6e-8).
@@ -94,11 +96,11 @@ constexpr double kResampleTol = 1e-8;
 constexpr double kResampleKeep = 0.7;
 struct ResampleChunk {
     int64_t src, weights;
-    int32_t dst, len, nodes, pad;
+    int32_t dst, len, nodes, span;
 };
 struct ResamplePair {
-    int64_t offset;  // [len][nodes], then [nodes][len]
-    int32_t len, nodes;
+    int64_t offset;  // [span][nodes], then [nodes][span]
+    int32_t span, nodes;
 };
 // The device tables of a plan's resampled observation.
 struct Resample {

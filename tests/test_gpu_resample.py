@@ -62,6 +62,17 @@ def test_resampled_rows_match_oracle(S, T, C, kernel):
     assert not np.array_equal(vis, direct.astype(np.complex64))  # the rows were resampled
 
 
+# the longest chunk (1024 timesteps) and one more, and a short wavelength whose
+# subgrids need more nodes than a whole chunk may have
+@pytest.mark.parametrize("S,T,C,f0", [(32, 1024, 2, 1e9), (32, 1050, 2, 1e9), (64, 700, 3, 3e9)])
+def test_long_chunks(S, T, C, f0):
+    ob = observation.custom(G=640, S=S, K=4, L=2, n_ant=6, T=T, C=C, f0=f0, f1=1.01 * f0, noise=0.1, seed=6)
+    layers, vis, ref_layers, ref_vis, direct = _both(ob, ob.partition(), ob.uvw, "fp32")
+    assert _rel(layers, ref_layers) <= TOL
+    assert _rel(vis, ref_vis) <= TOL
+    assert not np.array_equal(vis, direct.astype(np.complex64))
+
+
 @pytest.mark.parametrize("kernel", ["mfma_bf16", "mfma_fp16"])
 def test_resampled_rows_on_the_matrix_kernels(kernel):
     """From 2^18 visibilities the split-precision kernels work on resampled rows."""
