@@ -264,7 +264,10 @@ struct Descent {
 constexpr int kLdsTiles = 1024;
 constexpr int kResTiles = 38;  // 4 KB each
 constexpr Key kStalled = ~(Key)0;
-constexpr int kGatePolls = 1 << 19;  // a fraction of a second
+// Polls of the gate: a fraction of a second for the form that wants every CU's
+// LDS for itself, after which the other one is tried; that one waits longer, as
+// other programs' kernels may hold the CUs.
+constexpr int kGatePollsRes = 1 << 19, kGatePolls = 1 << 25;
 constexpr int kMaxPolls = 1 << 28;
 
 // The slots' tags before turn 0 (neither buffer holds its first turn) and the
@@ -287,9 +290,9 @@ __device__ __forceinline__ Key await_slot(const Key* slot, unsigned tag) {
 // Whether all workgroups of the launch are resident: the last to arrive opens
 // the gate, the first to lose patience shuts it, and the first verdict holds
 // for all.  Nothing has been changed before it.
-__device__ __forceinline__ bool all_resident(Key* gate, Key nwg) {
+__device__ __forceinline__ bool all_resident(Key* gate, Key nwg, int polls) {
     if (__hip_atomic_fetch_add(gate, (Key)1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 == nwg) atomicCAS(gate + 1, (Key)0, (Key)1);
-    for (int i = 0; i < kGatePolls; i++)
+    for (int i = 0; i < polls; i++)
         if (const Key v = poll(gate + 1)) return v == 1;
     const Key before = atomicCAS(gate + 1, (Key)0, (Key)2);
     return before == 1;
@@ -307,7 +310,7 @@ __global__ __launch_bounds__(kDescent) void descent_kernel(Descent a) {
     __shared__ int s_go;
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int H = a.H, W = a.W, OH = a.OH, OW = a.OW, me = blockIdx.x, nwg = OH * OW;
-    if (t == 0) s_go = all_resident(a.slots + 2 * kCopies * nwg, nwg);
+    if (t == 0) s_go = all_resident(a.slots + 2 * kCopies * nwg, nwg, RES ? kGatePollsRes : kGatePolls);
     const int ntx = (W + kTile - 1) / kTile, nty = (H + kTile - 1) / kTile;
     const int oy = me / OW, ox = me - oy * OW;
     const int nrow = (nty - oy + OH - 1) / OH, ncol = (ntx - ox + OW - 1) / OW, nlocal = nrow * ncol;
