@@ -248,7 +248,12 @@ int p9idg_capture_cycle(p9idg_plan* plan, int32_t grid_mode);
 int p9idg_launch_cycle(p9idg_plan* plan);
 int p9idg_download_residual(p9idg_plan* plan, void* out_c64);
 
-/* Device pointers of the plan's buffers (for zero-copy interop). */
+/* Device pointers of the plan's buffers (for zero-copy interop); NULL for those
+ * not wanted.  They stay valid for the plan's life (vis and model_vis: until an
+ * observation of another shape).  The caller may read and write them between any
+ * two calls, once the plan's work is done (p9idg_sync).  A plan whose grid
+ * pointer was handed out clears the whole grid in the PLAIN and WSUM modes, and
+ * looks for values outside the subgrids' bounding box before it images it. */
 int p9idg_device_buffers(p9idg_plan* plan, void** vis, void** grid, void** model_grid,
                          void** model_vis, void** image);
 /* Host copies of the plan's buffers. */

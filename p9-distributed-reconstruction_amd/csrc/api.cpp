@@ -111,6 +111,14 @@ struct p9idg_plan {
     // The footprints (per-layer bounding boxes of the subgrids, per mode)
     // live on the device.
     bool grid_clean = false, layers_clean = false, model_vis_clean = false;
+    // The caller holds the grid's / the model visibilities' pointer
+    // (p9idg_device_buffers) and may write through it between any two calls, so
+    // what an earlier call left there is not relied on.
+    bool grid_shared = false, model_vis_shared = false;
+    // whether such a grid holds anything outside the subgrids' box
+    // (launch_outside): two words that the checks use in turn
+    int32_t* d_wide = nullptr;
+    int32_t wide_turn = 0;
     int32_t grid_dirty_fp = -1, layers_dirty_fp = -1;
     Box* d_fp[3] = {nullptr, nullptr, nullptr};  // per grid mode
     int32_t n_fp[3] = {0, 0, 0};
@@ -474,12 +482,13 @@ void mark_gridded(p9idg_plan* p, int mode) {
 }
 
 // Brings the gridder target of `mode` to all-zero: the previous footprint
-// when the contents are known, the whole buffer otherwise (and always while
-// capturing, since a graph may be replayed after other work on the buffer).
+// when the contents are known, the whole buffer otherwise (a grid that the
+// caller may write, and always while capturing, since a graph may be replayed
+// after other work on the buffer).
 int zero_target(p9idg_plan* p, int mode, float2* target, size_t n) {
     bool& clean = mode == P9IDG_GRID_WSTACK ? p->layers_clean : p->grid_clean;
     int32_t& fp = mode == P9IDG_GRID_WSTACK ? p->layers_dirty_fp : p->grid_dirty_fp;
-    if (p->capturing || !clean) {
+    if (p->capturing || !clean || (mode != P9IDG_GRID_WSTACK && p->grid_shared)) {
         P9_HIP(launch_fill_zero(target, n, p->stream));
     } else if (fp >= 0) {
         P9_HIP(launch_zero_boxes(target, p->d_fp[fp], p->n_fp[fp], p->c.grid_size, p->stream));
@@ -973,14 +982,23 @@ int layers_image(p9idg_plan* p, double inv_n, int shift) {
 
 // Whether the buffer of `mode` is known to be zero outside that mode's boxes.
 bool footprint_known(const p9idg_plan* p, int mode) {
-    return p->n_fp[mode] > 0 && (mode == P9IDG_GRID_WSTACK ? p->layers_clean && p->layers_dirty_fp == mode
-                                                           : p->grid_clean && p->grid_dirty_fp == mode);
+    return mode == P9IDG_GRID_WSTACK ? p->layers_clean && p->layers_dirty_fp == mode
+                                     : p->grid_clean && p->grid_dirty_fp == mode;
+}
+
+int ensure_wide(p9idg_plan* p) {
+    if (p->d_wide) return P9IDG_OK;
+    if (int st = dev_alloc(&p->d_wide, (size_t)2)) return st;
+    P9_HIP(launch_reset_counter(p->d_wide, p->stream));
+    return P9IDG_OK;
 }
 
 // Inverse FFT of the grid buffer(s) and the image extraction: over the
 // subgrids' bounding box when it is known (kernels_fft.hip; the buffers are
-// left as they are), else over the whole grid.
-int do_grid_to_image(p9idg_plan* p, int mode) {
+// left as they are), else over the whole grid.  gridded: in one step with the
+// gridding; otherwise a caller that holds the grid's pointer may have written
+// anywhere in it since, and the device finds out.
+int do_grid_to_image(p9idg_plan* p, int mode, bool gridded = false) {
     if (int st = check_obs(p)) return st;
     DeviceGuard dg(p->device);
     const int G = p->c.grid_size;
@@ -989,15 +1007,24 @@ int do_grid_to_image(p9idg_plan* p, int mode) {
     if (int st_ = record(p, 5)) return st_;
     const bool wstack = mode == P9IDG_GRID_WSTACK;
     if (wstack && !p->d_layers) return fail(P9IDG_ERR_STATE, "no layers gridded");
-    if (p->have_line && mode >= P9IDG_GRID_PLAIN && mode <= P9IDG_GRID_WSUM && footprint_known(p, mode)) {
+    const bool shared = !wstack && p->grid_shared && !gridded;
+    if (p->have_line && mode >= P9IDG_GRID_PLAIN && mode <= P9IDG_GRID_WSUM && p->n_fp[mode] > 0 &&
+        (shared || footprint_known(p, mode))) {
         if (int st = ensure_line(p)) return st;
         const Box u = p->fp_union[mode];
+        int32_t* wide = nullptr;
+        if (shared) {
+            if (int st = ensure_wide(p)) return st;
+            wide = p->d_wide + (p->wide_turn & 1);
+            P9_HIP(launch_outside(p->d_grid, u, G, wide, p->d_wide + (~p->wide_turn & 1), p->stream));
+            p->wide_turn ^= 1;
+        }
         if (wstack) {
             if (int st = dev_alloc(&p->d_lsum, grid_elems(p))) return st;
             P9_HIP(launch_sum_boxes(p->d_layers, p->d_fp[mode], p->n_fp[mode], G, u, p->d_lsum, p->stream));
         }
-        P9_HIP(launch_line_image(wstack ? p->d_lsum : p->d_grid, wstack, u, p->line, p->d_line_tw, p->d_line_mid, inv_n,
-                                 p->d_image, p->stream));
+        P9_HIP(launch_line_image(wstack ? p->d_lsum : p->d_grid, wstack, u, wide, p->line, p->d_line_tw, p->d_line_mid,
+                                 inv_n, p->d_image, p->stream));
     } else if (wstack) {
         if (int st = layers_image(p, inv_n, 1)) return st;
     } else {
@@ -1051,7 +1078,7 @@ int cycle_step(p9idg_plan* p, int grid_mode) {
     int st = do_exec_grid(p, grid_mode);
     p->grid_src = src;
     if (st) return st;
-    return do_grid_to_image(p, grid_mode);
+    return do_grid_to_image(p, grid_mode, true);
 }
 
 void drop_graph(p9idg_plan* p) {
@@ -1255,6 +1282,7 @@ int p9idg_destroy(p9idg_plan* p) {
     dev_free(p->d_lsum);
     dev_free(p->d_line_tw);
     dev_free(p->d_line_mid);
+    dev_free(p->d_wide);
     dev_free(p->d_twiddle);
     dev_free(p->d_phasor);
     dev_free(p->d_rtab);
@@ -1689,7 +1717,7 @@ int p9idg_launch_cycle(p9idg_plan* p) {
         mark_gridded(p, p->cycle_mode);
     else
         p->grid_clean = false;
-    p->model_vis_clean = true;
+    p->model_vis_clean = !p->model_vis_shared;
     return P9IDG_OK;
 }
 
@@ -1803,10 +1831,16 @@ int p9idg_device_buffers(p9idg_plan* p, void** vis, void** grid, void** model_gr
                          void** model_vis, void** image) {
     if (int st = check_plan(p)) return st;
     if (vis) *vis = p->d_vis;
-    if (grid) *grid = p->d_grid;
-    mark_unknown(p);  // the caller may write the buffers
+    mark_unknown(p);  // the caller may write the buffers, now and later
+    if (grid) {
+        *grid = p->d_grid;
+        p->grid_shared = true;
+    }
     if (model_grid) *model_grid = p->d_model_grid;
-    if (model_vis) *model_vis = p->d_model_vis;
+    if (model_vis) {
+        *model_vis = p->d_model_vis;
+        p->model_vis_shared = true;
+    }
     if (image) *image = p->d_image;
     return P9IDG_OK;
 }
@@ -2088,7 +2122,7 @@ int batch_launch_groups(p9idg_batch* b, int what, bool zero) {
 void batch_mark(p9idg_batch* b, int what) {
     for (p9idg_plan* p : b->plans) {
         if (what & 1) mark_gridded(p, b->grid_mode);
-        if (what & 2) p->model_vis_clean = true;
+        if (what & 2) p->model_vis_clean = !p->model_vis_shared;
     }
 }
 

@@ -34,15 +34,39 @@ __global__ void sum_boxes_kernel(const float2* layers, const Box* boxes, int nbo
     }
 }
 
+// *wide: whether the quadrant-swapped grid holds anything outside u (storage
+// row blockIdx.x); *next, the following check's word, is cleared.  The grid of a
+// caller that writes into it from time to time is read once (75 MB at 3072^2)
+// instead of transformed over its whole width: gridding and image 2048^2 132 -> 83
+// us, 3072^2 243 -> 102 (the box alone, unchecked: 61 and 77).
+__global__ __launch_bounds__(kLine) void outside_kernel(const float2* grid, int G, Box u, int32_t* wide, int32_t* next) {
+    const int h = G / 2, f = blockIdx.x, v = f >= h ? f - h : f + h;
+    const bool row = v >= u.y0 && v < u.y1;
+    const float4* in = reinterpret_cast<const float4*>(grid + (size_t)f * G);  // G is even
+    bool any = false;
+    for (int i = threadIdx.x; i < h; i += kLine) {
+        const uint4 e = __builtin_bit_cast(uint4, in[i]);
+        const int c = 2 * i, x0 = c >= h ? c - h : c + h, x1 = c + 1 >= h ? c + 1 - h : c + 1 + h;
+        any |= !(row && x0 >= u.x0 && x0 < u.x1) && (e.x | e.y);
+        any |= !(row && x1 >= u.x0 && x1 < u.x1) && (e.z | e.w);
+    }
+    if (__syncthreads_or(any) && threadIdx.x == 0) *wide = 1;
+    if (f == 0 && threadIdx.x == 0) *next = 0;
+}
+__device__ __forceinline__ Box box_of(Box u, const int32_t* wide, int G) { return wide && *wide ? Box{0, 0, G, 0, G} : u; }
+
 // ToImage, columns: column u.x0 + c of the box (dense array, or the
-// quadrant-swapped grid) over v; mid[y][c] for every storage row y.
+// quadrant-swapped grid) over v; mid[y][c] for every storage row y.  wide: the
+// box is the whole grid where that word is set.
 template <int MAXN, int LINES>
-__global__ __launch_bounds__(kLine * LINES) void image_columns_kernel(const float2* src, bool dense, Box u,
+__global__ __launch_bounds__(kLine * LINES) void image_columns_kernel(const float2* src, bool dense, Box box, const int32_t* wide,
                                                                                    LinePlan plan, const float2* tw,
                                                                                    float2* mid) {
     __shared__ float2 s_line[LINES][line_slots(MAXN)];
     const int t = threadIdx.x % kLine, l = threadIdx.x / kLine, G = plan.n, h = G / 2;
+    const Box u = box_of(box, wide, G);
     const int w = u.x1 - u.x0, c = blockIdx.x * LINES + l;
+    if ((int)blockIdx.x * LINES >= w) return;  // whole workgroups
     float2* line = s_line[l];
     for (int f = t; f < G; f += kLine) {
         const int v = f >= h ? f - h : f + h;  // grid row of frequency f
@@ -65,10 +89,12 @@ __global__ __launch_bounds__(kLine * LINES) void image_columns_kernel(const floa
 // ToImage, rows: storage rows 2 b and 2 b + 1 over u; image rows scaled by
 // inv_n, quadrant-swapped.
 template <int MAXN>
-__global__ __launch_bounds__(kLine) void image_rows_kernel(const float2* mid, Box u, LinePlan plan,
+__global__ __launch_bounds__(kLine) void image_rows_kernel(const float2* mid, Box box, const int32_t* wide, LinePlan plan,
                                                                         const float2* tw, double inv_n, float* img) {
     __shared__ float2 line[line_slots(MAXN)];
-    const int t = threadIdx.x, G = plan.n, h = G / 2, w = u.x1 - u.x0;
+    const int t = threadIdx.x, G = plan.n, h = G / 2;
+    const Box u = box_of(box, wide, G);
+    const int w = u.x1 - u.x0;
     const int y0 = 2 * blockIdx.x, y1 = y0 + 1;  // G is even
     const float2* r0 = mid + (size_t)y0 * w;
     const float2* r1 = r0 + w;
@@ -175,15 +201,20 @@ hipError_t launch_sum_boxes(const float2* layers, const Box* boxes, int nboxes, 
     return hipGetLastError();
 }
 
-hipError_t launch_line_image(const float2* src, bool dense, Box u, const LinePlan& p, const float2* tw, float2* mid,
-                             double inv_n, float* img, hipStream_t st) {
+hipError_t launch_outside(const float2* grid, Box u, int G, int32_t* wide, int32_t* next, hipStream_t st) {
+    hipLaunchKernelGGL(dev::outside_kernel, dim3(G), dim3(dev::kLine), 0, st, grid, G, u, wide, next);
+    return hipGetLastError();
+}
+
+hipError_t launch_line_image(const float2* src, bool dense, Box u, const int32_t* wide, const LinePlan& p, const float2* tw,
+                             float2* mid, double inv_n, float* img, hipStream_t st) {
     constexpr int L = 2;
-    const int w = u.x1 - u.x0;
+    const int w = wide ? p.n : u.x1 - u.x0;
 #define P9_COLS(N)                                                                                                      \
     hipLaunchKernelGGL((dev::image_columns_kernel<N, L>), dim3((w + L - 1) / L), dim3(dev::kLine * L), 0, st, src, dense, u, \
-                       p, tw, mid)
+                       wide, p, tw, mid)
 #define P9_ROWS(N) \
-    hipLaunchKernelGGL((dev::image_rows_kernel<N>), dim3(p.n / 2), dim3(dev::kLine), 0, st, mid, u, p, tw, inv_n, img)
+    hipLaunchKernelGGL((dev::image_rows_kernel<N>), dim3(p.n / 2), dim3(dev::kLine), 0, st, mid, u, wide, p, tw, inv_n, img)
     P9_LINE(P9_COLS);
     if (hipError_t e = hipGetLastError()) return e;
     P9_LINE(P9_ROWS);

@@ -215,9 +215,13 @@ bool line_plan(int n, LinePlan& p, bool nine = false);  // nine: radix 9 too (FP
 // The w-layers summed over the union u of their boxes, dense.
 hipError_t launch_sum_boxes(const float2* layers, const Box* boxes, int nboxes, int G, Box u, float2* out, hipStream_t st);
 // Quadrant-swapped real image x inv_n of a grid that is zero outside u: src is
-// that box (dense) or the quadrant-swapped grid; mid: G x (u.x1 - u.x0).
-hipError_t launch_line_image(const float2* src, bool dense, Box u, const LinePlan& p, const float2* tw, float2* mid,
-                             double inv_n, float* img, hipStream_t st);
+// that box (dense) or the quadrant-swapped grid; mid: G x (u.x1 - u.x0), or G x G
+// with `wide`: where that word is set, the grid may hold values everywhere.
+hipError_t launch_line_image(const float2* src, bool dense, Box u, const int32_t* wide, const LinePlan& p, const float2* tw,
+                             float2* mid, double inv_n, float* img, hipStream_t st);
+// Sets *wide (0 before) if the quadrant-swapped grid holds anything outside u,
+// and *next to 0.
+hipError_t launch_outside(const float2* grid, Box u, int G, int32_t* wide, int32_t* next, hipStream_t st);
 // Forward transform of the quadrant-swapped image; mid: (G / 2 + 1) x G.
 hipError_t launch_line_grid(const float* img, const LinePlan& p, const float2* tw, float2* mid, float2* grid,
                             hipStream_t st);

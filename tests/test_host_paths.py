@@ -1,0 +1,29 @@
+"""The library's host code on a HIP runtime without a GPU (tests/fake): which
+kernels the calls launch, on which devices, and what happens when an allocation
+is refused."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+FAKE = os.path.join(HERE, "fake")
+ROCM = os.environ.get("ROCM", "/opt/rocm")
+
+
+@pytest.fixture(scope="module")
+def fake(tmp_path_factory):
+    out = str(tmp_path_factory.mktemp("fake") / "libfake_hip.so")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-fPIC", "-shared", "-w", "-D__HIP_PLATFORM_AMD__", "-I" + os.path.join(ROCM, "include"),
+                    "-o", out, os.path.join(FAKE, "fake_hip.cpp")], check=True)
+    return out
+
+
+def _run(fake, scenario):
+    r = subprocess.run([sys.executable, os.path.join(FAKE, "scenarios.py"), fake, scenario], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0 and r.stdout.strip().endswith("done"), r.stdout + r.stderr
+
+
+def test_held_grid_pointer(fake):
+    _run(fake, "held_grid_pointer")
