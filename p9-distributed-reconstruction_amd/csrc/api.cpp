@@ -568,6 +568,7 @@ int ensure_host_stage(p9idg_plan* p) {
 
 // complex64 device buffer -> complex128 host array
 int download_c128(p9idg_plan* p, const float2* src, double* dst, size_t n) {
+    DeviceGuard dg(p->device);  // the stage's events belong to it
     if (int st = ensure_host_stage(p)) return st;
     const size_t pieces = (n + kHostPiece - 1) / kHostPiece;
     auto copy = [&](size_t i) -> int {

@@ -45,8 +45,9 @@ T handle(int device) {
     fake().device_of[p] = device;
     return reinterpret_cast<T>(p);
 }
-hipError_t launch(const char* how, const void* f, dim3 g, dim3 b, void** args) {
+hipError_t launch(const char* how, const void* f, dim3 g, dim3 b, void** args, hipStream_t st) {
     Fake& k = fake();
+    if (k.device_of[st] != k.device) return hipErrorInvalidHandle;
     const std::string name = k.kernels.count(f) ? k.kernels[f] : "?";
     note(how + name + " " + shape(g, b));
     // a launch has fewer than 2^32 threads in each dimension
@@ -220,9 +221,9 @@ hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
 hipError_t hipGraphExecDestroy(hipGraphExec_t) { return hipSuccess; }
 
 // --- launches
-hipError_t hipLaunchKernel(const void* f, dim3 g, dim3 b, void** args, size_t, hipStream_t) { return launch("", f, g, b, args); }
-hipError_t hipLaunchCooperativeKernel(const void* f, dim3 g, dim3 b, void** args, unsigned, hipStream_t) {
-    return launch("cooperative ", f, g, b, args);
+hipError_t hipLaunchKernel(const void* f, dim3 g, dim3 b, void** args, size_t, hipStream_t st) { return launch("", f, g, b, args, st); }
+hipError_t hipLaunchCooperativeKernel(const void* f, dim3 g, dim3 b, void** args, unsigned, hipStream_t st) {
+    return launch("cooperative ", f, g, b, args, st);
 }
 
 // --- hipFFT

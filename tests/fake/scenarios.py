@@ -76,6 +76,29 @@ def held_grid_pointer():
     assert columns(lambda: p.exec_grid_to_image(p9idg.GRID_WSTACK))[0] < G // 2
 
 
+def other_device():
+    """Every call on a plan of device 1 while device 0 is the current one."""
+    ob, p = make(device=1, G=320, S=16, K=4)  # more than one piece of a host array
+    grid = np.zeros((320, 320), np.complex128)
+    image = np.zeros((320, 320), np.float32)
+    calls = [lambda: p.grid(ob.vis), lambda: p.gridw(ob.vis), p.grid_psf, lambda: p.degrid(grid), lambda: p.degridw(grid),
+             lambda: p.to_image(ob.vis), p.calculate_psf, lambda: p.gridw_to_image(ob.vis), lambda: p.image_to_vis(image),
+             lambda: p.upload_vis(ob.vis), p.set_psf_vis, p.exec_grid, p.exec_degrid, p.exec_grid_to_image, p.exec_image_to_grid,
+             lambda: p.exec_cycle(), lambda: p.capture_cycle(), p.launch_cycle, p.download_grid, p.download_model_vis,
+             p.download_image, p.timings]
+    for call in calls:
+        call()
+    batch = p9idg.Batch([p])
+    batch.exec(3)
+    batch.capture(3)
+    batch.launch()
+    p.set_deterministic(True)
+    p.grid(ob.vis)
+    current = ctypes.c_int(-1)
+    fake.hipGetDevice(ctypes.byref(current))
+    assert current.value == 0
+
+
 if __name__ == "__main__":
     globals()[sys.argv[2]]()
     print("done")

@@ -27,3 +27,7 @@ def _run(fake, scenario):
 
 def test_held_grid_pointer(fake):
     _run(fake, "held_grid_pointer")
+
+
+def test_calls_on_a_plan_of_another_device(fake):
+    _run(fake, "other_device")
