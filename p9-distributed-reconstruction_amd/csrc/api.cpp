@@ -342,8 +342,9 @@ bool want_resample(const p9idg_plan* p) {
 
 // Splits the subgrids' timesteps into chunks, measures which of them can be
 // resampled (a chunk that cannot as a whole is tried in halves) and, where that
-// pays, builds the resampled observation.  Called with the plan's stream idle
-// and the tracks' upload queued.
+// pays, builds the resampled observation.  Where its memory is refused the plan
+// works on the observation's own rows.  Called with the plan's stream idle and
+// the tracks' upload queued.
 int build_resample(p9idg_plan* p, int T, int C, const double* freq) {
     p->have_rs = p->resampled = false;
     std::vector<p9idg_subgrid> meta = p->direct.meta;
@@ -378,7 +379,7 @@ int build_resample(p9idg_plan* p, int T, int C, const double* freq) {
     std::vector<int32_t> nodes;
     for (int pass = 0; pass < 3 && !pending.empty(); pass++) {
         const size_t n = pending.size(), nodes_at = padded(n * sizeof(ResampleChunk));
-        if (int st = dev_reserve(p->d_rs_chunks, p->alloc_rs_chunks, nodes_at + n * sizeof(int32_t))) return st;
+        if (dev_reserve(p->d_rs_chunks, p->alloc_rs_chunks, nodes_at + n * sizeof(int32_t))) return P9IDG_OK;
         ResampleChunk* const d_chunks = reinterpret_cast<ResampleChunk*>(p->d_rs_chunks);
         int32_t* const d_nodes = reinterpret_cast<int32_t*>(p->d_rs_chunks + nodes_at);
         chunks.clear();
@@ -406,7 +407,7 @@ int build_resample(p9idg_plan* p, int T, int C, const double* freq) {
     int64_t kept = 0;
     for (const ResampleChunk& c : chunks) kept += c.nodes > 0 ? c.nodes : c.len;
     if ((double)kept > kResamplePays * (double)rows) return P9IDG_OK;
-    if (int st = dev_reserve(p->d_rs_chunks, p->alloc_rs_chunks, nc * sizeof(ResampleChunk))) return st;
+    if (dev_reserve(p->d_rs_chunks, p->alloc_rs_chunks, nc * sizeof(ResampleChunk))) return P9IDG_OK;
     p->rs.chunks = reinterpret_cast<ResampleChunk*>(p->d_rs_chunks);
     // rows in subgrid order, one weight table per (span, nodes) pair
     constexpr int kNodeSteps = kResampleMaxNodes / 4 + 1;
@@ -448,7 +449,7 @@ int build_resample(p9idg_plan* p, int T, int C, const double* freq) {
     const size_t at_pairs = place(pairs.size() * sizeof(ResamplePair)), at_weights = place(weights * sizeof(float)),
                  at_uvw = place((size_t)dst * 3 * sizeof(double)), at_vis = place((size_t)dst * C * sizeof(float2)),
                  at_meta = place(meta.size() * sizeof(p9idg_subgrid)), at_order = place(meta.size() * sizeof(int32_t));
-    if (int st = dev_reserve(p->d_rs_rows, p->alloc_rs_rows, end)) return st;
+    if (dev_reserve(p->d_rs_rows, p->alloc_rs_rows, end)) return P9IDG_OK;
     ResamplePair* const d_pairs = reinterpret_cast<ResamplePair*>(p->d_rs_rows + at_pairs);
     p->rs.weights = reinterpret_cast<float*>(p->d_rs_rows + at_weights);
     p->d_rs_uvw = reinterpret_cast<double*>(p->d_rs_rows + at_uvw);
@@ -507,18 +508,28 @@ int ensure_fft_one(p9idg_plan* p) {
 }
 
 // The line transforms' twiddles and buffer (allocated once: a recorded graph
-// may hold them).
-int ensure_line(p9idg_plan* p) {
-    if (p->d_line_tw && p->d_line_mid) return P9IDG_OK;
+// may hold them).  *ready: they exist; a refused allocation leaves the library's
+// transform, and so does a capture, in which nothing can be allocated.
+int ensure_line(p9idg_plan* p, bool* ready) {
+    *ready = p->have_line && p->d_line_tw && p->d_line_mid;
+    if (*ready || !p->have_line || p->capturing) return P9IDG_OK;
     const int G = p->c.grid_size;
     std::vector<float2> tw(G);
     for (int k = 0; k < G; k++) {
         const double a = 2.0 * M_PI * (double)k / (double)G;
         tw[k] = make_float2((float)std::cos(a), (float)std::sin(a));
     }
-    if (int st = dev_alloc(&p->d_line_mid, (size_t)G * G)) return st;
-    if (int st = dev_alloc(&p->d_line_tw, (size_t)G)) return st;
-    P9_HIP(hipMemcpy(p->d_line_tw, tw.data(), G * sizeof(float2), hipMemcpyHostToDevice));
+    float2* d_tw = nullptr;
+    if (dev_alloc(&d_tw, (size_t)G) || dev_alloc(&p->d_line_mid, (size_t)G * G)) {
+        dev_free(d_tw);
+        return P9IDG_OK;
+    }
+    if (hipError_t e = hipMemcpy(d_tw, tw.data(), G * sizeof(float2), hipMemcpyHostToDevice)) {
+        dev_free(d_tw);
+        return hip_fail(e, "line twiddles");
+    }
+    p->d_line_tw = d_tw;
+    *ready = true;
     return P9IDG_OK;
 }
 
@@ -553,23 +564,36 @@ int upload_c128(p9idg_plan* p, const double* src, float2* dst, size_t n) {
 constexpr size_t kHostPiece = 1 << 16, kHostSlots = 4;
 static_assert(sizeof(p9idg_plan::h_ev) / sizeof(hipEvent_t) == kHostSlots, "an event per piece");
 
-int ensure_host_stage(p9idg_plan* p) {
+// Whether the pieces exist.
+bool ensure_host_stage(p9idg_plan* p) {
     for (auto& ev : p->h_ev)
-        if (!ev) P9_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
-    if (p->h_stage) return P9IDG_OK;
+        if (!ev && hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess) {
+            ev = nullptr;
+            (void)hipGetLastError();
+            return false;
+        }
+    if (p->h_stage) return true;
     if (hipHostMalloc(reinterpret_cast<void**>(&p->h_stage), kHostSlots * kHostPiece * sizeof(float2), hipHostMallocDefault) !=
         hipSuccess) {
         p->h_stage = nullptr;
         (void)hipGetLastError();
-        return fail(P9IDG_ERR_ALLOC, "pinned host allocation failed");
     }
-    return P9IDG_OK;
+    return p->h_stage != nullptr;
 }
 
 // complex64 device buffer -> complex128 host array
 int download_c128(p9idg_plan* p, const float2* src, double* dst, size_t n) {
     DeviceGuard dg(p->device);  // the stage's events belong to it
-    if (int st = ensure_host_stage(p)) return st;
+    if (!ensure_host_stage(p)) {  // no pinned memory to be had: one pageable copy
+        std::vector<float2> all(n);
+        P9_HIP(hipMemcpyAsync(all.data(), src, n * sizeof(float2), hipMemcpyDeviceToHost, p->stream));
+        P9_HIP(hipStreamSynchronize(p->stream));
+        for (size_t j = 0; j < n; j++) {
+            dst[2 * j] = (double)all[j].x;
+            dst[2 * j + 1] = (double)all[j].y;
+        }
+        return P9IDG_OK;
+    }
     const size_t pieces = (n + kHostPiece - 1) / kHostPiece;
     auto copy = [&](size_t i) -> int {
         const size_t k = i % kHostSlots;
@@ -987,10 +1011,11 @@ bool footprint_known(const p9idg_plan* p, int mode) {
                                      : p->grid_clean && p->grid_dirty_fp == mode;
 }
 
-int ensure_wide(p9idg_plan* p) {
-    if (p->d_wide) return P9IDG_OK;
-    if (int st = dev_alloc(&p->d_wide, (size_t)2)) return st;
+int ensure_wide(p9idg_plan* p, bool* ready) {
+    *ready = p->d_wide != nullptr;
+    if (*ready || p->capturing || dev_alloc(&p->d_wide, (size_t)2)) return P9IDG_OK;
     P9_HIP(launch_reset_counter(p->d_wide, p->stream));
+    *ready = true;
     return P9IDG_OK;
 }
 
@@ -1009,13 +1034,16 @@ int do_grid_to_image(p9idg_plan* p, int mode, bool gridded = false) {
     const bool wstack = mode == P9IDG_GRID_WSTACK;
     if (wstack && !p->d_layers) return fail(P9IDG_ERR_STATE, "no layers gridded");
     const bool shared = !wstack && p->grid_shared && !gridded;
-    if (p->have_line && mode >= P9IDG_GRID_PLAIN && mode <= P9IDG_GRID_WSUM && p->n_fp[mode] > 0 &&
-        (shared || footprint_known(p, mode))) {
-        if (int st = ensure_line(p)) return st;
+    bool line = false;
+    if (mode >= P9IDG_GRID_PLAIN && mode <= P9IDG_GRID_WSUM && p->n_fp[mode] > 0 && (shared || footprint_known(p, mode))) {
+        if (int st = ensure_line(p, &line)) return st;
+        if (line && shared)
+            if (int st = ensure_wide(p, &line)) return st;
+    }
+    if (line) {
         const Box u = p->fp_union[mode];
         int32_t* wide = nullptr;
         if (shared) {
-            if (int st = ensure_wide(p)) return st;
             wide = p->d_wide + (p->wide_turn & 1);
             P9_HIP(launch_outside(p->d_grid, u, G, wide, p->d_wide + (~p->wide_turn & 1), p->stream));
             p->wide_turn ^= 1;
@@ -1045,8 +1073,10 @@ int do_grid_to_image(p9idg_plan* p, int mode, bool gridded = false) {
 int do_image_to_grid(p9idg_plan* p, bool library = false) {
     if (int st = check_obs(p)) return st;
     DeviceGuard dg(p->device);
-    if (p->have_line && !library) {
-        if (int st = ensure_line(p)) return st;
+    bool line = false;
+    if (!library)
+        if (int st = ensure_line(p, &line)) return st;
+    if (line) {
         if (int st = span_begin(p, P9IDG_STAGE_TO_UVW)) return st;
         P9_HIP(launch_line_grid(p->d_image, p->line, p->d_line_tw, p->d_line_mid, p->d_model_grid, p->stream));
         return span_end(p);

@@ -99,6 +99,75 @@ def other_device():
     assert current.value == 0
 
 
+def refused_memory():
+    """Refused memory that only the faster paths want: the resampled rows', the
+    line transforms', the pinned pieces'.  The calls work without it, a recorded
+    cycle too, and the resampled rows are back with the next observation."""
+    ob, p = make(nodes=8)  # resampled
+    part = ob.partition()
+    p.exec_grid()
+    assert "gather_rows_kernel" in launches(log())
+    p.close()
+    # the allocations around the analysis of the tracks, refused in turn
+    p = p9idg.Plan(ob.c)
+    log()
+    p.set_observation(ob.uvw, ob.freq, part)
+    p.exec_grid()
+    text = log()
+    p.close()
+    at = [i for i, x in enumerate(text) if x.startswith("analyse_kernel")][0]
+    before = [i for i in range(at) if text[i].startswith("malloc")]
+    after = [i for i in range(at, len(text)) if text[i].startswith("malloc")]
+    for i in (before[-1], after[0]):
+        size = int(text[i].split()[1])
+        q = p9idg.Plan(ob.c)
+        fake.fake_fail_allocations(size, size)
+        q.set_observation(ob.uvw, ob.freq, part)
+        q.exec_grid()
+        q.exec_degrid()
+        text2 = log()
+        assert "refused %d" % size in text2
+        names = launches(text2)
+        assert not set(names) & {"gather_rows_kernel", "spread_rows_kernel"} and "grid_fp32_queue_kernel" in names, names
+        fake.fake_fail_allocations(1, 0)
+        q.set_observation(ob.uvw, ob.freq, part)
+        log()
+        q.exec_grid()
+        assert "gather_rows_kernel" in launches(log())
+        q.close()
+    # the line transforms' buffer has the size of a complex grid: refused once the plan has its own
+    for cycle in (False, True):
+        q = p9idg.Plan(ob.c)
+        q.set_observation(ob.uvw, ob.freq, part)
+        q.exec_grid(p9idg.GRID_WSUM)
+        fake.fake_fail_allocations(160 * 160 * 8, 160 * 160 * 8)
+        log()
+        if cycle:
+            fake.fake_fail_allocations(160 * 160 * 8, 160 * 160 * 8)
+            q.capture_cycle(p9idg.GRID_WSUM)
+            text = log()
+            inside = text[text.index("begin capture"):text.index("end capture")]
+            assert not [x for x in inside if x.startswith(("malloc", "refused"))]
+        else:
+            q.exec_grid_to_image(p9idg.GRID_WSUM)
+            q.exec_image_to_grid()
+            text = log()
+        assert "hipfftExecC2C" in text and not [x for x in text if x.startswith("image_columns")]
+        fake.fake_fail_allocations(1, 0)
+        q.exec_grid(p9idg.GRID_WSUM)
+        log()
+        q.exec_grid_to_image(p9idg.GRID_WSUM)
+        assert "image_columns_kernel" in launches(log())
+        q.close()
+    fake.fake_fail_pinned(1)
+    with p9idg.Plan(ob.c) as q:
+        q.set_observation(ob.uvw, ob.freq, part)
+        model = np.arange(160 * 160, dtype=np.complex64).reshape(160, 160)
+        q.upload_model_grid(model)
+        assert q.grid(ob.vis).shape == (160, 160)
+        assert np.array_equal(q.download_model_grid(), model)
+
+
 if __name__ == "__main__":
     globals()[sys.argv[2]]()
     print("done")

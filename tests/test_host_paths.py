@@ -31,3 +31,7 @@ def test_held_grid_pointer(fake):
 
 def test_calls_on_a_plan_of_another_device(fake):
     _run(fake, "other_device")
+
+
+def test_refused_memory_of_the_faster_paths(fake):
+    _run(fake, "refused_memory")
