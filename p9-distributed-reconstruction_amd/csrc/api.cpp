@@ -369,7 +369,7 @@ int build_resample(p9idg_plan* p, int T, int C, const double* freq) {
         if (nt > 0) cut((int64_t)m.baseline_idx * T + m.time_sample_start, rows, nt, (nt + kResampleMaxLen - 1) / kResampleMaxLen);
         rows += std::max(nt, 0);
     }
-    if (rows * C < kResampleMinVis || rows > INT32_MAX) return P9IDG_OK;
+    if (rows * C < kResampleMinVis || rows > INT32_MAX || !resample_launches((int64_t)pending.size(), 1)) return P9IDG_OK;
     // corner pixel and highest wavenumber (Gridder.cs:163-174; n in double: an upper estimate suffices)
     double fmax = 0.0;
     for (int i = 0; i < C; i++) fmax = std::max(fmax, std::fabs(freq[i]));
@@ -406,7 +406,7 @@ int build_resample(p9idg_plan* p, int T, int C, const double* freq) {
     const size_t nc = chunks.size();
     int64_t kept = 0;
     for (const ResampleChunk& c : chunks) kept += c.nodes > 0 ? c.nodes : c.len;
-    if ((double)kept > kResamplePays * (double)rows) return P9IDG_OK;
+    if ((double)kept > kResamplePays * (double)rows || !resample_launches((int64_t)nc, C)) return P9IDG_OK;
     if (dev_reserve(p->d_rs_chunks, p->alloc_rs_chunks, nc * sizeof(ResampleChunk))) return P9IDG_OK;
     p->rs.chunks = reinterpret_cast<ResampleChunk*>(p->d_rs_chunks);
     // rows in subgrid order, one weight table per (span, nodes) pair

@@ -461,11 +461,12 @@ namespace {
 // 11.1 -> 9.5 us; with up to 512, split FP16 at subgrid 64 346 -> 340 us and
 // three uneven observations 634 -> 625.
 constexpr int64_t kSplitUnits = 8192;
-int64_t row_units(const Resample& r, int C) { return (int64_t)r.nchunks * ((2 * C + 15) / 16); }
+int64_t row_units(int64_t nchunks, int C) { return nchunks * ((2 * C + 15) / 16); }
 }  // namespace
+bool resample_launches(int64_t nchunks, int C) { return row_units(nchunks, C) <= (int64_t)(UINT32_MAX / 256); }
 hipError_t launch_resample_gather(const Resample& r, int C, const float2* vis, float2* out, hipStream_t st) {
     if (r.nchunks <= 0) return hipSuccess;
-    const int64_t units = row_units(r, C);
+    const int64_t units = row_units(r.nchunks, C);
     const bool split = units < kSplitUnits;
     hipLaunchKernelGGL(split ? dev::gather_rows_kernel<4> : dev::gather_rows_kernel<1>,
                        dim3((unsigned)(split ? units : (units + 3) / 4)), dim3(256), 0, st, r.chunks, r.nchunks,
@@ -475,7 +476,7 @@ hipError_t launch_resample_gather(const Resample& r, int C, const float2* vis, f
 }
 hipError_t launch_resample_spread(const Resample& r, int C, const float2* rows, float2* vis, hipStream_t st) {
     if (r.nchunks <= 0) return hipSuccess;
-    hipLaunchKernelGGL(dev::spread_rows_kernel, dim3((unsigned)row_units(r, C)), dim3(256), 0, st, r.chunks,
+    hipLaunchKernelGGL(dev::spread_rows_kernel, dim3((unsigned)row_units(r.nchunks, C)), dim3(256), 0, st, r.chunks,
                        (2 * C + 15) / 16, r.weights, 2 * C, reinterpret_cast<const float*>(rows),
                        reinterpret_cast<float*>(vis));
     return hipGetLastError();

@@ -195,6 +195,10 @@ hipError_t launch_zero_boxes(float2* base, const Box* boxes, int nboxes, int G, 
 hipError_t launch_gather_slots(const GatherBin* bins, int nbins, const GatherChunk* chunks, int nchunks,
                                const int32_t* slots, const SlotCorner* corners, const float2* scratch, int S, int G,
                                float2* partial, float2* base, hipStream_t st);
+// Whether launches over so many chunks of C channels (a workgroup for each 8
+// channels of a chunk at most) have fewer than 2^32 threads; short subgrids by
+// the million do not, and keep their own rows and the work queue.
+bool resample_launches(int64_t nchunks, int C);
 // nodes[i]: nodes that chunk i needs (0: not resampled).  kl, kn: highest
 // wavenumber / 2 pi times the corner pixel's l and n.
 hipError_t launch_resample_analyse(const ResampleChunk* chunks, int nchunks, const double* uvw, double kl, double kn,

@@ -27,6 +27,7 @@ struct Fake {
     // what analyse_kernel answers for every chunk, and how many of the next
     // deconvolver launches find their workgroups not all resident
     int nodes = 0, stalls = 0;
+    hipError_t last = hipSuccess;
     dim3 grid, block;
     size_t shmem = 0;
     hipStream_t stream = nullptr;
@@ -47,11 +48,11 @@ T handle(int device) {
 }
 hipError_t launch(const char* how, const void* f, dim3 g, dim3 b, void** args, hipStream_t st) {
     Fake& k = fake();
-    if (k.device_of[st] != k.device) return hipErrorInvalidHandle;
+    if (k.device_of[st] != k.device) return k.last = hipErrorInvalidHandle;
     const std::string name = k.kernels.count(f) ? k.kernels[f] : "?";
     note(how + name + " " + shape(g, b));
     // a launch has fewer than 2^32 threads in each dimension
-    if ((size_t)g.x * b.x > 0xFFFFFFFFull) return hipErrorInvalidConfiguration;
+    if ((size_t)g.x * b.x > 0xFFFFFFFFull) return k.last = hipErrorInvalidConfiguration;
     if (name.find("analyse_kernel") != std::string::npos) {
         int32_t* out = *static_cast<int32_t**>(args[4]);
         for (unsigned i = 0; i < g.x; i++) out[i] = k.nodes;
@@ -133,14 +134,18 @@ hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int* n, const void*, int
 }
 const char* hipGetErrorName(hipError_t) { return "hipError"; }
 const char* hipGetErrorString(hipError_t) { return "fake error"; }
-hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipGetLastError() {
+    const hipError_t e = fake().last;
+    fake().last = hipSuccess;
+    return e;
+}
 
 // --- memory
 hipError_t hipMalloc(void** p, size_t n) {
     Fake& f = fake();
     if (n >= f.fail_from && n <= f.fail_to) {
         note("refused " + std::to_string(n));
-        return hipErrorOutOfMemory;
+        return f.last = hipErrorOutOfMemory;
     }
     *p = std::calloc(n, 1);
     f.blocks[*p] = n;

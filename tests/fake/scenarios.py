@@ -168,6 +168,26 @@ def refused_memory():
         assert np.array_equal(q.download_model_grid(), model)
 
 
+def many_short_subgrids():
+    """Subgrids of 16 timesteps by the ten thousand with 4096 channels: a
+    workgroup per chunk and 8 channels would be more threads than a launch has,
+    so the plan keeps the observation's rows; a tenth of them is resampled."""
+    C = 4096
+    for B, resampled in ((1000, True), (35000, False)):
+        c = p9idg.GriddingConstants(B * 16 * C, 320, 32, 4, 16, 7e-6, 1, 0.0)
+        part = np.zeros(B, p9idg.SUBGRID_DTYPE)
+        part["baselineIdx"], part["timeSampleCount"] = np.arange(B), 16
+        part["UPixel"] = part["VPixel"] = 100
+        fake.fake_nodes(8)
+        p = p9idg.Plan(c)
+        p.set_observation(np.zeros((B, 16, 3)), np.linspace(1e9, 1.1e9, C), part)
+        p.exec_grid()
+        p.exec_degrid()
+        names = launches(log())
+        assert ("gather_rows_kernel" in names) == ("spread_rows_kernel" in names) == resampled
+        p.close()
+
+
 if __name__ == "__main__":
     globals()[sys.argv[2]]()
     print("done")

@@ -35,3 +35,7 @@ def test_calls_on_a_plan_of_another_device(fake):
 
 def test_refused_memory_of_the_faster_paths(fake):
     _run(fake, "refused_memory")
+
+
+def test_more_chunks_than_a_launch_has_threads(fake):
+    _run(fake, "many_short_subgrids")
