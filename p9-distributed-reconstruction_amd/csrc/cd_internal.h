@@ -37,10 +37,15 @@ struct DescentShape {
 };
 hipError_t descent_shape(int H, int W, int p2h, int p2w, DescentShape* shape);
 size_t descent_slots(const DescentShape& shape);  // words
-// Up to `limit` (> 0) iterations on x and g.  resident: with the gradients in
-// LDS where they fit, one workgroup per CU.  tiles: OH OW local words.
+// kResident: gradients in LDS, one workgroup per CU; kShared: gradients in
+// memory, beside other kernels' workgroups; kSingle: one workgroup, which waits
+// for nobody.
+enum DescentForm { kResident, kShared, kSingle };
+DescentForm descent_form(const DescentShape& shape);  // the fastest that fits
+// Up to `limit` (> 0) iterations on x and g.  tiles: max(OH OW local, all tiles)
+// words.
 hipError_t launch_descent(float* x, float* g, const float* amap, const float* psf2, int p2h, int p2w, int H, int W,
-                          const DescentShape& shape, bool resident, float lambda, float alpha, float epsilon, int limit,
+                          const DescentShape& shape, DescentForm form, float lambda, float alpha, float epsilon, int limit,
                           Key* slots, Key* tiles, State* state, hipStream_t st);
 
 // PaddedConvolver / CalcPaddedFourierCorrelation pieces (complex double

@@ -373,6 +373,8 @@ struct p9cd {
     float* d_amap = nullptr;
     float* d_psf2 = nullptr;
     cd::DescentShape shape;
+    cd::DescentForm form = cd::kResident;  // that the next call starts with
+    int fallbacks = 0;                     // calls since that is not the fastest
     cd::Key* d_tiles = nullptr;
     cd::Key* d_slots = nullptr;
     cd::State* d_state = nullptr;
@@ -384,6 +386,9 @@ struct p9cd {
 namespace {
 
 constexpr int kPerLaunch = 1 << 14;  // iterations of one launch: some 50 ms at most
+// Calls after which the fastest form is tried again: its gate's patience, half a
+// second at most, is then a small part of them.
+constexpr int kFallbackCalls = 64;
 
 int cd_abs_max(p9cd* c, const float* d_x, const float* d_g, float lambda, float alpha, float* out) {
     P9_HIP(cd::launch_tiles_all(d_x, d_g, c->d_amap, c->H, c->W, lambda, alpha, c->d_tiles, c->stream));
@@ -400,16 +405,18 @@ int cd_run(p9cd* c, float* d_x, float* d_g, float lambda, float alpha, int32_t m
     cd::State& s = *c->h_state;
     s = cd::State{};
     int32_t made = 0;
-    bool resident = true;
+    const cd::DescentForm fastest = cd::descent_form(c->shape);
+    if (c->form < fastest || (c->form > fastest && ++c->fallbacks > kFallbackCalls)) c->form = fastest;
     while (!s.done && made < max_iter) {
-        P9_HIP(cd::launch_descent(d_x, d_g, c->d_amap, c->d_psf2, c->p2h, c->p2w, c->H, c->W, c->shape, resident, lambda,
+        P9_HIP(cd::launch_descent(d_x, d_g, c->d_amap, c->d_psf2, c->p2h, c->p2w, c->H, c->W, c->shape, c->form, lambda,
                                   alpha, eps, std::min(max_iter - made, kPerLaunch), c->d_slots, c->d_tiles, c->d_state,
                                   c->stream));
         P9_HIP(hipMemcpyAsync(&s, c->d_state, sizeof(s), hipMemcpyDeviceToHost, c->stream));
         P9_HIP(hipStreamSynchronize(c->stream));
-        if (s.stalled == 1 && resident) {
-            // another program holds part of the CUs' LDS: the form that shares them
-            resident = false;
+        if (s.stalled == 1 && c->form != cd::kSingle) {
+            // other kernels hold the CUs, or their LDS: the form that needs less of them
+            c->form = c->form == cd::kResident ? cd::kShared : cd::kSingle;
+            c->fallbacks = 0;
             s = cd::State{};
             continue;
         }

@@ -265,8 +265,8 @@ constexpr int kLdsTiles = 1024;
 constexpr int kResTiles = 38;  // 4 KB each
 constexpr Key kStalled = ~(Key)0;
 // Polls of the gate: a fraction of a second for the form that wants every CU's
-// LDS for itself, after which the other one is tried; that one waits longer, as
-// other programs' kernels may hold the CUs.
+// LDS for itself, after which the one that shares the CUs is tried; that one waits
+// longer, as other programs' kernels may hold them, and gives way to one workgroup.
 constexpr int kGatePollsRes = 1 << 19, kGatePolls = 1 << 25;
 constexpr int kMaxPolls = 1 << 28;
 
@@ -527,17 +527,21 @@ hipError_t descent_shape(int H, int W, int p2h, int p2w, DescentShape* shape) {
     return hipSuccess;
 }
 
+DescentForm descent_form(const DescentShape& shape) { return shape.local <= kResTiles ? kResident : kShared; }
+
 size_t descent_slots(const DescentShape& shape) { return 2 * kCopies * (size_t)shape.OH * shape.OW + 2; }
 
 hipError_t launch_descent(float* x, float* g, const float* amap, const float* psf2, int p2h, int p2w, int H, int W,
-                          const DescentShape& shape, bool resident, float lambda, float alpha, float epsilon, int limit,
+                          const DescentShape& shape, DescentForm form, float lambda, float alpha, float epsilon, int limit,
                           Key* slots, Key* tiles, State* state, hipStream_t st) {
-    const int n = shape.OH * shape.OW, words = 2 * kCopies * n;
+    DescentShape sh = shape;
+    if (form == kSingle) sh = {1, 1, ((H + kTile - 1) / kTile) * ((W + kTile - 1) / kTile)};
+    const int n = sh.OH * sh.OW, words = 2 * kCopies * n;
     hipLaunchKernelGGL(reset_slots_kernel, dim3((words + 2 + kThreads - 1) / kThreads), dim3(kThreads), 0, st, slots, words);
     if (hipError_t e = hipGetLastError()) return e;
-    Descent a{x, g, amap, psf2, p2h, p2w, H, W, shape.OH, shape.OW, lambda, alpha, epsilon, limit, slots, tiles, shape.local, state};
+    Descent a{x, g, amap, psf2, p2h, p2w, H, W, sh.OH, sh.OW, lambda, alpha, epsilon, limit, slots, tiles, sh.local, state};
     void* args[] = {&a};
-    return hipLaunchCooperativeKernel(descent_of(shape.local, resident), dim3(n), dim3(kDescent), args, 0, st);
+    return hipLaunchCooperativeKernel(descent_of(sh.local, form == kResident), dim3(n), dim3(kDescent), args, 0, st);
 }
 
 hipError_t launch_amap(const double* scan, int ph, int pw, int H, int W, float* amap, hipStream_t st) {

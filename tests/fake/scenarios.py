@@ -188,6 +188,37 @@ def many_short_subgrids():
         p.close()
 
 
+def crowded_descent():
+    """The deconvolver while other kernels hold the CUs: the form that shares
+    them, then the one workgroup that waits for nobody; no form twice, and the
+    next calls start with the one that worked."""
+
+    def forms(stalls, cd, shape):
+        fake.fake_stalls(stalls)
+        log()
+        x, g = np.zeros(shape, np.float32), np.ones(shape, np.float32)
+        res = cd.Deconvolve(x, g, 0.1, 0.1, 5, 1e-6)
+        assert res.IterationCount == 1
+        # <LDS, RES> and the workgroups
+        return [(re.search(r"descent_kernelILb(\d)ELb(\d)", t).groups(), int(t.split()[-3]))
+                for t in fake.fake_log().decode().splitlines() if "descent_kernel" in t]
+
+    psf = np.ones((16, 16), np.float32)
+    shape = (320, 320)  # 100 tiles on 64 workgroups
+    cd = p9idg.FastSerialCD(shape, psf)
+    resident, shared, single = (("1", "1"), 64), (("1", "0"), 64), (("1", "0"), 1)
+    assert forms(0, cd, shape) == [resident]
+    assert forms(1, cd, shape) == [resident, shared]
+    assert forms(0, cd, shape) == [shared]
+    assert forms(1, cd, shape) == [shared, single]
+    assert [forms(0, cd, shape) for _ in range(64)] == [[single]] * 64
+    assert forms(0, cd, shape) == [resident]
+    assert forms(2, cd, shape) == [resident, shared, single]
+    shape = (256 * 32 * 39 + 5, 1)  # 40 tiles per workgroup: gradients not in LDS
+    cd = p9idg.FastSerialCD(shape, np.ones((4, 4), np.float32))
+    assert forms(1, cd, shape) == [(("1", "0"), 256), (("0", "0"), 1)]
+
+
 if __name__ == "__main__":
     globals()[sys.argv[2]]()
     print("done")

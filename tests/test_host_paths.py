@@ -39,3 +39,7 @@ def test_refused_memory_of_the_faster_paths(fake):
 
 def test_more_chunks_than_a_launch_has_threads(fake):
     _run(fake, "many_short_subgrids")
+
+
+def test_deconvolver_beside_other_kernels(fake):
+    _run(fake, "crowded_descent")
