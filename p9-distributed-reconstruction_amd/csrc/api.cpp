@@ -990,25 +990,33 @@ int do_exec_degrid(p9idg_plan* p, int mode, bool direct = false) {
     return P9IDG_OK;
 }
 
-// FFT.WStackIFFTFloat (FFT.cs:188-215): sum over layers of
-// (float)(Re(IFFT(layer)) / N).  The inverse FFT is linear and applies no
-// per-layer w-screen, so it runs once on the sum of the layers (identical up
-// to the per-layer float rounding).  The layers are left as they are.
-int layers_image(p9idg_plan* p, double inv_n, int shift) {
-    const int G = p->c.grid_size;
-    if (int st = dev_alloc(&p->d_lsum, grid_elems(p))) return st;
-    if (int st = ensure_fft_one(p)) return st;
-    P9_HIP(launch_sum_layers(p->d_layers, p->c.wlayer_count, grid_elems(p), p->d_lsum, p->stream));
-    P9_FFT(hipfftExecC2C(p->fft_one, reinterpret_cast<hipfftComplex*>(p->d_lsum),
-                         reinterpret_cast<hipfftComplex*>(p->d_lsum), HIPFFT_BACKWARD));
-    P9_HIP(launch_layers_to_image(p->d_lsum, 1, G, inv_n, shift, p->d_image, p->stream));
-    return P9IDG_OK;
-}
-
 // Whether the buffer of `mode` is known to be zero outside that mode's boxes.
 bool footprint_known(const p9idg_plan* p, int mode) {
     return mode == P9IDG_GRID_WSTACK ? p->layers_clean && p->layers_dirty_fp == mode
                                      : p->grid_clean && p->grid_dirty_fp == mode;
+}
+
+// FFT.WStackIFFTFloat (FFT.cs:188-215): sum over layers of
+// (float)(Re(IFFT(layer)) / N).  The inverse FFT is linear and applies no
+// per-layer w-screen, so it runs once on the sum of the layers (identical up
+// to the per-layer float rounding).  The layers are left as they are; when
+// their footprint is known only the union of the footprint boxes is summed
+// (3001^2, 32 layers: gridding and image 627 us, with all layers 1076).
+int layers_image(p9idg_plan* p, double inv_n, int shift) {
+    const int G = p->c.grid_size, W = P9IDG_GRID_WSTACK;
+    if (int st = dev_alloc(&p->d_lsum, grid_elems(p))) return st;
+    if (int st = ensure_fft_one(p)) return st;
+    if (footprint_known(p, W)) {
+        P9_HIP(launch_fill_zero(p->d_lsum, grid_elems(p), p->stream));
+        if (p->n_fp[W] > 0)
+            P9_HIP(launch_sum_layer_boxes(p->d_layers, p->d_fp[W], p->n_fp[W], G, p->fp_union[W], p->d_lsum, p->stream));
+    } else {
+        P9_HIP(launch_sum_layers(p->d_layers, p->c.wlayer_count, grid_elems(p), p->d_lsum, p->stream));
+    }
+    P9_FFT(hipfftExecC2C(p->fft_one, reinterpret_cast<hipfftComplex*>(p->d_lsum),
+                         reinterpret_cast<hipfftComplex*>(p->d_lsum), HIPFFT_BACKWARD));
+    P9_HIP(launch_layers_to_image(p->d_lsum, 1, G, inv_n, shift, p->d_image, p->stream));
+    return P9IDG_OK;
 }
 
 int ensure_wide(p9idg_plan* p, bool* ready) {

@@ -239,6 +239,8 @@ hipError_t launch_conv_spectrum(const float* psf, int rows, int cols, int yoff, 
 hipError_t launch_conv(const float* img, int rows, int cols, const LinePlan& p, const double2* tw, double2* mid,
                        const double2* spectrum, float* out, hipStream_t st);
 hipError_t launch_sum_layers(const float2* layers, int L, size_t GG, float2* out, hipStream_t st);
+hipError_t launch_sum_layer_boxes(const float2* layers, const Box* boxes, int nboxes, int G, Box u,
+                                  float2* out, hipStream_t st);
 hipError_t launch_scale_c64(float2* p, size_t n, double inv_norm, hipStream_t st);
 
 }  // namespace p9idg

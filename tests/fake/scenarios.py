@@ -219,6 +219,24 @@ def crowded_descent():
     assert forms(1, cd, shape) == [(("1", "0"), 256), (("0", "0"), 1)]
 
 
+def layer_sum_without_line_transform():
+    """A w-stacked image at a size without a line transform sums the layers over
+    the subgrids' boxes when they are known, in a recorded cycle too; layers that
+    came from elsewhere are summed as they are."""
+    ob, p = make(G=161)
+    p.exec_grid(p9idg.GRID_WSTACK)
+    log()
+    p.exec_grid_to_image(p9idg.GRID_WSTACK)
+    names = launches(log())
+    assert "sum_layer_boxes_kernel" in names and "sum_layers_kernel" not in names, names
+    p.capture_cycle(p9idg.GRID_WSTACK)
+    names = launches(log())
+    assert names.count("sum_layer_boxes_kernel") == 2 and "sum_layers_kernel" not in names
+    p9idg.FFT.WStackIFFTFloat(np.zeros((2, 161, 161), np.complex128), 1)
+    names = launches(log())
+    assert "sum_layers_kernel" in names and "sum_layer_boxes_kernel" not in names
+
+
 if __name__ == "__main__":
     globals()[sys.argv[2]]()
     print("done")

@@ -43,3 +43,7 @@ def test_more_chunks_than_a_launch_has_threads(fake):
 
 def test_deconvolver_beside_other_kernels(fake):
     _run(fake, "crowded_descent")
+
+
+def test_layer_sum_without_line_transform(fake):
+    _run(fake, "layer_sum_without_line_transform")
