@@ -160,8 +160,12 @@ int p9idg_set_deterministic(p9idg_plan* plan, int32_t on);
  * degrid_chunk visibilities of one subgrid (0 = whole subgrids), with
  * `workgroups` persistent workgroups in each direction (0 = CUs x
  * occupancy); queue == 0 launches one workgroup per subgrid.  Defaults:
- * 1, 2048, 2048, 0.  get_launch reports the gridder's workgroups (autotune
- * may pick another count for the degridder). */
+ * 1, 2048, 2048, 0; on time-resampled rows (p9idg_set_observation), whose
+ * subgrids are short, 0, 2048, 2048, 0.  set_launch sets the shape of both the
+ * launches on the observation's own rows and those on resampled rows; autotune
+ * sets that of the rows which the plan's device-resident launches use, and
+ * get_launch reports it (the gridder's workgroups: autotune may pick another
+ * count for the degridder). */
 int p9idg_set_launch(p9idg_plan* plan, int32_t queue, int32_t grid_chunk, int32_t degrid_chunk,
                      int32_t workgroups);
 int p9idg_get_launch(const p9idg_plan* plan, int32_t* queue, int32_t* grid_chunk,
@@ -173,7 +177,12 @@ int p9idg_get_launch(const p9idg_plan* plan, int32_t* queue, int32_t* grid_chunk
  * otherwise; keeps the fastest and returns its gridder / degridder kernel
  * times.  Overwrites the grid / layer and model visibility buffers. */
 int p9idg_autotune(p9idg_plan* plan, int32_t reps, float* grid_ms, float* degrid_ms);
-/* Uploads uvw, frequencies and the partition to HBM (once per observation). */
+/* Uploads uvw, frequencies and the partition to HBM (once per observation).
+ * From 2^14 visibilities (2^18 for the MFMA kernels) the plan grids and
+ * degrids a time-resampled observation where that leaves at most 0.6 of the
+ * rows: a few tenths of them are kept, with as much device memory more.  The
+ * calls that return complex doubles of visibilities (degrid, degridw,
+ * image_to_vis) evaluate every timestep. */
 int p9idg_set_observation(p9idg_plan* plan, const double* uvw, int32_t nr_baselines,
                           int32_t nr_timesteps, const double* freq, int32_t nr_channels,
                           const p9idg_subgrid* meta, int64_t nr_subgrids);

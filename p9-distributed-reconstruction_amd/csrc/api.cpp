@@ -91,9 +91,12 @@ struct p9idg_plan {
         WorkItem* d_items_grid = nullptr;
         WorkItem* d_items_degrid = nullptr;
         int32_t nitems_grid = 0, nitems_degrid = 0;
+        // launch shape (tunable): queue mode, visibilities per work item, the
+        // persistent workgroups of either direction (0: CUs x occupancy; the
+        // degridder's are half the size)
+        int32_t use_queue = 1, grid_chunk = 2048, degrid_chunk = 2048, workgroups = 0, workgroups_degrid = 0;
     } direct, rs_view;
     int32_t* d_counter = nullptr;
-    // launch shape (tunable): queue mode, visibilities per work item, workgroups
     // residual visibilities (vis - model_vis, 0 where flagged) and the
     // gridder's input selector
     float2* d_resid = nullptr;
@@ -129,12 +132,6 @@ struct p9idg_plan {
     bool have_line = false;
     float2* d_line_tw = nullptr;
     float2* d_line_mid = nullptr;
-    int32_t use_queue = 1;
-    bool launch_chosen = false;  // by p9idg_set_launch or p9idg_autotune
-    int32_t grid_chunk = 2048;
-    int32_t degrid_chunk = 2048;
-    int32_t workgroups = 0;         // gridder's persistent workgroups (0: CUs x occupancy)
-    int32_t workgroups_degrid = 0;  // the degridder's (its workgroups are half the size)
 
     // deterministic adder: each gridder work item writes its subgrid to a
     // scratch slot, then gather_slots sums the slots per grid tile in slot order
@@ -719,7 +716,7 @@ void free_gather(p9idg_plan::Gather& g) {
 }
 
 // The view that the plan's launches use.
-const p9idg_plan::View& active_view(const p9idg_plan* p) { return p->resampled ? p->rs_view : p->direct; }
+p9idg_plan::View& active_view(p9idg_plan* p) { return p->resampled ? p->rs_view : p->direct; }
 
 void free_items(p9idg_plan::View& v) {
     dev_free(v.d_items_grid);
@@ -746,29 +743,21 @@ int upload_items(p9idg_plan* p) {
     free_items(p->direct);
     free_items(p->rs_view);
     if (p->nsub == 0) return P9IDG_OK;
-    p9idg_plan::View& v = p->resampled ? p->rs_view : p->direct;
-    if (int st = upload_list(make_items(v.meta, v.order, p->C, p->grid_chunk), v.d_items_grid, v.nitems_grid, p->stream))
+    p9idg_plan::View& v = active_view(p);
+    if (int st = upload_list(make_items(v.meta, v.order, p->C, v.grid_chunk), v.d_items_grid, v.nitems_grid, p->stream))
         return st;
-    if (int st = upload_list(make_items(v.meta, v.order, p->C, p->degrid_chunk), v.d_items_degrid, v.nitems_degrid, p->stream))
+    if (int st = upload_list(make_items(v.meta, v.order, p->C, v.degrid_chunk), v.d_items_degrid, v.nitems_degrid, p->stream))
         return st;
     p9idg_plan::View& d = p->direct;
     if (p->resampled)
-        return upload_list(make_items(d.meta, d.order, p->C, p->degrid_chunk), d.d_items_degrid, d.nitems_degrid, p->stream);
+        return upload_list(make_items(d.meta, d.order, p->C, d.degrid_chunk), d.d_items_degrid, d.nitems_degrid, p->stream);
     return P9IDG_OK;
 }
 
-// Whether launches run persistent workgroups over the work queue.  A resampled
-// observation's subgrids are short (a few hundred rows at most), so unless the
-// caller has chosen a launch shape each is one workgroup that the hardware
-// dispatches: the queue's claims would be a tenth of its time.  Split BF16, grid /
-// degrid us with the queue -> without: 3072^2 207 / 195 -> 187 / 178, 512^2 106 /
-// 72 -> 69 / 65, 2048^2 68 / 49 -> 57 / 41.
-bool queue_on(const p9idg_plan* p) { return p->use_queue != 0 && (p->launch_chosen || !p->resampled); }
-
-LaunchCfg launch_cfg(const p9idg_plan* p, bool grid) {
+LaunchCfg launch_cfg(const p9idg_plan::View& v, bool grid) {
     LaunchCfg cfg;
-    cfg.queue = queue_on(p);
-    cfg.workgroups = grid ? p->workgroups : p->workgroups_degrid;
+    cfg.queue = v.use_queue != 0;
+    cfg.workgroups = grid ? v.workgroups : v.workgroups_degrid;
     return cfg;
 }
 
@@ -819,7 +808,7 @@ int prepare_gather(p9idg_plan* p, int mode) {
     const int S = p->c.subgrid_size, G = p->c.grid_size, L = p->c.wlayer_count;
     const p9idg_plan::View& v = active_view(p);
     const std::vector<WorkItem> items =
-        make_items(v.meta, v.order, p->C, queue_on(p) ? p->grid_chunk : 0);
+        make_items(v.meta, v.order, p->C, v.use_queue ? v.grid_chunk : 0);
     const size_t need = items.size() * (size_t)S * S;
     P9_HIP(hipStreamSynchronize(p->stream));  // queued launches may still use the old buffers
     if (p->alloc_scratch != need) {
@@ -936,10 +925,10 @@ int do_exec_grid(p9idg_plan* p, int mode) {
         P9_HIP(launch_resample_gather(p->rs, p->C, p->grid_src == P9IDG_SRC_RESIDUAL ? p->d_resid : p->d_vis, p->d_rs_vis,
                                       p->stream));
     if (p->kernel == P9IDG_KERNEL_FP32 || p->kernel == P9IDG_KERNEL_FP32_SEP)
-        e = launch_grid_fp32(a, p->c.subgrid_size, p->kernel == P9IDG_KERNEL_FP32_SEP, launch_cfg(p, true),
+        e = launch_grid_fp32(a, p->c.subgrid_size, p->kernel == P9IDG_KERNEL_FP32_SEP, launch_cfg(active_view(p), true),
                              p->stream);
     else
-        e = launch_grid_mfma(a, p->c.subgrid_size, p->kernel, launch_cfg(p, true), p->stream);
+        e = launch_grid_mfma(a, p->c.subgrid_size, p->kernel, launch_cfg(active_view(p), true), p->stream);
     if (e != hipSuccess) return hip_fail(e, "gridder launch");
     if (p->deterministic) {
         const p9idg_plan::Gather& gt = p->gather[mode];
@@ -978,10 +967,10 @@ int do_exec_degrid(p9idg_plan* p, int mode, bool direct = false) {
     if (int st_ = record(p, 3)) return st_;
     hipError_t e;
     if (p->kernel == P9IDG_KERNEL_FP32 || p->kernel == P9IDG_KERNEL_FP32_SEP)
-        e = launch_degrid_fp32(a, p->c.subgrid_size, p->kernel == P9IDG_KERNEL_FP32_SEP, launch_cfg(p, false),
+        e = launch_degrid_fp32(a, p->c.subgrid_size, p->kernel == P9IDG_KERNEL_FP32_SEP, launch_cfg(v, false),
                                p->stream);
     else
-        e = launch_degrid_mfma(a, p->c.subgrid_size, p->kernel, launch_cfg(p, false), p->stream);
+        e = launch_degrid_mfma(a, p->c.subgrid_size, p->kernel, launch_cfg(v, false), p->stream);
     if (e != hipSuccess) return hip_fail(e, "degridder launch");
     if (resampled) P9_HIP(launch_resample_spread(p->rs, p->C, p->d_rs_vis, p->d_model_vis, p->stream));
     if (int st = span_end(p)) return st;
@@ -1257,6 +1246,14 @@ int p9idg_create(const p9idg_constants* c, int32_t device, p9idg_plan** plan) {
         if (e != hipSuccess) return bail(hip_fail(e, "hipEventCreate"));
     }
     for (int i = 0; i < 8; i++) p->mark[i] = p->ev[i];
+    // A resampled observation's subgrids are short (a few hundred rows at most), so
+    // each is one workgroup that the hardware dispatches: the queue's claims would
+    // be a tenth of its time.  Split BF16, grid / degrid us with the queue ->
+    // without: 3072^2 207 / 195 -> 187 / 178, 512^2 106 / 72 -> 69 / 65, 2048^2 68 /
+    // 49 -> 57 / 41.  The observation's own rows run to thousands of visibilities
+    // per subgrid and keep the queue: degridw, 10 antennas x 1000 timesteps x 16
+    // channels, 2435 us without it, 886 with.
+    p->rs_view.use_queue = 0;
     const int S = c->subgrid_size, G = c->grid_size;
     p->have_line = line_plan(G, p->line);
     // tables: twiddles exp(+2 pi i m / S) and the adder phasor
@@ -1379,12 +1376,13 @@ int p9idg_set_launch(p9idg_plan* p, int32_t queue, int32_t grid_chunk, int32_t d
     if (int st = check_plan(p)) return st;
     if (grid_chunk < 0 || degrid_chunk < 0 || workgroups < 0)
         return fail(P9IDG_ERR_ARGUMENT, "negative launch parameter");
-    p->use_queue = queue != 0;
-    p->launch_chosen = true;
-    p->grid_chunk = grid_chunk;
-    p->degrid_chunk = degrid_chunk;
-    p->workgroups = workgroups;
-    p->workgroups_degrid = workgroups;
+    for (p9idg_plan::View* v : {&p->direct, &p->rs_view}) {
+        v->use_queue = queue != 0;
+        v->grid_chunk = grid_chunk;
+        v->degrid_chunk = degrid_chunk;
+        v->workgroups = workgroups;
+        v->workgroups_degrid = workgroups;
+    }
     if (p->have_obs) return upload_items(p);
     return P9IDG_OK;
 }
@@ -1392,10 +1390,11 @@ int p9idg_set_launch(p9idg_plan* p, int32_t queue, int32_t grid_chunk, int32_t d
 int p9idg_get_launch(const p9idg_plan* p, int32_t* queue, int32_t* grid_chunk,
                      int32_t* degrid_chunk, int32_t* workgroups) {
     if (int st = check_plan(p)) return st;
-    if (queue) *queue = p->use_queue;
-    if (grid_chunk) *grid_chunk = p->grid_chunk;
-    if (degrid_chunk) *degrid_chunk = p->degrid_chunk;
-    if (workgroups) *workgroups = p->workgroups;
+    const p9idg_plan::View& v = p->resampled ? p->rs_view : p->direct;
+    if (queue) *queue = v.use_queue;
+    if (grid_chunk) *grid_chunk = v.grid_chunk;
+    if (degrid_chunk) *degrid_chunk = v.degrid_chunk;
+    if (workgroups) *workgroups = v.workgroups;
     return P9IDG_OK;
 }
 
@@ -1798,17 +1797,15 @@ int p9idg_autotune(p9idg_plan* p, int32_t reps, float* grid_ms, float* degrid_ms
     for (int chunk : {512, 1024, 2048, 4096, 0})
         for (int wg : {0, cus, 2 * cus, 4 * cus}) cands.push_back({1, chunk, wg});
     float best[2] = {1e30f, 1e30f};
-    Cand pick[2] = {{p->use_queue, p->grid_chunk, p->workgroups},
-                    {p->use_queue, p->degrid_chunk, p->workgroups_degrid}};
-    const int32_t q0 = p->use_queue, g0 = p->grid_chunk, d0 = p->degrid_chunk, w0 = p->workgroups;
-    p->launch_chosen = true;
+    p9idg_plan::View& v = active_view(p);  // the launches that are timed
+    Cand pick[2] = {{v.use_queue, v.grid_chunk, v.workgroups}, {v.use_queue, v.degrid_chunk, v.workgroups_degrid}};
     bool warm = false;
     for (const Cand& c : cands) {
-        p->use_queue = c.queue;
-        p->grid_chunk = c.chunk;
-        p->degrid_chunk = c.chunk;
-        p->workgroups = c.wg;
-        p->workgroups_degrid = c.wg;
+        v.use_queue = c.queue;
+        v.grid_chunk = c.chunk;
+        v.degrid_chunk = c.chunk;
+        v.workgroups = c.wg;
+        v.workgroups_degrid = c.wg;
         if (int st = upload_items(p)) return st;
         // the first launches of a plan run on low clocks: not the first candidate's time
         for (int dir = 0; dir < 2 && !warm; dir++) {
@@ -1831,19 +1828,15 @@ int p9idg_autotune(p9idg_plan* p, int32_t reps, float* grid_ms, float* degrid_ms
             }
         }
     }
-    (void)q0;
-    (void)g0;
-    (void)d0;
-    (void)w0;
     // the queue flag is shared by both directions: take it from the direction
     // with the larger time, workgroups and chunks from each (with the queue
     // off they are unused)
     const int dom = best[0] >= best[1] ? 0 : 1;
-    p->use_queue = pick[dom].queue;
-    p->workgroups = pick[0].wg;
-    p->workgroups_degrid = pick[1].wg;
-    p->grid_chunk = pick[0].chunk;
-    p->degrid_chunk = pick[1].chunk;
+    v.use_queue = pick[dom].queue;
+    v.workgroups = pick[0].wg;
+    v.workgroups_degrid = pick[1].wg;
+    v.grid_chunk = pick[0].chunk;
+    v.degrid_chunk = pick[1].chunk;
     p->collect = collect;
     if (int st = upload_items(p)) return st;
     if (grid_ms) *grid_ms = best[0];
@@ -2265,8 +2258,8 @@ int p9idg_batch_prepare(p9idg_batch* b, int32_t grid_mode, int32_t degrid_mode) 
             p9idg_batch::Group g;
             g.S = p->c.subgrid_size;
             g.kernel = p->kernel;
-            g.workgroups = p->workgroups;
-            g.workgroups_degrid = p->workgroups_degrid;
+            g.workgroups = active_view(p).workgroups;
+            g.workgroups_degrid = active_view(p).workgroups_degrid;
             g.members.push_back(i);
             b->groups.push_back(g);
         }
@@ -2284,11 +2277,11 @@ int p9idg_batch_prepare(p9idg_batch* b, int32_t grid_mode, int32_t degrid_mode) 
             ag.push_back(a);
             KernelArgs d = make_args(p, degrid_mode, p->resampled);
             ad.push_back(d);
-            for (WorkItem w : make_items(v.meta, v.order, p->C, p->grid_chunk)) {
+            for (WorkItem w : make_items(v.meta, v.order, p->C, v.grid_chunk)) {
                 w.inst = m;
                 ig.push_back(w);
             }
-            for (WorkItem w : make_items(v.meta, v.order, p->C, p->degrid_chunk)) {
+            for (WorkItem w : make_items(v.meta, v.order, p->C, v.degrid_chunk)) {
                 w.inst = m;
                 id.push_back(w);
             }

@@ -237,6 +237,32 @@ def layer_sum_without_line_transform():
     assert "sum_layers_kernel" in names and "sum_layer_boxes_kernel" not in names
 
 
+def direct_launches_of_a_resampled_plan():
+    """The calls that degrid every timestep keep the work queue and its items
+    where the plan's own launches are one workgroup per resampled subgrid, after
+    an autotune of those as well; a chosen shape holds for both."""
+    ob, p = make(nodes=8)
+    grid, image = np.zeros((160, 160), np.complex128), np.zeros((160, 160), np.float32)
+    direct = (lambda: p.degrid(grid), lambda: p.degridw(grid), lambda: p.image_to_vis(image))
+
+    def degridder(call):
+        log()
+        call()
+        return [x for x in launches(log()) if x.startswith("degrid_fp32")]
+
+    for tuned in (False, True):
+        assert degridder(p.exec_degrid) == ["degrid_fp32_kernel"] and not p.get_launch()["queue"]
+        for call in direct:
+            assert degridder(call) == ["degrid_fp32_queue_kernel"]
+        p.autotune(1)  # every candidate takes as long here: the first, without a queue, is kept
+    p.set_launch(queue=False)
+    for call in direct + (p.exec_degrid,):
+        assert degridder(call) == ["degrid_fp32_kernel"]
+    p.set_launch(queue=True, degrid_chunk=128)
+    for call in direct + (p.exec_degrid,):
+        assert degridder(call) == ["degrid_fp32_queue_kernel"]
+
+
 if __name__ == "__main__":
     globals()[sys.argv[2]]()
     print("done")

@@ -47,3 +47,7 @@ def test_deconvolver_beside_other_kernels(fake):
 
 def test_layer_sum_without_line_transform(fake):
     _run(fake, "layer_sum_without_line_transform")
+
+
+def test_direct_launches_of_a_resampled_plan(fake):
+    _run(fake, "direct_launches_of_a_resampled_plan")
