@@ -180,9 +180,13 @@ int p9idg_autotune(p9idg_plan* plan, int32_t reps, float* grid_ms, float* degrid
 /* Uploads uvw, frequencies and the partition to HBM (once per observation).
  * From 2^14 visibilities (2^18 for the MFMA kernels) the plan grids and
  * degrids a time-resampled observation where that leaves at most 0.6 of the
- * rows: a few tenths of them are kept, with as much device memory more.  The
- * calls that return complex doubles of visibilities (degrid, degridw,
- * image_to_vis) evaluate every timestep. */
+ * rows: typically a tenth to a sixth of them, with as much device memory more
+ * for their visibilities and tracks and up to a few MB of tables.  The first
+ * such call on an observation builds it (0.1 to 0.9 ms, where one pass gains
+ * 0.05 to 1.5 ms), and the work items of a launch shape with a queue are listed
+ * by the first launch.  The calls that return complex doubles of visibilities
+ * (degrid, degridw, image_to_vis) evaluate every timestep and need neither
+ * rows nor memory for them. */
 int p9idg_set_observation(p9idg_plan* plan, const double* uvw, int32_t nr_baselines,
                           int32_t nr_timesteps, const double* freq, int32_t nr_channels,
                           const p9idg_subgrid* meta, int64_t nr_subgrids);

@@ -59,6 +59,7 @@ struct p9idg_plan {
     bool plain_adder_ok = true;  // every subgrid passes Adder.cs:30-31
     bool chan_uniform = false;   // wavenumbers equally spaced (to 1e-12 relative)
     int64_t gridded_vis = 0;
+    double max_freq = 0.0;  // largest |frequency|
 
     // device buffers
     double* d_uvw = nullptr;
@@ -140,7 +141,7 @@ struct p9idg_plan {
     size_t alloc_scratch = 0;  // float2 elements
     // Tile lists of each grid mode, kept side by side: building one mode's
     // lists never frees another's, which a captured graph may be using.
-    // They stay valid until the work items change (upload_items).
+    // They stay valid until the rows or the work items change (drop_lists).
     struct Gather {
         bool valid = false;
         GatherBin* d_bins = nullptr;
@@ -155,8 +156,10 @@ struct p9idg_plan {
     // index its rows (baseline 0, rows from time_sample_start), d_rs_uvw holds
     // its tracks and d_rs_vis its visibilities: the gridder's input, gathered
     // from the visibilities before each launch, or the degridder's output,
-    // spread to the timesteps after it.  have_rs: built for this observation;
-    // resampled: used by the plan's kernel (want_resample).
+    // spread to the timesteps after it.  Built by the first call that uses it
+    // (ensure_rows).  rs_tried: for this observation; have_rs: it paid and is there;
+    // resampled: the plan's launches use it.
+    bool rs_tried = false;
     bool have_rs = false;
     bool resampled = false;
     Resample rs;
@@ -317,35 +320,42 @@ int build_footprints(p9idg_plan* p, const p9idg_subgrid* meta, int64_t nsub) {
     return P9IDG_OK;
 }
 
+// The indices 0 .. n - 1 in ascending order of key(i) in [0, keys), equal keys in
+// their own order.
+template <typename Key>
+std::vector<int32_t> order_by(size_t n, size_t keys, Key key) {
+    std::vector<int32_t> start(keys + 1, 0), out(n);
+    for (size_t i = 0; i < n; i++) start[key(i) + 1]++;
+    for (size_t k = 0; k < keys; k++) start[k + 1] += start[k];
+    for (size_t i = 0; i < n; i++) out[start[key(i)]++] = (int32_t)i;
+    return out;
+}
+
 // A view's schedule (most rows first) and its arrays on the device.
 int upload_view(p9idg_plan* p, p9idg_plan::View& v) {
-    v.order.resize(v.meta.size());
-    std::iota(v.order.begin(), v.order.end(), 0);
-    std::stable_sort(v.order.begin(), v.order.end(), [&](int32_t a, int32_t b) {
-        return v.meta[a].time_sample_count > v.meta[b].time_sample_count;
-    });
+    int32_t most = 0;
+    for (const p9idg_subgrid& m : v.meta) most = std::max(most, m.time_sample_count);
+    v.order = order_by(v.meta.size(), (size_t)most + 1, [&](size_t i) { return (size_t)(most - v.meta[i].time_sample_count); });
     if (v.meta.empty()) return P9IDG_OK;
     P9_HIP(hipMemcpyAsync(v.d_meta, v.meta.data(), v.meta.size() * sizeof(p9idg_subgrid), hipMemcpyHostToDevice, p->stream));
     P9_HIP(hipMemcpyAsync(v.d_order, v.order.data(), v.order.size() * sizeof(int32_t), hipMemcpyHostToDevice, p->stream));
     return P9IDG_OK;
 }
 
-// Whether the plan's kernel works on the resampled rows.
+// Whether the plan's kernel works on resampled rows where they pay.
 bool want_resample(const p9idg_plan* p) {
-    return p->have_rs && (p->kernel == P9IDG_KERNEL_FP32 || p->kernel == P9IDG_KERNEL_FP32_SEP
-                              ? true
-                              : p->gridded_vis >= kResampleMinVisMfma);
+    const bool fp32 = p->kernel == P9IDG_KERNEL_FP32 || p->kernel == P9IDG_KERNEL_FP32_SEP;
+    return p->gridded_vis >= (fp32 ? kResampleMinVis : kResampleMinVisMfma);
 }
 
 // Splits the subgrids' timesteps into chunks, measures which of them can be
 // resampled (a chunk that cannot as a whole is tried in halves) and, where that
 // pays, builds the resampled observation.  Where its memory is refused the plan
-// works on the observation's own rows.  Called with the plan's stream idle and
-// the tracks' upload queued.
-int build_resample(p9idg_plan* p, int T, int C, const double* freq) {
-    p->have_rs = p->resampled = false;
+// works on the observation's own rows.  Nothing queued uses the arrays that it
+// fills (p9idg_set_observation waits for what did).
+int build_resample(p9idg_plan* p) {
     std::vector<p9idg_subgrid> meta = p->direct.meta;
-    const int S = p->c.subgrid_size;
+    const int S = p->c.subgrid_size, T = p->T, C = p->C;
     const float image_size = p->c.scale_arcsec * (float)p->c.grid_size;
     // a chunk and its place in the subgrids' order
     struct Piece {
@@ -366,10 +376,9 @@ int build_resample(p9idg_plan* p, int T, int C, const double* freq) {
         if (nt > 0) cut((int64_t)m.baseline_idx * T + m.time_sample_start, rows, nt, (nt + kResampleMaxLen - 1) / kResampleMaxLen);
         rows += std::max(nt, 0);
     }
-    if (rows * C < kResampleMinVis || rows > INT32_MAX || !resample_launches((int64_t)pending.size(), 1)) return P9IDG_OK;
+    if (rows > INT32_MAX || !resample_launches((int64_t)pending.size(), 1)) return P9IDG_OK;
     // corner pixel and highest wavenumber (Gridder.cs:163-174; n in double: an upper estimate suffices)
-    double fmax = 0.0;
-    for (int i = 0; i < C; i++) fmax = std::max(fmax, std::fabs(freq[i]));
+    const double fmax = p->max_freq;
     const double l = (0.5 * S - 0.5) * (double)image_size / S, t = 2.0 * l * l;
     const double kl = fmax / 299792458.0 * l, kn = fmax / 299792458.0 * (t < 1.0 ? t / (t + std::sqrt(1.0 - t)) : 1.0);
     std::vector<ResampleChunk> chunks;
@@ -388,6 +397,7 @@ int build_resample(p9idg_plan* p, int T, int C, const double* freq) {
         P9_HIP(hipStreamSynchronize(p->stream));
         std::vector<Piece> tried;
         tried.swap(pending);
+        const size_t before = done.size();
         for (size_t i = 0; i < n; i++) {
             Piece& x = tried[i];
             x.c.nodes = nodes[i];
@@ -396,8 +406,9 @@ int build_resample(p9idg_plan* p, int T, int C, const double* freq) {
             else
                 done.push_back(x);
         }
+        // each pass adds its chunks in the subgrids' order
+        std::inplace_merge(done.begin(), done.begin() + before, done.end(), [](const Piece& a, const Piece& b) { return a.at < b.at; });
     }
-    std::sort(done.begin(), done.end(), [](const Piece& a, const Piece& b) { return a.at < b.at; });
     chunks.clear();
     for (const Piece& x : done) chunks.push_back(x.c);
     const size_t nc = chunks.size();
@@ -433,10 +444,25 @@ int build_resample(p9idg_plan* p, int T, int C, const double* freq) {
         m.time_sample_start = row0;
         m.time_sample_count = dst - row0;
     }
-    // largest first, chunks of one table side by side
-    std::stable_sort(chunks.begin(), chunks.end(), [](const ResampleChunk& a, const ResampleChunk& b) {
-        return a.len * a.nodes != b.len * b.nodes ? a.len * a.nodes > b.len * b.nodes : a.weights < b.weights;
+    // largest first, chunks of one table side by side: the kinds that occur, then
+    // the chunks by kind
+    auto kind_of = [&](const ResampleChunk& c) { return (size_t)c.len * kNodeSteps + c.nodes / 4; };
+    std::vector<int32_t> rank((size_t)(kResampleMaxLen + 1) * kNodeSteps, -1);
+    std::vector<const ResampleChunk*> kinds;
+    for (const ResampleChunk& c : chunks)
+        if (rank[kind_of(c)] < 0) {
+            rank[kind_of(c)] = 0;
+            kinds.push_back(&c);
+        }
+    std::sort(kinds.begin(), kinds.end(), [](const ResampleChunk* a, const ResampleChunk* b) {
+        if (a->len * a->nodes != b->len * b->nodes) return a->len * a->nodes > b->len * b->nodes;
+        return a->weights != b->weights ? a->weights < b->weights : a->len > b->len;
     });
+    for (size_t k = 0; k < kinds.size(); k++) rank[kind_of(*kinds[k])] = (int32_t)k;
+    std::vector<ResampleChunk> sorted;
+    sorted.reserve(nc);
+    for (int32_t k : order_by(nc, kinds.size(), [&](size_t n) { return (size_t)rank[kind_of(chunks[n])]; })) sorted.push_back(chunks[k]);
+    chunks.swap(sorted);
     size_t end = 0;
     auto place = [&](size_t bytes) {
         const size_t at = end;
@@ -726,32 +752,60 @@ void free_items(p9idg_plan::View& v) {
 
 int upload_list(const std::vector<WorkItem>& items, WorkItem*& d, int32_t& n, hipStream_t st) {
     if (items.size() > (size_t)INT32_MAX) return fail(P9IDG_ERR_ARGUMENT, "too many work items");
-    if (int s = dev_alloc(&d, items.size())) return s;
-    P9_HIP(hipMemcpyAsync(d, items.data(), items.size() * sizeof(WorkItem), hipMemcpyHostToDevice, st));
-    P9_HIP(hipStreamSynchronize(st));
+    WorkItem* q = nullptr;
+    if (int s = dev_alloc(&q, items.size())) return s;
+    hipError_t e = hipMemcpyAsync(q, items.data(), items.size() * sizeof(WorkItem), hipMemcpyHostToDevice, st);
+    if (e == hipSuccess) e = hipStreamSynchronize(st);
+    if (e != hipSuccess) {
+        dev_free(q);
+        return hip_fail(e, "work items");
+    }
+    d = q;
     n = (int32_t)items.size();
     return P9IDG_OK;
 }
 
-// The active view's work items for the plan's launch shape, and the direct
-// degridder's (p9idg_degrid and the other calls that return double).
-int upload_items(p9idg_plan* p) {
+// Drops what depends on the rows in use.
+int drop_lists(p9idg_plan* p) {
     DeviceGuard dg(p->device);
     P9_HIP(hipStreamSynchronize(p->stream));  // queued launches may still read the old arrays
-    drop_graph(p);  // a captured step holds the old item arrays and tile lists
+    drop_graph(p);  // a captured step holds the item arrays and tile lists
     for (auto& g : p->gather) free_gather(g);
+    return P9IDG_OK;
+}
+
+// And what depends on the observation or the launch shape.
+int drop_items(p9idg_plan* p) {
+    DeviceGuard dg(p->device);
+    if (int st = drop_lists(p)) return st;
     free_items(p->direct);
     free_items(p->rs_view);
-    if (p->nsub == 0) return P9IDG_OK;
-    p9idg_plan::View& v = active_view(p);
-    if (int st = upload_list(make_items(v.meta, v.order, p->C, v.grid_chunk), v.d_items_grid, v.nitems_grid, p->stream))
-        return st;
-    if (int st = upload_list(make_items(v.meta, v.order, p->C, v.degrid_chunk), v.d_items_degrid, v.nitems_degrid, p->stream))
-        return st;
-    p9idg_plan::View& d = p->direct;
-    if (p->resampled)
-        return upload_list(make_items(d.meta, d.order, p->C, d.degrid_chunk), d.d_items_degrid, d.nitems_degrid, p->stream);
     return P9IDG_OK;
+}
+
+// A view's work items of one direction, if its launches read any.  Like
+// ensure_rows, made by the first call that needs them: a captured step has run
+// eagerly before.
+int ensure_items(p9idg_plan* p, p9idg_plan::View& v, bool grid) {
+    WorkItem*& d = grid ? v.d_items_grid : v.d_items_degrid;
+    if (!v.use_queue || d || p->nsub == 0) return P9IDG_OK;
+    return upload_list(make_items(v.meta, v.order, p->C, grid ? v.grid_chunk : v.degrid_chunk), d,
+                       grid ? v.nitems_grid : v.nitems_degrid, p->stream);
+}
+
+// Which rows the plan's launches use; builds the resampled ones for the first
+// call that does.  Plans that only degrid every timestep (p9idg_degridw,
+// p9idg_image_to_vis) never pay for them.
+int ensure_rows(p9idg_plan* p) {
+    if (p->capturing) return P9IDG_OK;
+    const bool want = want_resample(p);
+    if (want && !p->rs_tried) {
+        if (int st = build_resample(p)) return st;
+        p->rs_tried = true;
+    }
+    if (p->resampled == (want && p->have_rs)) return P9IDG_OK;
+    p->resampled = !p->resampled;
+    return drop_lists(p);
 }
 
 LaunchCfg launch_cfg(const p9idg_plan::View& v, bool grid) {
@@ -804,7 +858,7 @@ KernelArgs make_args(const p9idg_plan* p, int mode, bool resampled) {
 // mode frees nothing that a graph captured in another mode uses.
 int prepare_gather(p9idg_plan* p, int mode) {
     p9idg_plan::Gather& gt = p->gather[mode];
-    if (gt.valid) return P9IDG_OK;  // valid until the work items change (upload_items)
+    if (gt.valid) return P9IDG_OK;  // valid until the rows or the work items change (drop_lists)
     const int S = p->c.subgrid_size, G = p->c.grid_size, L = p->c.wlayer_count;
     const p9idg_plan::View& v = active_view(p);
     const std::vector<WorkItem> items =
@@ -906,10 +960,13 @@ int do_exec_grid(p9idg_plan* p, int mode) {
         target = p->d_layers;
         n *= (size_t)p->c.wlayer_count;
     }
+    if (int st = ensure_rows(p)) return st;
+    p9idg_plan::View& v = active_view(p);
+    if (int st = ensure_items(p, v, true)) return st;
     KernelArgs a = make_args(p, mode, p->resampled);
     a.grid = target;
-    a.items = active_view(p).d_items_grid;
-    a.nitems = active_view(p).nitems_grid;
+    a.items = v.d_items_grid;
+    a.nitems = v.nitems_grid;
     if (p->deterministic) {
         if (p->capturing && !p->gather[mode].valid)
             return fail(P9IDG_ERR_STATE, "deterministic adder not prepared for this mode before capture");
@@ -925,10 +982,10 @@ int do_exec_grid(p9idg_plan* p, int mode) {
         P9_HIP(launch_resample_gather(p->rs, p->C, p->grid_src == P9IDG_SRC_RESIDUAL ? p->d_resid : p->d_vis, p->d_rs_vis,
                                       p->stream));
     if (p->kernel == P9IDG_KERNEL_FP32 || p->kernel == P9IDG_KERNEL_FP32_SEP)
-        e = launch_grid_fp32(a, p->c.subgrid_size, p->kernel == P9IDG_KERNEL_FP32_SEP, launch_cfg(active_view(p), true),
+        e = launch_grid_fp32(a, p->c.subgrid_size, p->kernel == P9IDG_KERNEL_FP32_SEP, launch_cfg(v, true),
                              p->stream);
     else
-        e = launch_grid_mfma(a, p->c.subgrid_size, p->kernel, launch_cfg(active_view(p), true), p->stream);
+        e = launch_grid_mfma(a, p->c.subgrid_size, p->kernel, launch_cfg(v, true), p->stream);
     if (e != hipSuccess) return hip_fail(e, "gridder launch");
     if (p->deterministic) {
         const p9idg_plan::Gather& gt = p->gather[mode];
@@ -949,9 +1006,13 @@ int do_exec_degrid(p9idg_plan* p, int mode, bool direct = false) {
     if (mode != P9IDG_DEGRID_PLAIN && mode != P9IDG_DEGRID_WSTACK)
         return fail(P9IDG_ERR_ARGUMENT, "unknown degrid mode");
     DeviceGuard dg(p->device);
+    if (!direct)
+        if (int st = ensure_rows(p)) return st;
     const bool resampled = p->resampled && !direct;
+    p9idg_plan::View& v = resampled ? p->rs_view : p->direct;
+    const LaunchCfg cfg = launch_cfg(v, false);
+    if (int st = ensure_items(p, v, false)) return st;
     KernelArgs a = make_args(p, mode, resampled);
-    const p9idg_plan::View& v = resampled ? p->rs_view : p->direct;
     a.items = v.d_items_degrid;
     a.nitems = v.nitems_degrid;
     // Gridder.cs:96: uncovered timesteps stay 0; only the degridder writes
@@ -967,10 +1028,9 @@ int do_exec_degrid(p9idg_plan* p, int mode, bool direct = false) {
     if (int st_ = record(p, 3)) return st_;
     hipError_t e;
     if (p->kernel == P9IDG_KERNEL_FP32 || p->kernel == P9IDG_KERNEL_FP32_SEP)
-        e = launch_degrid_fp32(a, p->c.subgrid_size, p->kernel == P9IDG_KERNEL_FP32_SEP, launch_cfg(v, false),
-                               p->stream);
+        e = launch_degrid_fp32(a, p->c.subgrid_size, p->kernel == P9IDG_KERNEL_FP32_SEP, cfg, p->stream);
     else
-        e = launch_degrid_mfma(a, p->c.subgrid_size, p->kernel, launch_cfg(v, false), p->stream);
+        e = launch_degrid_mfma(a, p->c.subgrid_size, p->kernel, cfg, p->stream);
     if (e != hipSuccess) return hip_fail(e, "degridder launch");
     if (resampled) P9_HIP(launch_resample_spread(p->rs, p->C, p->d_rs_vis, p->d_model_vis, p->stream));
     if (int st = span_end(p)) return st;
@@ -1350,10 +1410,6 @@ int p9idg_set_kernel(p9idg_plan* p, int32_t kernel) {
         return fail(P9IDG_ERR_ARGUMENT, "unknown kernel");
     if (p->kernel != kernel) drop_graph(p);  // a captured step holds the old kernel
     p->kernel = kernel;
-    if (p->have_obs && p->resampled != want_resample(p)) {
-        p->resampled = !p->resampled;
-        return upload_items(p);
-    }
     return P9IDG_OK;
 }
 
@@ -1383,13 +1439,17 @@ int p9idg_set_launch(p9idg_plan* p, int32_t queue, int32_t grid_chunk, int32_t d
         v->workgroups = workgroups;
         v->workgroups_degrid = workgroups;
     }
-    if (p->have_obs) return upload_items(p);
+    if (p->have_obs) return drop_items(p);
     return P9IDG_OK;
 }
 
 int p9idg_get_launch(const p9idg_plan* p, int32_t* queue, int32_t* grid_chunk,
                      int32_t* degrid_chunk, int32_t* workgroups) {
     if (int st = check_plan(p)) return st;
+    if (p->have_obs) {
+        DeviceGuard dg(p->device);
+        if (int st = ensure_rows(const_cast<p9idg_plan*>(p))) return st;  // the plan's results stay the same
+    }
     const p9idg_plan::View& v = p->resampled ? p->rs_view : p->direct;
     if (queue) *queue = v.use_queue;
     if (grid_chunk) *grid_chunk = v.grid_chunk;
@@ -1473,7 +1533,6 @@ int p9idg_set_observation(p9idg_plan* p, const double* uvw, int32_t B, int32_t T
     P9_HIP(hipMemcpyAsync(p->d_wavenumbers, k.data(), C * sizeof(double), hipMemcpyHostToDevice, p->stream));
     p->direct.meta.assign(meta, meta + nsub);
     if (int st = upload_view(p, p->direct)) return st;
-    if (int st = build_resample(p, T, C, freq)) return st;
     P9_HIP(hipStreamSynchronize(p->stream));
     p->chan_uniform = uniform;
     p->B = B;
@@ -1482,10 +1541,12 @@ int p9idg_set_observation(p9idg_plan* p, const double* uvw, int32_t B, int32_t T
     p->nsub = nsub;
     p->plain_adder_ok = plain_ok;
     p->gridded_vis = gridded;
-    p->resampled = want_resample(p);
+    p->max_freq = 0.0;
+    for (int i = 0; i < C; i++) p->max_freq = std::max(p->max_freq, std::fabs(freq[i]));
+    p->rs_tried = p->have_rs = p->resampled = false;
     mark_unknown(p);
     if (int st = build_footprints(p, meta, nsub)) return st;
-    if (int st = upload_items(p)) return st;
+    if (int st = drop_items(p)) return st;
     p->have_obs = true;
     return P9IDG_OK;
 }
@@ -1797,6 +1858,7 @@ int p9idg_autotune(p9idg_plan* p, int32_t reps, float* grid_ms, float* degrid_ms
     for (int chunk : {512, 1024, 2048, 4096, 0})
         for (int wg : {0, cus, 2 * cus, 4 * cus}) cands.push_back({1, chunk, wg});
     float best[2] = {1e30f, 1e30f};
+    if (int st = ensure_rows(p)) return st;
     p9idg_plan::View& v = active_view(p);  // the launches that are timed
     Cand pick[2] = {{v.use_queue, v.grid_chunk, v.workgroups}, {v.use_queue, v.degrid_chunk, v.workgroups_degrid}};
     bool warm = false;
@@ -1806,7 +1868,7 @@ int p9idg_autotune(p9idg_plan* p, int32_t reps, float* grid_ms, float* degrid_ms
         v.degrid_chunk = c.chunk;
         v.workgroups = c.wg;
         v.workgroups_degrid = c.wg;
-        if (int st = upload_items(p)) return st;
+        if (int st = drop_items(p)) return st;
         // the first launches of a plan run on low clocks: not the first candidate's time
         for (int dir = 0; dir < 2 && !warm; dir++) {
             float ms = 0.f;
@@ -1838,7 +1900,7 @@ int p9idg_autotune(p9idg_plan* p, int32_t reps, float* grid_ms, float* degrid_ms
     v.grid_chunk = pick[0].chunk;
     v.degrid_chunk = pick[1].chunk;
     p->collect = collect;
-    if (int st = upload_items(p)) return st;
+    if (int st = drop_items(p)) return st;
     if (grid_ms) *grid_ms = best[0];
     if (degrid_ms) *degrid_ms = best[1];
     return P9IDG_OK;
@@ -2247,6 +2309,7 @@ int p9idg_batch_prepare(p9idg_batch* b, int32_t grid_mode, int32_t degrid_mode) 
         if (p->deterministic) return fail(P9IDG_ERR_UNSUPPORTED, "the deterministic adder is not available in batches");
         if (grid_mode == P9IDG_GRID_WSTACK)
             if (int st = ensure_layers(p)) return st;
+        if (int st = ensure_rows(p)) return st;
         P9_HIP(hipStreamSynchronize(p->stream));
         bool found = false;
         for (auto& g : b->groups)

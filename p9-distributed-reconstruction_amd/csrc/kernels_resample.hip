@@ -65,16 +65,39 @@ __device__ __forceinline__ int base_sample(int b, int nb, int len) {
     return min(max(s, b), len - nb + b);  // distinct: at least b from either end
 }
 
+// The chunk's base samples in LDS: the track there, the timesteps and the
+// Lagrange form's constant factors 1 / prod (t_b - t_q), which every node shares.
+// All threads of the workgroup.
+struct Base {
+    double track[kBase][3], t[kBase], inv[kBase];
+};
+__device__ __forceinline__ void load_base(Base& s, const double* track, int nb, int len) {
+    const int tid = threadIdx.x;
+    if (tid < nb) {
+        const int t = base_sample(tid, nb, len);
+        s.t[tid] = (double)t;
+        for (int k = 0; k < 3; k++) s.track[tid][k] = track[(size_t)t * 3 + k];
+    }
+    __syncthreads();
+    if (tid < nb) {
+        double p = 1.0;
+        for (int q = 0; q < nb; q++)
+            if (q != tid) p *= s.t[tid] - s.t[q];
+        s.inv[tid] = 1.0 / p;
+    }
+    __syncthreads();
+}
+
 // The track at time t from the nb base samples (Lagrange form, FP64).
-__device__ __forceinline__ void track_at(double t, const double (*base)[3], const int* bt, int nb, double out[3]) {
+__device__ __forceinline__ void track_at(double t, const Base& s, int nb, double out[3]) {
     out[0] = out[1] = out[2] = 0.0;
     for (int b = 0; b < nb; b++) {
-        double w = 1.0;
+        double w = s.inv[b];
         for (int q = 0; q < nb; q++)
-            if (q != b) w *= (t - (double)bt[q]) / (double)(bt[b] - bt[q]);
-        out[0] += w * base[b][0];
-        out[1] += w * base[b][1];
-        out[2] += w * base[b][2];
+            if (q != b) w *= t - s.t[q];
+        out[0] += w * s.track[b][0];
+        out[1] += w * s.track[b][1];
+        out[2] += w * s.track[b][2];
     }
 }
 
@@ -86,29 +109,33 @@ __device__ __forceinline__ double block_max_d(double v, double* red) {
     return fmax(fmax(red[0], red[1]), fmax(red[2], red[3]));
 }
 
-// One workgroup per chunk (thread t: timesteps t, t + 256, ...): the smallest
-// multiple of four nodes whose interpolant reproduces the corner phasors of
-// every timestep to kResampleTol, or 0.  kl, kn: highest wavenumber / 2 pi times
-// the corner pixel's l and n.
+// One workgroup per chunk (thread t: timesteps t, t + 256): a multiple of four
+// nodes whose interpolant reproduces the corner phasors of every timestep to
+// kResampleTol, or 0: the first that does from an estimate of the phase on.  kl,
+// kn: highest wavenumber / 2 pi times the corner pixel's l and n.
+//
+// The interpolant is evaluated in its barycentric form, with weights (-1)^j
+// sin(th_j) / (x - x_j), whose rounding cancels between numerator and denominator:
+// a division per timestep and node instead of four sines.  No timestep is a node:
+// the timesteps' x are rational, and the rational cosines 0 and 1 / 2 take J = 2 j +
+// 1 or 2 J = 3 (2 j + 1), but J is even (an accident of rounding would fail the
+// test, no more).  Headline tracks 1040 -> 232 us, 780 baselines x 500 timesteps
+// 203 -> 57, 276 x 300 77 -> 35.
 __global__ __launch_bounds__(kAnalyse) void analyse_kernel(const ResampleChunk* chunks, const double* uvw, double kl,
                                                            double kn, int32_t* nodes_out) {
     static_assert(kAnalyse == 256, "four waves reduce");
-    __shared__ double s_base[kBase][3];
-    __shared__ int s_bt[kBase];
+    constexpr int kPer = kResampleMaxLen / kAnalyse;
+    __shared__ Base s_base;
     __shared__ double2 s_node[kMaxNodes][4];
+    __shared__ double2 s_bary[kMaxNodes];  // x_j and (-1)^j sin(th_j)
     __shared__ double s_red[4];
     const ResampleChunk c = chunks[blockIdx.x];
     const int tid = threadIdx.x, len = c.len, span = c.span;
     const int nb = min(kBase, len);
     const double* track = uvw + (size_t)c.src * 3;
-    if (tid < nb) {
-        const int t = base_sample(tid, nb, len);
-        s_bt[tid] = t;
-        for (int k = 0; k < 3; k++) s_base[tid][k] = track[(size_t)t * 3 + k];
-    }
-    __syncthreads();
+    load_base(s_base, track, nb, len);
     // a timestep's corner phasors relative to the chunk's first sample; the largest phase in turns
-    const double u0 = s_base[0][0], v0 = s_base[0][1], w0 = s_base[0][2];
+    const double u0 = s_base.track[0][0], v0 = s_base.track[0][1], w0 = s_base.track[0][2];
     auto corners = [&](double u, double v, double w, double2* out) {
         const double du = (u - u0) * kl, dv = (v - v0) * kl, dw = (w - w0) * kn;
         double most = 0.0;
@@ -121,10 +148,13 @@ __global__ __launch_bounds__(kAnalyse) void analyse_kernel(const ResampleChunk* 
         // not finite: fails every test below
         return fabs(du) < 1e12 && fabs(dv) < 1e12 && fabs(dw) < 1e12 ? most : 1e9;
     };
-    double phase = 0.0;
-    for (int t = tid; t < len; t += kAnalyse) {
-        double2 own[4];
-        phase = fmax(phase, corners(track[(size_t)t * 3], track[(size_t)t * 3 + 1], track[(size_t)t * 3 + 2], own));
+    double2 own[kPer][4];
+    double x[kPer], phase = 0.0;
+#pragma unroll
+    for (int k = 0; k < kPer; k++) {
+        const int t = tid + k * kAnalyse;
+        if (t < len) phase = fmax(phase, corners(track[(size_t)t * 3], track[(size_t)t * 3 + 1], track[(size_t)t * 3 + 2], own[k]));
+        x[k] = 1.0 - 2.0 * (double)t / (double)(span - 1);
     }
     // start where the Chebyshev coefficients 2 (z / 2)^J / J! of exp(i z s) fall
     // below the tolerance for z of half the span from the first sample
@@ -141,8 +171,10 @@ __global__ __launch_bounds__(kAnalyse) void analyse_kernel(const ResampleChunk* 
     for (int J = (start + 3) & ~3; J <= limit; J += 4) {  // uniform
         __syncthreads();  // the previous candidate's nodes are read
         if (tid < J) {
-            double p[3];
-            track_at(0.5 * (double)(span - 1) * (1.0 - cos(node_angle(tid, J))), s_base, s_bt, nb, p);
+            double s, co, p[3];
+            sincos(node_angle(tid, J), &s, &co);
+            s_bary[tid] = make_double2(co, tid & 1 ? -s : s);
+            track_at(0.5 * (double)(span - 1) * (1.0 - co), s_base, nb, p);
             double2 n[4];
             corners(p[0], p[1], p[2], n);
 #pragma unroll
@@ -150,25 +182,31 @@ __global__ __launch_bounds__(kAnalyse) void analyse_kernel(const ResampleChunk* 
         }
         __syncthreads();
         double err = 0.0;
-        for (int t = tid; t < len && err <= kResampleTol; t += kAnalyse) {
-            double2 e[4];
-            corners(track[(size_t)t * 3], track[(size_t)t * 3 + 1], track[(size_t)t * 3 + 2], e);
-            const double th = angle_of((double)t, span);
+#pragma unroll
+        for (int k = 0; k < kPer; k++) {
+            if (tid + k * kAnalyse >= len) continue;
+            double den = 0.0;
+            double2 num[4] = {};
             for (int j = 0; j < J; j++) {
-                const double w = cardinal(th, node_angle(j, J), J);
+                const double2 b = s_bary[j];
+                const double w = b.y / (x[k] - b.x);
+                den += w;
 #pragma unroll
                 for (int q = 0; q < 4; q++) {
-                    e[q].x -= w * s_node[j][q].x;
-                    e[q].y -= w * s_node[j][q].y;
+                    num[q].x += w * s_node[j][q].x;
+                    num[q].y += w * s_node[j][q].y;
                 }
             }
+            const double inv = 1.0 / den;
 #pragma unroll
             for (int q = 0; q < 4; q++) {
-                const double m = fmax(fabs(e[q].x), fabs(e[q].y));
+                const double ex = own[k][q].x - num[q].x * inv, ey = own[k][q].y - num[q].y * inv;
+                const double m = fmax(fabs(ex), fabs(ey));
                 // fmax passes over a NaN, so both parts are looked at
-                err = m <= kResampleTol && e[q].x == e[q].x && e[q].y == e[q].y ? fmax(err, m) : 1e9;
+                err = m <= kResampleTol && ex == ex && ey == ey ? fmax(err, m) : 1e9;
                 if (err > kResampleTol) break;
             }
+            if (err > kResampleTol) break;
         }
         if (block_max_d(err, s_red) <= kResampleTol) {
             found = J;
@@ -178,14 +216,15 @@ __global__ __launch_bounds__(kAnalyse) void analyse_kernel(const ResampleChunk* 
     if (tid == 0) nodes_out[blockIdx.x] = found;
 }
 
-// Weights of one (span, nodes) pair per workgroup, FP64 rounded to float, in
-// both orders: [t][j] for the degridder's interpolation, [j][t] behind it for
+// Weights of one (span, nodes) pair per kWeightParts workgroups, FP64 rounded to
+// float, in both orders: [t][j] for the degridder's interpolation, [j][t] behind it for
 // the gridder's sums.
+constexpr int kWeightParts = 16;  // headline tracks: 150 us with one, 51
 __global__ void weights_kernel(const ResamplePair* pairs, float* weights) {
-    const ResamplePair p = pairs[blockIdx.x];
+    const ResamplePair p = pairs[blockIdx.x / kWeightParts];
     float* tj = weights + p.offset;
     float* jt = tj + (size_t)p.span * p.nodes;
-    for (int i = threadIdx.x; i < p.span * p.nodes; i += blockDim.x) {
+    for (int i = (blockIdx.x % kWeightParts) * blockDim.x + threadIdx.x; i < p.span * p.nodes; i += kWeightParts * blockDim.x) {
         const int t = i / p.nodes, j = i - t * p.nodes;
         const float w = (float)cardinal(angle_of((double)t, p.span), node_angle(j, p.nodes), p.nodes);
         tj[i] = w;
@@ -196,8 +235,7 @@ __global__ void weights_kernel(const ResamplePair* pairs, float* weights) {
 // Track rows of the resampled observation: the track at the nodes, or the
 // chunk's own rows where it is not resampled.
 __global__ __launch_bounds__(kAnalyse) void node_track_kernel(const ResampleChunk* chunks, const double* uvw, double* out) {
-    __shared__ double s_base[kBase][3];
-    __shared__ int s_bt[kBase];
+    __shared__ Base s_base;
     const ResampleChunk c = chunks[blockIdx.x];
     const int tid = threadIdx.x, nb = min(kBase, c.len);
     const double* track = uvw + (size_t)c.src * 3;
@@ -205,15 +243,10 @@ __global__ __launch_bounds__(kAnalyse) void node_track_kernel(const ResampleChun
         for (int i = tid; i < 3 * c.len; i += blockDim.x) out[(size_t)c.dst * 3 + i] = track[i];
         return;
     }
-    if (tid < nb) {
-        const int t = base_sample(tid, nb, c.len);
-        s_bt[tid] = t;
-        for (int k = 0; k < 3; k++) s_base[tid][k] = track[(size_t)t * 3 + k];
-    }
-    __syncthreads();
+    load_base(s_base, track, nb, c.len);
     if (tid < c.nodes) {
         double p[3];
-        track_at(0.5 * (double)(c.span - 1) * (1.0 - cos(node_angle(tid, c.nodes))), s_base, s_bt, nb, p);
+        track_at(0.5 * (double)(c.span - 1) * (1.0 - cos(node_angle(tid, c.nodes))), s_base, nb, p);
         for (int k = 0; k < 3; k++) out[((size_t)c.dst + tid) * 3 + k] = p[k];
     }
 }
@@ -448,7 +481,7 @@ hipError_t launch_resample_analyse(const ResampleChunk* chunks, int nchunks, con
 hipError_t launch_resample_tables(const ResamplePair* pairs, int npairs, float* weights, const ResampleChunk* chunks,
                                   int nchunks, const double* uvw, double* out, hipStream_t st) {
     if (npairs > 0) {
-        hipLaunchKernelGGL(dev::weights_kernel, dim3(npairs), dim3(256), 0, st, pairs, weights);
+        hipLaunchKernelGGL(dev::weights_kernel, dim3(npairs * dev::kWeightParts), dim3(256), 0, st, pairs, weights);
         if (hipError_t e = hipGetLastError()) return e;
     }
     if (nchunks > 0)

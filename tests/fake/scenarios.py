@@ -241,7 +241,7 @@ def direct_launches_of_a_resampled_plan():
     """The calls that degrid every timestep keep the work queue and its items
     where the plan's own launches are one workgroup per resampled subgrid, after
     an autotune of those as well; a chosen shape holds for both."""
-    ob, p = make(nodes=8)
+    ob, p = make(nodes=8, T=400)  # subgrids of more visibilities than an item holds
     grid, image = np.zeros((160, 160), np.complex128), np.zeros((160, 160), np.float32)
     direct = (lambda: p.degrid(grid), lambda: p.degridw(grid), lambda: p.image_to_vis(image))
 
@@ -261,6 +261,50 @@ def direct_launches_of_a_resampled_plan():
     p.set_launch(queue=True, degrid_chunk=128)
     for call in direct + (p.exec_degrid,):
         assert degridder(call) == ["degrid_fp32_queue_kernel"]
+
+
+def preparation():
+    """Setting an observation neither looks for resampled rows nor lists work
+    items: the calls that degrid every timestep never need the rows, the launches
+    without a queue no items, and what the others need is made once; a recorded
+    cycle allocates nothing, and kernels that work on the own rows below 2^18
+    visibilities do not ask for others."""
+    made = ("analyse_kernel", "weights_kernel", "node_track_kernel")
+    ob, p = make(nodes=8)
+    part = ob.partition()
+    assert 1 << 14 <= part.subgrids["timeSampleCount"].sum() * 8 < 1 << 18
+    grid, image = np.zeros((160, 160), np.complex128), np.zeros((160, 160), np.float32)
+
+    def rows(call):
+        log()
+        call()
+        text = log()
+        return [x for x in launches(text) if x in made], len([x for x in text if x.startswith("malloc")])
+
+    p.set_observation(ob.uvw, ob.freq, part)
+    for call in (lambda: p.set_observation(ob.uvw, ob.freq, part), lambda: p.degridw(grid), lambda: p.image_to_vis(image)):
+        assert rows(call)[0] == []
+    names, allocations = rows(lambda: p.exec_degrid())
+    assert names == list(made) and allocations == 2  # the chunks, the rows
+    for call in (p.exec_degrid, lambda: p.degridw(grid)):
+        assert rows(call) == ([], 0)
+    assert rows(p.exec_grid)[0] == []
+    for mode in (p9idg.GRID_WSTACK, p9idg.GRID_WSUM):
+        p.set_observation(ob.uvw, ob.freq, part)
+        log()
+        p.capture_cycle(mode)
+        text = log()
+        inside = text[text.index("begin capture"):]
+        assert not [x for x in inside if x.startswith("malloc")] and "gather_rows_kernel" in launches(inside)
+    p.set_observation(ob.uvw, ob.freq, part)
+    assert rows(lambda: p9idg.Batch([p]))[0] == list(made)
+    p.set_observation(ob.uvw, ob.freq, part)
+    assert rows(p.get_launch)[0] == list(made)
+    p.set_kernel("mfma_bf16")
+    p.set_observation(ob.uvw, ob.freq, part)
+    assert rows(p.exec_grid) == ([], 1) and rows(p.exec_grid) == ([], 0)  # the queue's items, once
+    p.set_kernel("fp32")
+    assert rows(p.exec_grid)[0] == list(made)
 
 
 if __name__ == "__main__":

@@ -51,3 +51,7 @@ def test_layer_sum_without_line_transform(fake):
 
 def test_direct_launches_of_a_resampled_plan(fake):
     _run(fake, "direct_launches_of_a_resampled_plan")
+
+
+def test_preparation_is_left_to_the_calls_that_need_it(fake):
+    _run(fake, "preparation")
