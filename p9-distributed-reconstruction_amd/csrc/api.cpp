@@ -97,6 +97,7 @@ struct p9idg_plan {
         // degridder's are half the size)
         int32_t use_queue = 1, grid_chunk = 2048, degrid_chunk = 2048, workgroups = 0, workgroups_degrid = 0;
     } direct, rs_view;
+    bool launch_chosen = false;  // by p9idg_set_launch
     int32_t* d_counter = nullptr;
     // residual visibilities (vis - model_vis, 0 where flagged) and the
     // gridder's input selector
@@ -808,6 +809,17 @@ int ensure_rows(p9idg_plan* p) {
     return drop_lists(p);
 }
 
+// Whether a call that degrids every timestep uses the work queue: not where it
+// would cut no subgrid, unless the caller chose the shape.  Degridder us, queue /
+// none: FP32 longest 480 visibilities 112 / 105, 1500 126 / 120, 16000 396 / 1920;
+// split BF16 480 28 / 21, 1500 54 / 40, 8000 91 / 103, 16000 55 / 172; the
+// separable FP32 form is the faster one on the queue (1600 239 / 286).
+bool direct_queue(const p9idg_plan* p) {
+    const p9idg_plan::View& v = p->direct;
+    if (!v.use_queue || p->launch_chosen || p->kernel == P9IDG_KERNEL_FP32_SEP || v.order.empty()) return v.use_queue != 0;
+    return (int64_t)v.meta[v.order[0]].time_sample_count * p->C > v.degrid_chunk;  // the longest comes first
+}
+
 LaunchCfg launch_cfg(const p9idg_plan::View& v, bool grid) {
     LaunchCfg cfg;
     cfg.queue = v.use_queue != 0;
@@ -1010,8 +1022,10 @@ int do_exec_degrid(p9idg_plan* p, int mode, bool direct = false) {
         if (int st = ensure_rows(p)) return st;
     const bool resampled = p->resampled && !direct;
     p9idg_plan::View& v = resampled ? p->rs_view : p->direct;
-    const LaunchCfg cfg = launch_cfg(v, false);
-    if (int st = ensure_items(p, v, false)) return st;
+    LaunchCfg cfg = launch_cfg(v, false);
+    if (direct) cfg.queue = direct_queue(p);
+    if (cfg.queue)
+        if (int st = ensure_items(p, v, false)) return st;
     KernelArgs a = make_args(p, mode, resampled);
     a.items = v.d_items_degrid;
     a.nitems = v.nitems_degrid;
@@ -1432,6 +1446,7 @@ int p9idg_set_launch(p9idg_plan* p, int32_t queue, int32_t grid_chunk, int32_t d
     if (int st = check_plan(p)) return st;
     if (grid_chunk < 0 || degrid_chunk < 0 || workgroups < 0)
         return fail(P9IDG_ERR_ARGUMENT, "negative launch parameter");
+    p->launch_chosen = true;
     for (p9idg_plan::View* v : {&p->direct, &p->rs_view}) {
         v->use_queue = queue != 0;
         v->grid_chunk = grid_chunk;

@@ -263,6 +263,22 @@ def direct_launches_of_a_resampled_plan():
         assert degridder(call) == ["degrid_fp32_queue_kernel"]
 
 
+def short_direct_launches():
+    """Where the queue would cut no subgrid the calls that degrid every timestep
+    launch a workgroup for each, except the separable FP32 form."""
+    image = np.zeros((160, 160), np.float32)
+    for kernel, T, kind in (("fp32", 256, "kernel"), ("fp32", 257, "queue_kernel"), ("mfma_bf16", 60, "kernel"), ("mfma_bf16", 300, "queue_kernel"),
+                            ("fp32_sep", 60, "queue_kernel")):
+        ob, p = make(kernel=kernel, T=T)  # 8 channels, items of 2048 visibilities
+        assert ob.partition().subgrids["timeSampleCount"].max() == T
+        p.image_to_vis(image)
+        names = [x for x in launches(log()) if x.startswith("degrid")]
+        assert names == ["degrid_%s_%s" % ("fp32" if "fp32" in kernel else "mfma", kind)], (names, kernel, T)
+        p.set_launch(queue=True)
+        p.image_to_vis(image)
+        assert "queue" in [x for x in launches(log()) if x.startswith("degrid")][0]
+
+
 def preparation():
     """Setting an observation neither looks for resampled rows nor lists work
     items: the calls that degrid every timestep never need the rows, the launches

@@ -55,3 +55,7 @@ def test_direct_launches_of_a_resampled_plan(fake):
 
 def test_preparation_is_left_to_the_calls_that_need_it(fake):
     _run(fake, "preparation")
+
+
+def test_short_direct_launches(fake):
+    _run(fake, "short_direct_launches")
