@@ -96,7 +96,8 @@ typedef enum p9idg_vis_type { P9IDG_C128 = 0, P9IDG_C64 = 1 } p9idg_vis_type;
 /* Phasor arithmetic of the gridder and degridder. */
 typedef enum p9idg_kernel {
     P9IDG_KERNEL_FP32 = 0,      /* per-pixel phasors on the FP32 vector ALUs */
-    P9IDG_KERNEL_MFMA_BF16 = 1, /* split hi/lo BF16 MFMA contraction, FP32 accumulate */
+    P9IDG_KERNEL_MFMA_BF16 = 1, /* split hi/lo BF16 MFMA contraction, FP32 accumulate
+                                   (a third part on time-resampled rows) */
     P9IDG_KERNEL_MFMA_FP16 = 2, /* split hi/lo FP16 MFMA contraction, FP32 accumulate */
     P9IDG_KERNEL_FP32_SEP = 3   /* the MFMA kernels' separable phasors (2 S per visibility)
                                    contracted with FP32 FMAs on the vector ALUs; gridder for

@@ -858,6 +858,7 @@ KernelArgs make_args(const p9idg_plan* p, int mode, bool resampled) {
     a.split_k[1] = 0xBF800000u;
     a.split_k[2] = 0x0000BC00u;
     a.counter = p->d_counter;
+    a.rows = resampled;
     return a;
 }
 
@@ -2194,12 +2195,13 @@ int batch_launch_group(p9idg_batch* b, p9idg_batch::Group& g, bool grid, bool ze
             P9_HIP(launch_fill_zero(p->d_model_vis, vis_elems(p), st));
         }
     }
+    const bool rows = std::find(g.resampled.begin(), g.resampled.end(), true) != g.resampled.end();
     if (grid) {
-        BatchArgs ba{g.d_args_grid, g.d_items_grid, g.n_grid, g.d_counter};
+        BatchArgs ba{g.d_args_grid, g.d_items_grid, g.n_grid, g.d_counter, rows};
         const hipError_t e = launch_grid_batch(ba, g.S, g.kernel, g.workgroups, st);
         return e == hipSuccess ? P9IDG_OK : hip_fail(e, "batched gridder launch");
     }
-    BatchArgs ba{g.d_args_degrid, g.d_items_degrid, g.n_degrid, g.d_counter};
+    BatchArgs ba{g.d_args_degrid, g.d_items_degrid, g.n_degrid, g.d_counter, rows};
     hipError_t e = launch_degrid_batch(ba, g.S, g.kernel, g.workgroups_degrid, st);
     for (size_t m = 0; m < g.members.size(); m++) {
         const p9idg_plan* p = b->plans[g.members[m]];

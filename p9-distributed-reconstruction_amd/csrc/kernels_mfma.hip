@@ -23,8 +23,8 @@
 // Phases are evaluated in FP64 (coefficients and per-entry phase), reduced to
 // [0, 1) turns and passed to the hardware sin/cos.  The GEMM operands of
 // the main terms are split x = hi + lo in BF16 (or FP16) and multiplied as
-// hi*hi + hi*lo + lo*hi with FP32 accumulation; the correction terms use the
-// hi parts only.  FP16 operands are normalised by powers of two (exact) per
+// hi*hi + hi*lo + lo*hi with FP32 accumulation (BF16 on time-resampled rows:
+// PrecBF16Rows); the correction terms use the hi parts only.  FP16 operands are normalised by powers of two (exact) per
 // subgrid so the low parts stay in FP16's normal range.
 #include "device_addsplit.h"
 
@@ -56,6 +56,8 @@ struct PrecBF16 {
     typedef __bf16 T;
     typedef bf16x8 V;
     static constexpr bool kNormalise = false;
+    static constexpr bool kThird = false;
+    static constexpr int kMid = 0;
     __device__ static __forceinline__ f32x16 mma(u32x4 a, u32x4 b, f32x16 c) {
         return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(V, a), __builtin_bit_cast(V, b), c, 0, 0, 0);
     }
@@ -71,17 +73,43 @@ struct PrecBF16 {
     __device__ static __forceinline__ HiLo split(float a, float b, SplitK k) {
         HiLo r;
         r.hi = pack(a, b);
-        const bf16x2 h = __builtin_bit_cast(bf16x2, r.hi);
-        const float la = __builtin_amdgcn_fdot2_f32_bf16(h, __builtin_bit_cast(bf16x2, k.bf16_lo), a, false);
-        const float lb = __builtin_amdgcn_fdot2_f32_bf16(h, __builtin_bit_cast(bf16x2, k.bf16_hi), b, false);
-        r.lo = pack(la, lb);
+        residual(r.hi, k, a, b);
+        r.lo = pack(a, b);
         return r;
     }
+    __device__ static __forceinline__ void residual(uint32_t part, SplitK k, float& a, float& b) {
+        const bf16x2 h = __builtin_bit_cast(bf16x2, part);
+        a = __builtin_amdgcn_fdot2_f32_bf16(h, __builtin_bit_cast(bf16x2, k.bf16_lo), a, false);
+        b = __builtin_amdgcn_fdot2_f32_bf16(h, __builtin_bit_cast(bf16x2, k.bf16_hi), b, false);
+    }
+};
+// Split BF16 on time-resampled rows.  A resampled row stands for some ten
+// timesteps, so a sum has a tenth of the terms to average the operands' rounding
+// (2^-18) and the missing lo * lo over, and the rounding grows threefold beside
+// everything else.  The gridder's operands therefore have a third part, with the
+// products lo * lo, hi * third and third * hi: 12 MFMAs more for each 16.  RMS
+// error of the image against 64 bits, own rows / resampled in two parts / in
+// three: headline 5.5e-7 / 5.4e-7 / 3.9e-7, 435 baselines x 600 x 8 every 2 s
+// 5.4e-7 / 7.4e-7 / 4.8e-7, 5 channels 3.9e-7 / 6.3e-7 / 3.1e-7; headline gridding
+// and image 223 -> 251 us, three uneven observations 600 -> 664.  The degridder's pixels have a third part (4 MFMAs
+// more): their rounding is the same for all rows of a subgrid, so it is what an
+// image of residuals shows most.  Visibilities 3.9e-6 -> 3.0e-6, image of the
+// residuals at 2048^2 1.23e-5 (own rows 1.18e-5) -> 4.9e-6; headline prediction
+// 276 -> 281 us.
+struct PrecBF16Rows : PrecBF16 {
+    static constexpr bool kThird = true;
+    // The channel of 8 from which the gridders step their phasors both ways.  A
+    // step multiplies the rounding of the channel-step phasor once more: from the
+    // first channel the last has seven of it, from here four at most (headline
+    // image in two parts 5.4e-7 -> 4.8e-7, in the same time).
+    static constexpr int kMid = 3;
 };
 struct PrecF16 {
     typedef _Float16 T;
     typedef f16x8 V;
     static constexpr bool kNormalise = true;
+    static constexpr bool kThird = false;
+    static constexpr int kMid = 0;
     __device__ static __forceinline__ f32x16 mma(u32x4 a, u32x4 b, f32x16 c) {
         return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(V, a), __builtin_bit_cast(V, b), c, 0, 0, 0);
     }
@@ -111,6 +139,20 @@ struct PrecF16 {
         const HiLo s_ = P::split((a), (b), (K)); \
         EH = s_.hi;                              \
         EL = s_.lo;                              \
+    } while (0)
+// And the third part into E3 (not set where the operands have two).
+#define P9_SPLIT3(P, K, a, b, EH, EL, E3)               \
+    do {                                                \
+        if constexpr (P::kThird) {                      \
+            float a_ = (a), b_ = (b);                   \
+            EH = P::pack(a_, b_);                       \
+            P::residual(EH, (K), a_, b_);               \
+            EL = P::pack(a_, b_);                       \
+            P::residual(EL, (K), a_, b_);               \
+            E3 = P::pack(a_, b_);                       \
+        } else {                                        \
+            P9_SPLIT2(P, K, a, b, EH, EL);              \
+        }                                               \
     } while (0)
 // Negates both 16-bit values of every dword (sign bits).
 __device__ __forceinline__ u32x4 neg(u32x4 v) { return v ^ (u32x4){0x80008000u, 0x80008000u, 0x80008000u, 0x80008000u}; }
@@ -256,18 +298,29 @@ __device__ __forceinline__ void grid_mfma_body(const KernelArgs& a, int sidx, in
         if (j0 + ROUND < K) fetch(j0 + ROUND);
         const int nsteps = (min(ROUND, K - j0) + 15) / 16;
         for (int st = kpart; st < nsteps; st += WPK) {
-            u32x4 Lrh, Lrl, Lih, Lil, cLr, cLi, Arh, Arl, Aih, Ail;
+            u32x4 Lrh, Lrl, Lih, Lil, cLr, cLi, Arh, Arl, Aih, Ail, Lr3, Li3, Ar3, Ai3;
             const int jg = st * 16 + grp * 8;  // this lane group's 8 visibilities
             if (chan_rec) {
-                // one timestep's 8 channels: phasors at the first channel times
-                // the channel-step phasor (FP64 phases, FP32 products)
-                const double ca = s_a[jg], cb = s_b[jg], cc = s_c[jg];
-                const double da = s_a[jg + 1] - ca, db = s_b[jg + 1] - cb, dc = s_c[jg + 1] - cc;
-                float2 A = cis_f64(fma(ca, lcol, cc * ncol));
-                float2 B = cis_f64(fma(cb, lrow, cc * nrow));
+                // one timestep's 8 channels: phasors at a middle channel times
+                // powers of the channel-step phasor (FP64 phases, FP32 products)
+                const double ca = s_a[jg + P::kMid], cb = s_b[jg + P::kMid], cc = s_c[jg + P::kMid];
+                const double da = s_a[jg + P::kMid + 1] - ca, db = s_b[jg + P::kMid + 1] - cb, dc = s_c[jg + P::kMid + 1] - cc;
                 const float2 RA = cis_f64(fma(da, lcol, dc * ncol));
                 const float2 RB = cis_f64(fma(db, lrow, dc * nrow));
                 const float c0 = (float)cc * cscale, d0 = (float)dc * cscale;
+                float2 A8[8], B8[8];
+                A8[P::kMid] = cis_f64(fma(ca, lcol, cc * ncol));
+                B8[P::kMid] = cis_f64(fma(cb, lrow, cc * nrow));
+#pragma unroll
+                for (int e = P::kMid + 1; e < 8; e++) {
+                    A8[e] = cmulf(A8[e - 1], RA);
+                    B8[e] = cmulf(B8[e - 1], RB);
+                }
+#pragma unroll
+                for (int e = P::kMid; e > 0; e--) {
+                    A8[e - 1] = cmulf(A8[e], make_float2(RA.x, -RA.y));
+                    B8[e - 1] = cmulf(B8[e], make_float2(RB.x, -RB.y));
+                }
 #pragma unroll
                 for (int q = 0; q < 4; q++) {
                     float2 L[2], Aq[2];
@@ -275,20 +328,16 @@ __device__ __forceinline__ void grid_mfma_body(const KernelArgs& a, int sidx, in
 #pragma unroll
                     for (int h = 0; h < 2; h++) {
                         const int e = 2 * q + h;
-                        Aq[h] = A;
-                        L[h] = cmulf(s_v[jg + e], B);
-                        cf[h] = fmaf((float)e, d0, c0);
-                        if (e < 7) {
-                            A = cmulf(A, RA);
-                            B = cmulf(B, RB);
-                        }
+                        Aq[h] = A8[e];
+                        L[h] = cmulf(s_v[jg + e], B8[e]);
+                        cf[h] = fmaf((float)(e - P::kMid), d0, c0);
                     }
                     cLr[q] = P::pack(cf[0] * L[0].x, cf[1] * L[1].x);
                     cLi[q] = P::pack(cf[0] * L[0].y, cf[1] * L[1].y);
-                    P9_SPLIT2(P, sk, L[0].x, L[1].x, Lrh[q], Lrl[q]);
-                    P9_SPLIT2(P, sk, L[0].y, L[1].y, Lih[q], Lil[q]);
-                    P9_SPLIT2(P, sk, Aq[0].x, Aq[1].x, Arh[q], Arl[q]);
-                    P9_SPLIT2(P, sk, Aq[0].y, Aq[1].y, Aih[q], Ail[q]);
+                    P9_SPLIT3(P, sk, L[0].x, L[1].x, Lrh[q], Lrl[q], Lr3[q]);
+                    P9_SPLIT3(P, sk, L[0].y, L[1].y, Lih[q], Lil[q], Li3[q]);
+                    P9_SPLIT3(P, sk, Aq[0].x, Aq[1].x, Arh[q], Arl[q], Ar3[q]);
+                    P9_SPLIT3(P, sk, Aq[0].y, Aq[1].y, Aih[q], Ail[q], Ai3[q]);
                 }
             } else {
 #pragma unroll
@@ -305,10 +354,10 @@ __device__ __forceinline__ void grid_mfma_body(const KernelArgs& a, int sidx, in
                     }
                     cLr[q] = P::pack(cf[0] * L[0].x, cf[1] * L[1].x);
                     cLi[q] = P::pack(cf[0] * L[0].y, cf[1] * L[1].y);
-                    P9_SPLIT2(P, sk, L[0].x, L[1].x, Lrh[q], Lrl[q]);
-                    P9_SPLIT2(P, sk, L[0].y, L[1].y, Lih[q], Lil[q]);
-                    P9_SPLIT2(P, sk, A[0].x, A[1].x, Arh[q], Arl[q]);
-                    P9_SPLIT2(P, sk, A[0].y, A[1].y, Aih[q], Ail[q]);
+                    P9_SPLIT3(P, sk, L[0].x, L[1].x, Lrh[q], Lrl[q], Lr3[q]);
+                    P9_SPLIT3(P, sk, L[0].y, L[1].y, Lih[q], Lil[q], Li3[q]);
+                    P9_SPLIT3(P, sk, A[0].x, A[1].x, Arh[q], Arl[q], Ar3[q]);
+                    P9_SPLIT3(P, sk, A[0].y, A[1].y, Aih[q], Ail[q], Ai3[q]);
                 }
             }
             // Re M0 = Lr Ar - Li Ai, Im M0 = Lr Ai + Li Ar (hi*hi + hi*lo + lo*hi);
@@ -329,6 +378,22 @@ __device__ __forceinline__ void grid_mfma_body(const KernelArgs& a, int sidx, in
             acc0i = P::mma(Lih, Arl, acc0i);
             acc0n = P::mma(Lil, Aih, acc0n);
             acc0i = P::mma(Lil, Arh, acc0i);
+            if constexpr (P::kThird) {
+                acc0r = P::mma(Lrl, Arl, acc0r);
+                acc0i = P::mma(Lrl, Ail, acc0i);
+                acc0n = P::mma(Lil, Ail, acc0n);
+                acc0i = P::mma(Lil, Arl, acc0i);
+            }
+            if constexpr (P::kThird) {
+                acc0r = P::mma(Lrh, Ar3, acc0r);
+                acc0i = P::mma(Lrh, Ai3, acc0i);
+                acc0n = P::mma(Lih, Ai3, acc0n);
+                acc0i = P::mma(Lih, Ar3, acc0i);
+                acc0r = P::mma(Lr3, Arh, acc0r);
+                acc0i = P::mma(Lr3, Aih, acc0i);
+                acc0n = P::mma(Li3, Aih, acc0n);
+                acc0i = P::mma(Li3, Arh, acc0i);
+            }
         }
         __syncthreads();
     }
@@ -472,15 +537,14 @@ __device__ __forceinline__ void grid_mfma16_body(const KernelArgs& a, int sidx, 
     // (ca, cc) for coordinate tile t: channel stepping or direct evaluation
     auto phasors = [&](int jg, const double* co, int t, float2 (&out)[8]) {
         if (chan_rec) {
-            const double ca = co[jg], cc = w_c[jg];
-            const double da = co[jg + 1] - ca, dc = w_c[jg + 1] - cc;
-            float2 A = cis_f64(fma(ca, lt[t], cc * nt[t]));
-            const float2 R = cis_f64(fma(da, lt[t], dc * nt[t]));
+            const double ca = co[jg + P::kMid], cc = w_c[jg + P::kMid];
+            const double da = co[jg + P::kMid + 1] - ca, dc = w_c[jg + P::kMid + 1] - cc;
+            out[P::kMid] = cis_f64(fma(ca, lt[t], cc * nt[t]));
+            const float2 R = cis_f64(fma(da, lt[t], dc * nt[t])), Rb = make_float2(R.x, -R.y);
 #pragma unroll
-            for (int e = 0; e < 8; e++) {
-                out[e] = A;
-                if (e < 7) A = cmulf(A, R);
-            }
+            for (int e = P::kMid + 1; e < 8; e++) out[e] = cmulf(out[e - 1], R);
+#pragma unroll
+            for (int e = P::kMid; e > 0; e--) out[e - 1] = cmulf(out[e], Rb);
         } else {
 #pragma unroll
             for (int e = 0; e < 8; e++) out[e] = cis_f64(fma(co[jg + e], lt[t], w_c[jg + e] * nt[t]));
@@ -507,18 +571,19 @@ __device__ __forceinline__ void grid_mfma16_body(const KernelArgs& a, int sidx, 
             const int jg = st * 32 + grp * 8;  // this lane group's 8 visibilities
             // x-phasors of the column tiles, split; -Ai carries the products'
             // minus signs (one negation per column tile, not three per row tile)
-            u32x4 Arh[NT], Arl[NT], Aih[NT], Ail[NT], nAih[NT], nAil[NT];
+            u32x4 Arh[NT], Arl[NT], Aih[NT], Ail[NT], nAih[NT], nAil[NT], Ar3[NT], Ai3[NT], nAi3[NT];
 #pragma unroll
             for (int t = 0; t < NT; t++) {
                 float2 A[8];
                 phasors(jg, w_a, t, A);
 #pragma unroll
                 for (int q = 0; q < 4; q++) {
-                    P9_SPLIT2(P, sk, A[2 * q].x, A[2 * q + 1].x, Arh[t][q], Arl[t][q]);
-                    P9_SPLIT2(P, sk, A[2 * q].y, A[2 * q + 1].y, Aih[t][q], Ail[t][q]);
+                    P9_SPLIT3(P, sk, A[2 * q].x, A[2 * q + 1].x, Arh[t][q], Arl[t][q], Ar3[t][q]);
+                    P9_SPLIT3(P, sk, A[2 * q].y, A[2 * q + 1].y, Aih[t][q], Ail[t][q], Ai3[t][q]);
                 }
                 nAih[t] = neg(Aih[t]);
                 nAil[t] = neg(Ail[t]);
+                if constexpr (P::kThird) nAi3[t] = neg(Ai3[t]);
             }
             // c of the 8 visibilities (FP32; scaled for FP16)
             float cf[8];
@@ -528,14 +593,14 @@ __device__ __forceinline__ void grid_mfma16_body(const KernelArgs& a, int sidx, 
             for (int r = 0; r < NT; r++) {
                 float2 B[8];
                 phasors(jg, w_b, r, B);
-                u32x4 Lrh, Lrl, Lih, Lil, cLr, cLi;
+                u32x4 Lrh, Lrl, Lih, Lil, cLr, cLi, Lr3, Li3;
 #pragma unroll
                 for (int q = 0; q < 4; q++) {
                     const float2 L0 = cmulf(w_v[jg + 2 * q], B[2 * q]), L1 = cmulf(w_v[jg + 2 * q + 1], B[2 * q + 1]);
                     cLr[q] = P::pack(cf[2 * q] * L0.x, cf[2 * q + 1] * L1.x);
                     cLi[q] = P::pack(cf[2 * q] * L0.y, cf[2 * q + 1] * L1.y);
-                    P9_SPLIT2(P, sk, L0.x, L1.x, Lrh[q], Lrl[q]);
-                    P9_SPLIT2(P, sk, L0.y, L1.y, Lih[q], Lil[q]);
+                    P9_SPLIT3(P, sk, L0.x, L1.x, Lrh[q], Lrl[q], Lr3[q]);
+                    P9_SPLIT3(P, sk, L0.y, L1.y, Lih[q], Lil[q], Li3[q]);
                 }
 #pragma unroll
                 for (int q = 0; q < NT; q++) {
@@ -558,6 +623,22 @@ __device__ __forceinline__ void grid_mfma16_body(const KernelArgs& a, int sidx, 
                     m0i = P::mma16(Lih, Arl[q], m0i);
                     m0r = P::mma16(Lil, nAih[q], m0r);
                     m0i = P::mma16(Lil, Arh[q], m0i);
+                    if constexpr (P::kThird) {
+                        m0r = P::mma16(Lrl, Arl[q], m0r);
+                        m0i = P::mma16(Lrl, Ail[q], m0i);
+                        m0r = P::mma16(Lil, nAil[q], m0r);
+                        m0i = P::mma16(Lil, Arl[q], m0i);
+                    }
+                    if constexpr (P::kThird) {
+                        m0r = P::mma16(Lrh, Ar3[q], m0r);
+                        m0i = P::mma16(Lrh, Ai3[q], m0i);
+                        m0r = P::mma16(Lih, nAi3[q], m0r);
+                        m0i = P::mma16(Lih, Ar3[q], m0i);
+                        m0r = P::mma16(Lr3, Arh[q], m0r);
+                        m0i = P::mma16(Lr3, Aih[q], m0i);
+                        m0r = P::mma16(Li3, nAih[q], m0r);
+                        m0i = P::mma16(Li3, Arh[q], m0i);
+                    }
                 }
             }
         }
@@ -644,7 +725,7 @@ __device__ __forceinline__ void degrid_mfma_body(const KernelArgs& a, int sidx, 
 
     // A operand: pixels_copy[y][x] = subgrid[(y+S/2)%S][(x+S/2)%S] (Gridder.cs:101-117)
     // at y = 16 rt + col, x = 32 ks + 8 grp + e; P split hi/lo and r P
-    u32x4 Prh[RT][KS], Prl[RT][KS], Pih[RT][KS], Pil[RT][KS], Qr[RT][KS], Qi[RT][KS];
+    u32x4 Prh[RT][KS], Prl[RT][KS], Pih[RT][KS], Pil[RT][KS], Qr[RT][KS], Qi[RT][KS], Pr3[RT][KS], Pi3[RT][KS];
 #pragma unroll
     for (int rt = 0; rt < RT; rt++) {
 #pragma unroll
@@ -665,8 +746,8 @@ __device__ __forceinline__ void degrid_mfma_body(const KernelArgs& a, int sidx, 
                         rr[u] = a.rtab[y * S + x] * rscale;
                     }
                 }
-                P9_SPLIT2(P, sk, pv[0].x, pv[1].x, Prh[rt][ks][q], Prl[rt][ks][q]);
-                P9_SPLIT2(P, sk, pv[0].y, pv[1].y, Pih[rt][ks][q], Pil[rt][ks][q]);
+                P9_SPLIT3(P, sk, pv[0].x, pv[1].x, Prh[rt][ks][q], Prl[rt][ks][q], Pr3[rt][ks][q]);
+                P9_SPLIT3(P, sk, pv[0].y, pv[1].y, Pih[rt][ks][q], Pil[rt][ks][q], Pi3[rt][ks][q]);
                 Qr[rt][ks][q] = P::pack(rr[0] * pv[0].x, rr[1] * pv[1].x);
                 Qi[rt][ks][q] = P::pack(rr[0] * pv[0].y, rr[1] * pv[1].y);
             }
@@ -678,7 +759,7 @@ __device__ __forceinline__ void degrid_mfma_body(const KernelArgs& a, int sidx, 
     // -Pr and -rPr, so no tile negates its x-phasors; S = 48 keeps the
     // registers and negates the phasors instead.
     constexpr bool kNegP = RT * KS <= 2;
-    u32x4 nPrh[RT][KS], nPrl[RT][KS], nQr[RT][KS];
+    u32x4 nPrh[RT][KS], nPrl[RT][KS], nQr[RT][KS], nPr3[RT][KS];
 #pragma unroll
     for (int rt = 0; rt < RT; rt++)
 #pragma unroll
@@ -687,6 +768,7 @@ __device__ __forceinline__ void degrid_mfma_body(const KernelArgs& a, int sidx, 
                 nPrh[rt][ks] = neg(Prh[rt][ks]);
                 nPrl[rt][ks] = neg(Prl[rt][ks]);
                 nQr[rt][ks] = neg(Qr[rt][ks]);
+                if constexpr (P::kThird) nPr3[rt][ks] = neg(Pr3[rt][ks]);
             }
 
     // One tile: Q0 = P conj(A), Q1 = (r P) conj(A) on the MFMA, then
@@ -724,6 +806,12 @@ __device__ __forceinline__ void degrid_mfma_body(const KernelArgs& a, int sidx, 
                     q0i[rt] = P::mma16(nPrh[rt][ks], Ail, q0i[rt]);
                     q0r[rt] = P::mma16(Pil[rt][ks], Aih, q0r[rt]);
                     q0i[rt] = P::mma16(nPrl[rt][ks], Aih, q0i[rt]);
+                    if constexpr (P::kThird) {
+                        q0r[rt] = P::mma16(Pr3[rt][ks], Arh, q0r[rt]);
+                        q0i[rt] = P::mma16(Pi3[rt][ks], Arh, q0i[rt]);
+                        q0r[rt] = P::mma16(Pi3[rt][ks], Aih, q0r[rt]);
+                        q0i[rt] = P::mma16(nPr3[rt][ks], Aih, q0i[rt]);
+                    }
                 }
             } else {
                 const u32x4 nAih = neg(Aih), nAil = neg(Ail);
@@ -745,6 +833,12 @@ __device__ __forceinline__ void degrid_mfma_body(const KernelArgs& a, int sidx, 
                     q0i[rt] = P::mma16(Prh[rt][ks], nAil, q0i[rt]);
                     q0r[rt] = P::mma16(Pil[rt][ks], Aih, q0r[rt]);
                     q0i[rt] = P::mma16(Prl[rt][ks], nAih, q0i[rt]);
+                    if constexpr (P::kThird) {
+                        q0r[rt] = P::mma16(Pr3[rt][ks], Arh, q0r[rt]);
+                        q0i[rt] = P::mma16(Pi3[rt][ks], Arh, q0i[rt]);
+                        q0r[rt] = P::mma16(Pi3[rt][ks], Aih, q0r[rt]);
+                        q0i[rt] = P::mma16(Pr3[rt][ks], nAih, q0i[rt]);
+                    }
                 }
             }
         }
@@ -890,7 +984,7 @@ __device__ __forceinline__ void degrid_mfma_body(const KernelArgs& a, int sidx, 
 template <int S, class P>
 __device__ __forceinline__ void degrid_mfma_wide_body(const KernelArgs& a, int sidx, int k0, int k1) {
     static_assert(S > 32 && S <= 64, "two 32-wide tiles per axis");
-    constexpr int RT = 2, KS = 4, NA = 6;  // row tiles, k-steps, operand arrays
+    constexpr int RT = 2, KS = 4, NA = P::kThird ? 8 : 6;  // row tiles, k-steps, operand arrays
     __shared__ float2 s_tile[2][S * S];
     __shared__ u32x4 s_op[RT * KS * NA * 64];
     __shared__ double s_l[64], s_n1[64];
@@ -924,7 +1018,7 @@ __device__ __forceinline__ void degrid_mfma_wide_body(const KernelArgs& a, int s
     for (int q = tid; q < RT * KS * 64; q += kThreads) {
         const int ln = q & 63, h = (q >> 6) % KS, rt = q / (64 * KS);
         const int y = rt * 32 + (ln & 31);
-        u32x4 prh, prl, pih, pil, qr, qi;
+        u32x4 prh, prl, pih, pil, qr, qi, pr3, pi3;
 #pragma unroll
         for (int w = 0; w < 4; w++) {  // elements 2w, 2w+1
             float2 pv[2];
@@ -941,8 +1035,8 @@ __device__ __forceinline__ void degrid_mfma_wide_body(const KernelArgs& a, int s
                     rr[u] = a.rtab[y * S + x] * rscale;
                 }
             }
-            P9_SPLIT2(P, sk, pv[0].x, pv[1].x, prh[w], prl[w]);
-            P9_SPLIT2(P, sk, pv[0].y, pv[1].y, pih[w], pil[w]);
+            P9_SPLIT3(P, sk, pv[0].x, pv[1].x, prh[w], prl[w], pr3[w]);
+            P9_SPLIT3(P, sk, pv[0].y, pv[1].y, pih[w], pil[w], pi3[w]);
             qr[w] = P::pack(rr[0] * pv[0].x, rr[1] * pv[1].x);
             qi[w] = P::pack(rr[0] * pv[0].y, rr[1] * pv[1].y);
         }
@@ -953,6 +1047,10 @@ __device__ __forceinline__ void degrid_mfma_wide_body(const KernelArgs& a, int s
         op[3 * 64] = pil;
         op[4 * 64] = qr;
         op[5 * 64] = qi;
+        if constexpr (P::kThird) {
+            op[6 * 64] = pr3;
+            op[7 * 64] = pi3;
+        }
     }
     __syncthreads();
     const float out_scale = a.degrid_scale / pscale;
@@ -1013,6 +1111,13 @@ __device__ __forceinline__ void degrid_mfma_wide_body(const KernelArgs& a, int s
                 q0i = P::mma(prh, nAil, q0i);
                 q0r = P::mma(pil, Aih[h], q0r);
                 q0i = P::mma(prl, nAih, q0i);
+                if constexpr (P::kThird) {
+                    const u32x4 pr3 = op[6 * 64], pi3 = op[7 * 64];
+                    q0r = P::mma(pr3, Arh[h], q0r);
+                    q0i = P::mma(pi3, Arh[h], q0i);
+                    q0r = P::mma(pi3, Aih[h], q0r);
+                    q0i = P::mma(pr3, nAih, q0i);
+                }
             }
 #pragma unroll
             for (int r = 0; r < 16; r++) {
@@ -1108,14 +1213,22 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kDegri
         }                                                                                          \
     } while (0)
 
+#define P9_MFMA_PREC(KERNEL, QKERNEL, SV)                           \
+    if (f16)                                                        \
+        P9_LAUNCH_MFMA(KERNEL, QKERNEL, SV, dev::PrecF16);          \
+    else if (a.rows)                                                \
+        P9_LAUNCH_MFMA(KERNEL, QKERNEL, SV, dev::PrecBF16Rows);     \
+    else                                                            \
+        P9_LAUNCH_MFMA(KERNEL, QKERNEL, SV, dev::PrecBF16);
+
 #define P9_MFMA_SWITCH(KERNEL, QKERNEL)                                              \
     switch (S) {                                                                     \
-        case 8: if (f16) P9_LAUNCH_MFMA(KERNEL, QKERNEL, 8, dev::PrecF16); else P9_LAUNCH_MFMA(KERNEL, QKERNEL, 8, dev::PrecBF16); break;    \
-        case 16: if (f16) P9_LAUNCH_MFMA(KERNEL, QKERNEL, 16, dev::PrecF16); else P9_LAUNCH_MFMA(KERNEL, QKERNEL, 16, dev::PrecBF16); break; \
-        case 24: if (f16) P9_LAUNCH_MFMA(KERNEL, QKERNEL, 24, dev::PrecF16); else P9_LAUNCH_MFMA(KERNEL, QKERNEL, 24, dev::PrecBF16); break; \
-        case 32: if (f16) P9_LAUNCH_MFMA(KERNEL, QKERNEL, 32, dev::PrecF16); else P9_LAUNCH_MFMA(KERNEL, QKERNEL, 32, dev::PrecBF16); break; \
-        case 48: if (f16) P9_LAUNCH_MFMA(KERNEL, QKERNEL, 48, dev::PrecF16); else P9_LAUNCH_MFMA(KERNEL, QKERNEL, 48, dev::PrecBF16); break; \
-        case 64: if (f16) P9_LAUNCH_MFMA(KERNEL, QKERNEL, 64, dev::PrecF16); else P9_LAUNCH_MFMA(KERNEL, QKERNEL, 64, dev::PrecBF16); break; \
+        case 8: P9_MFMA_PREC(KERNEL, QKERNEL, 8) break; \
+        case 16: P9_MFMA_PREC(KERNEL, QKERNEL, 16) break; \
+        case 24: P9_MFMA_PREC(KERNEL, QKERNEL, 24) break; \
+        case 32: P9_MFMA_PREC(KERNEL, QKERNEL, 32) break; \
+        case 48: P9_MFMA_PREC(KERNEL, QKERNEL, 48) break; \
+        case 64: P9_MFMA_PREC(KERNEL, QKERNEL, 64) break; \
         default: return hipErrorNotSupported;                                        \
     }
 
@@ -1149,6 +1262,9 @@ hipError_t batch_dispatch(bool grid, const BatchArgs& b, int kernel, int wg, hip
     if (kernel == P9IDG_KERNEL_MFMA_FP16)
         return grid ? launch_batch_kernel(dev::grid_mfma_batch_kernel<S, dev::PrecF16>, b, wg, st)
                     : launch_batch_kernel(dev::degrid_mfma_batch_kernel<S, dev::PrecF16>, b, wg, st);
+    if (b.rows)
+        return grid ? launch_batch_kernel(dev::grid_mfma_batch_kernel<S, dev::PrecBF16Rows>, b, wg, st)
+                    : launch_batch_kernel(dev::degrid_mfma_batch_kernel<S, dev::PrecBF16Rows>, b, wg, st);
     return grid ? launch_batch_kernel(dev::grid_mfma_batch_kernel<S, dev::PrecBF16>, b, wg, st)
                 : launch_batch_kernel(dev::degrid_mfma_batch_kernel<S, dev::PrecBF16>, b, wg, st);
 }

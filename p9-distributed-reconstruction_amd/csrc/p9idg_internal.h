@@ -145,6 +145,7 @@ struct KernelArgs {
     // (FP16) against these; as compile-time constants they would be folded
     // back into a conversion and a subtraction
     uint32_t split_k[3];
+    int32_t rows;  // time-resampled rows (split BF16 takes one more part)
     const WorkItem* items; // work queue (longest first)
     int32_t nitems;
     int32_t* counter;      // [2]: next item, finished workgroups; zero between launches
@@ -156,6 +157,7 @@ struct BatchArgs {
     const WorkItem* items;
     int32_t nitems;
     int32_t* counter;  // [2], as in KernelArgs
+    bool rows;         // a member's rows are resampled
 };
 
 // Launchers (kernels_*.hip); S is the subgrid size.
