@@ -14,9 +14,14 @@ Prints one JSON line.  Beside the headline it carries:
                   (per-pixel phasors, and the separable phasors of the MFMA
                   form), each autotuned, timed in this run
   hbm             achieved GB/s of the HBM-bound stages (target zeroing,
-                  ToImage, ToUVW), HIP events over repeated runs
-  roofline        the slower direction's kernel against the MFMA (or FP32)
-                  peak; roofline.other: the other direction's kernel
+                  ToImage, ToUVW), HIP events over repeated runs, of the bytes
+                  that their kernels read and write
+  roofline        the slower direction's kernel: its time, its HBM traffic in
+                  the committed profile, and the rate at which a direct sum
+                  over the visibilities would have to run to take as long
+                  (the kernels contract time-resampled rows, so that rate is
+                  not the pipes' and has no peak); roofline.other: the other
+                  direction's kernel
   error_vs_oracle the timed plan (its autotuned launch shape) against the FP64
                   oracle on the whole workload: dirty image, PSF, degridded
                   visibilities (max and RMS relative error)
@@ -37,7 +42,6 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, os.path.join(ROOT, "p9-distributed-reconstruction_amd"))
 
 METRIC = "Mvis/s grid+degrid, 3072² 32 w-layers: split-BF16 MFMA vs FP32, ≤1e-5 err"
-PEAK_TFLOPS = {"fp32": 157.3, "fp32_sep": 157.3, "mfma_bf16": 2500.0, "mfma_fp16": 2500.0}
 BOUND = {"fp32": "valu", "fp32_sep": "valu", "mfma_bf16": "mfma", "mfma_fp16": "mfma"}
 DTYPE = {"fp32": "f32", "fp32_sep": "f32", "mfma_bf16": "bf16 hi/lo split, f32 accumulate",
          "mfma_fp16": "f16 hi/lo split, f32 accumulate"}
@@ -209,7 +213,7 @@ def time_steps(plan, steps, warmup):
 
 def wstack_footprint(meta, G, S, L):
     """Per-layer bounding boxes of the w-stacked adder (AdderWStack.cs:29-70):
-    summed area and the union box's area, in pixels."""
+    summed area and the union box's height and width, in pixels."""
     X = meta["UPixel"].astype(np.int64)
     Y = meta["VPixel"].astype(np.int64)
     W = meta["WLambda"].astype(np.int64)
@@ -223,8 +227,28 @@ def wstack_footprint(meta, G, S, L):
         k = ok & (W == l)
         if k.any():
             area += int((Y[k].max() + S - Y[k].min()) * (X[k].max() + S - X[k].min()))
-    union = int((Y[ok].max() + S - Y[ok].min()) * (X[ok].max() + S - X[ok].min())) if ok.any() else 0
-    return area, union
+    if not ok.any():
+        return area, 0, 0
+    return area, int(Y[ok].max() + S - Y[ok].min()), int(X[ok].max() + S - X[ok].min())
+
+
+def stage_bytes(G, area, height, width):
+    """Bytes that the HBM-bound stages read and write at a grid size with line
+    transforms (even, 2^a 3^b 5^c, at most 4096): complex64 is 8 bytes."""
+    return {
+        # the footprint boxes of the previous gridding, zeroed before each gridder launch
+        "zero": 8 * area,
+        # the layer boxes summed into a dense box; its columns transformed over the grid's height; those rows
+        # transformed and written as image rows
+        "to_image": 8 * area + 8 * height * width + 8 * height * width + 2 * 8 * G * width + 4 * G * G,
+        # real columns transformed, half of their rows kept; those transformed and written with their mirrors
+        "to_uvw": 4 * G * G + 2 * 8 * (G // 2 + 1) * G + 8 * G * G,
+    }
+
+
+def direct_sum_tflops(S, n_vis, ms):
+    """The rate of the direct sum's complex MACs (8 S^2 per gridded visibility) in `ms`."""
+    return 8.0 * S * S * n_vis / (ms / 1e3) / 1e12
 
 
 def comparator(ob, part, kernel, steps, warmup, tune):
@@ -563,7 +587,7 @@ def main():
     ap.add_argument("--gpus", type=int, default=1)
     ap.add_argument("--steps", type=int, default=10)
     ap.add_argument("--warmup", type=int, default=2)
-    ap.add_argument("--kernel", default="mfma_bf16", choices=sorted(PEAK_TFLOPS))
+    ap.add_argument("--kernel", default="mfma_bf16", choices=sorted(BOUND))
     ap.add_argument("--launch", default=None, metavar="QUEUE,GRID_CHUNK,DEGRID_CHUNK,WORKGROUPS",
                     help="fixed launch shape instead of the autotuner's (e.g. 1,0,0,256)")
     ap.add_argument("--no-oracle", "--no-cpu-baseline", dest="no_oracle", action="store_true",
@@ -637,21 +661,11 @@ def main():
     ti_ms, ti_n = plan.timing_stage(p9idg.STAGE_TO_IMAGE)
     tu_ms, tu_n = plan.timing_stage(p9idg.STAGE_TO_UVW)
     plan.timing_reset(False)
-    area, union = wstack_footprint(part.subgrids, G, S, L)
-    GG = G * G
-    fft_bytes = 4 * GG * 8  # an in-place G x G complex64 FFT counted as two read + write passes
-    stage_bytes = {
-        # the footprint boxes of the previous gridding, zeroed before each gridder launch
-        "zero": area * 8,
-        # zero the layer sum, sum the layer boxes, inverse FFT, real part / N into the shifted image
-        "to_image": GG * 8 + area * 8 + union * 8 + fft_bytes + GG * 8 + GG * 4,
-        # shifted image into a complex grid, forward FFT
-        "to_uvw": GG * 4 + GG * 8 + fft_bytes,
-    }
+    moved = stage_bytes(G, *wstack_footprint(part.subgrids, G, S, L))
     stage_ms = {"zero": tm["zero_ms"], "to_image": ti_ms / max(ti_n, 1), "to_uvw": tu_ms / max(tu_n, 1)}
-    hbm = {k: {"ms": stage_ms[k], "bytes": int(stage_bytes[k]),
-               "gb_s": stage_bytes[k] / (stage_ms[k] / 1e3) / 1e9 if stage_ms[k] > 0 else None}
-           for k in stage_bytes}
+    hbm = {k: {"ms": stage_ms[k], "bytes": int(moved[k]),
+               "gb_s": moved[k] / (stage_ms[k] / 1e3) / 1e9 if stage_ms[k] > 0 else None}
+           for k in moved}
     for k, v in hbm.items():
         v["frac_of_peak"] = v["gb_s"] / HBM_PEAK_GBS if v["gb_s"] else None
     log("hbm stages: " + ", ".join("%s %.3f ms %.0f GB/s" % (k, v["ms"], v["gb_s"] or 0) for k, v in hbm.items()))
@@ -685,33 +699,22 @@ def main():
         vs_fp32["faster_fp32"] = best
         vs_fp32["ratio"] = value / vs_fp32[best]["value"]
 
-    # the direct sum's complex MAC per pixel and visibility, whatever the kernels contract: they work on the
-    # time-resampled rows, so `achieved` is a direct-sum equivalent, not the matrix pipe's load
-    flops_per_launch = 8.0 * S * S * n_vis
     dom_name, dom_ms = ("gridder", avg_g) if avg_g >= avg_d else ("degridder", avg_d)
-    achieved = flops_per_launch / (dom_ms / 1e3) / 1e12
-    peak = PEAK_TFLOPS[args.kernel]
+    oth_name, oth_ms = ("degridder", avg_d) if dom_name == "gridder" else ("gridder", avg_g)
     traffic, traffic_launch = profiled_traffic(args.kernel, dom_name)
     roofline = {
         "bound": BOUND[args.kernel],
         "kernel": dom_name,
-        "achieved": achieved,
-        "peak": peak,
-        "unit": "TFLOP/s",
-        "frac": achieved / peak,
+        "kernel_ms": dom_ms,
         "traffic": traffic,
         "traffic_launch": traffic_launch,
         "traffic_at_timed_launch": bool(traffic_launch) and all(
             traffic_launch.get(k) == tuning.get(k) for k in ("queue", "grid_chunk", "degrid_chunk", "workgroups")),
-        "flops_per_launch": flops_per_launch,
-        "flops_counted": "direct sum (8 S^2 per gridded visibility); the kernels contract time-resampled rows",
-        "kernel_ms": dom_ms,
+        # not a load of the pipes: the kernels contract time-resampled rows
+        "direct_sum_equivalent_tflops": direct_sum_tflops(S, n_vis, dom_ms),
+        "other": {"kernel": oth_name, "kernel_ms": oth_ms, "traffic": profiled_traffic(args.kernel, oth_name)[0],
+                  "direct_sum_equivalent_tflops": direct_sum_tflops(S, n_vis, oth_ms)},
     }
-    # the other direction's kernel against the same peak (same algorithmic work)
-    oth_name, oth_ms = ("degridder", avg_d) if dom_name == "gridder" else ("gridder", avg_g)
-    oth = flops_per_launch / (oth_ms / 1e3) / 1e12
-    roofline["other"] = {"kernel": oth_name, "achieved": oth, "frac": oth / peak, "kernel_ms": oth_ms,
-                         "traffic": profiled_traffic(args.kernel, oth_name)[0]}
     cpu, err = None, None
     if not args.no_oracle:
         cpu, err = oracle_checks(ob, part, gpu, model_grid)
