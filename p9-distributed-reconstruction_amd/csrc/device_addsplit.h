@@ -23,7 +23,7 @@ namespace dev {
 // subgrids each on the 3072^2 workload) and the adder is bound by the atomics
 // that queue on them: a thread per pixel with one atomic per part touches each
 // sector twice.  3072^2 gridding of resampled rows 215 -> 186 us.
-template <int S, int NTH = kThreads>
+template <int S>
 __device__ __forceinline__ void adder(const KernelArgs& a, const SubgridGeom& g,
                                       const float2* tile, float norm, int slot, const float2* ap) {
     const int G = a.G;
@@ -43,7 +43,7 @@ __device__ __forceinline__ void adder(const KernelArgs& a, const SubgridGeom& g,
         if (W < 0 || W >= a.L) return;  // metadata validated on the host
     }
     float* const layer = reinterpret_cast<float*>(a.grid + (a.mode == P9IDG_GRID_WSTACK ? (size_t)W * G * G : 0));
-    for (int q = item_tid(); q < 2 * S * S; q += NTH) {
+    for (int q = item_tid(); q < 2 * S * S; q += kThreads) {
         const int p = q >> 1, im = q & 1;
         const int y = p / S, x = p - (p / S) * S;
         const int y_ = neg ? S - 1 - y : y;

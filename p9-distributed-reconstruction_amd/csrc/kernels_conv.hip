@@ -1,9 +1,9 @@
 // The padded PSF correlation (PaddedConvolver.cs, Common.cs:146-160) on FP64
 // line transforms in LDS.
 //
-// The correlation is linear: the circular size n only has to reach H + rows - 1
-// (W + cols - 1), so it is the next even 2^a 3^b 5^c.  Image and result are
-// real: pairs of image rows share one complex transform, the n / 2 + 1 columns
+// The correlation is linear, so the circular size need not be the padded size
+// H + rows (W + cols) itself: n is the next even 2^a 3^b 5^c from there.  Image
+// and result are real: pairs of image rows share one complex transform, the n / 2 + 1 columns
 // that determine the rest are transformed, multiplied by the PSF's spectrum and
 // transformed back while they are in LDS, and pairs of result rows come out of
 // one complex transform.  3072^2 with a 192^2 PSF moves 0.4 GB; two 2-D library

@@ -91,11 +91,11 @@ struct PrecBF16 {
 // error of the image against 64 bits, own rows / resampled in two parts / in
 // three: headline 5.5e-7 / 5.4e-7 / 3.9e-7, 435 baselines x 600 x 8 every 2 s
 // 5.4e-7 / 7.4e-7 / 4.8e-7, 5 channels 3.9e-7 / 6.3e-7 / 3.1e-7; headline gridding
-// and image 223 -> 251 us, three uneven observations 600 -> 664.  The degridder's pixels have a third part (4 MFMAs
-// more): their rounding is the same for all rows of a subgrid, so it is what an
-// image of residuals shows most.  Visibilities 3.9e-6 -> 3.0e-6, image of the
-// residuals at 2048^2 1.23e-5 (own rows 1.18e-5) -> 4.9e-6; headline prediction
-// 276 -> 281 us.
+// and image 223 -> 251 us, three uneven observations 600 -> 664.  The degridder's
+// pixels have a third part (4 MFMAs more): their rounding is the same for all rows
+// of a subgrid, so it is what an image of residuals shows most.  Visibilities
+// 3.9e-6 -> 3.0e-6, image of the residuals at 2048^2 1.23e-5 (own rows 1.18e-5) ->
+// 4.9e-6; headline prediction 276 -> 281 us.
 struct PrecBF16Rows : PrecBF16 {
     static constexpr bool kThird = true;
     // The channel of 8 from which the gridders step their phasors both ways.  A

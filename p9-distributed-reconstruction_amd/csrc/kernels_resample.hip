@@ -17,15 +17,16 @@
 // Which chunks qualify is measured, not assumed: analyse_kernel evaluates the
 // interpolant at every timestep of the chunk, at the four corner pixels (where
 // the phase varies most) and the highest channel, against the phasor of the
-// track itself, and takes the smallest number of nodes whose error is below
-// kResampleTol everywhere.  A track with a jump, noise or a gap fails the test
-// and keeps its rows as they are.
+// track itself, from an estimate of the nodes that its phase needs upwards in
+// steps of four, and takes the first number whose error is below kResampleTol
+// everywhere.  A track with a jump, noise or a gap fails the test and keeps its
+// rows as they are.
 //
 // Long chunks need fewer nodes in all (they grow with the phase that a chunk
 // covers, with some ten on top for each), but more weights and products per
-// row.  3072^2, subgrid 32, at most 256 / 512 / 1024 timesteps: gridder 141 / 132
-// / 124 us, gather 45 / 50 / 66; images at 1024^2 with FP32 106 / 93 us, three
-// uneven observations 646 / 597.  A chunk that would need more than 64 nodes is
+// row.  3072^2, subgrid 32, at most 256 / 512 / 1024 timesteps: gridder (two-part
+// operands) 141 / 132 / 124 us, gather 45 / 50 / 66; images at 1024^2 with FP32
+// 106 / 93 us, three uneven observations 646 / 597.  A chunk that would need more than 64 nodes is
 // halved.
 #include "device_common.h"
 
