@@ -756,10 +756,11 @@ __device__ __forceinline__ void degrid_mfma_body(const KernelArgs& a, int sidx, 
     const float out_scale = a.degrid_scale / pscale;
     const float q1_back = kTwoPiF / rscale;
     // Up to S = 32 the products' minus signs sit on loop-invariant copies of
-    // -Pr and -rPr, so no tile negates its x-phasors; S = 48 keeps the
-    // registers and negates the phasors instead.
-    constexpr bool kNegP = RT * KS <= 2;
-    u32x4 nPrh[RT][KS], nPrl[RT][KS], nQr[RT][KS], nPr3[RT][KS];
+    // -Pr and -rPr, so no tile negates its x-phasors; S = 48 and pixels in three
+    // parts (256 registers and spills at S = 32, no faster) keep the registers
+    // and negate the phasors instead.
+    constexpr bool kNegP = RT * KS <= 2 && !P::kThird;
+    u32x4 nPrh[RT][KS], nPrl[RT][KS], nQr[RT][KS];
 #pragma unroll
     for (int rt = 0; rt < RT; rt++)
 #pragma unroll
@@ -768,7 +769,6 @@ __device__ __forceinline__ void degrid_mfma_body(const KernelArgs& a, int sidx, 
                 nPrh[rt][ks] = neg(Prh[rt][ks]);
                 nPrl[rt][ks] = neg(Prl[rt][ks]);
                 nQr[rt][ks] = neg(Qr[rt][ks]);
-                if constexpr (P::kThird) nPr3[rt][ks] = neg(Pr3[rt][ks]);
             }
 
     // One tile: Q0 = P conj(A), Q1 = (r P) conj(A) on the MFMA, then
@@ -806,12 +806,6 @@ __device__ __forceinline__ void degrid_mfma_body(const KernelArgs& a, int sidx, 
                     q0i[rt] = P::mma16(nPrh[rt][ks], Ail, q0i[rt]);
                     q0r[rt] = P::mma16(Pil[rt][ks], Aih, q0r[rt]);
                     q0i[rt] = P::mma16(nPrl[rt][ks], Aih, q0i[rt]);
-                    if constexpr (P::kThird) {
-                        q0r[rt] = P::mma16(Pr3[rt][ks], Arh, q0r[rt]);
-                        q0i[rt] = P::mma16(Pi3[rt][ks], Arh, q0i[rt]);
-                        q0r[rt] = P::mma16(Pi3[rt][ks], Aih, q0r[rt]);
-                        q0i[rt] = P::mma16(nPr3[rt][ks], Aih, q0i[rt]);
-                    }
                 }
             } else {
                 const u32x4 nAih = neg(Aih), nAil = neg(Ail);
